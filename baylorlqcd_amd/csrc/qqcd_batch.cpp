@@ -73,22 +73,18 @@ namespace {
 template <typename T> struct HostBuf {
   T *p = nullptr;
   size_t n = 0;
-  explicit HostBuf(size_t n_) : n(n_) { QQCD_HIP(hipHostMalloc((void **)&p, n * sizeof(T), hipHostMallocDefault)); }
-  ~HostBuf() {
-    if (p) (void)hipHostFree(p);
-  }
+  explicit HostBuf(size_t n_) : n(n_) { p = static_cast<T *>(pool_alloc_host(n * sizeof(T))); }
+  ~HostBuf() { pool_free_host(p); }
   T &operator[](size_t i) { return p[i]; }
 };
 
 template <typename T> struct DevBuf {
   T *p = nullptr;
   explicit DevBuf(size_t n) {
-    QQCD_HIP(hipMalloc((void **)&p, std::max<size_t>(n, 1) * sizeof(T)));
-    QQCD_HIP(hipMemset(p, 0, std::max<size_t>(n, 1) * sizeof(T)));
+    pool_get(&p, std::max<size_t>(n, 1) * sizeof(T));
+    QQCD_HIP(hipMemsetAsync(p, 0, std::max<size_t>(n, 1) * sizeof(T), ctx().stream));
   }
-  ~DevBuf() {
-    if (p) (void)hipFree(p);
-  }
+  ~DevBuf() { pool_free(p); }
 };
 
 struct Graph {
@@ -104,6 +100,8 @@ class Batch {
  public:
   Batch(Context &c, const double kappa[2], MultiSpinor &B, MultiSpinor &X, const Deflation &D, const BatchParams &p,
         std::vector<int> &id);
+  // copies from the pinned buffers may be queued when an error unwinds
+  ~Batch() { (void)hipStreamSynchronize(c.stream); }
   BatchStats run(int n);
 
  private:
@@ -116,7 +114,7 @@ class Batch {
   MBlas mb;
   MultiSchur A64, A32;
   MultiBuf R64, Bin, E, R;
-  std::vector<MultiBuf *> basis_bufs;
+  std::vector<std::unique_ptr<MultiBuf>> basis_bufs;
   std::vector<MultiSpinor> V;
   // FP16 basis only: the FP32 vector being orthogonalised and the newest
   // basis vector in FP32 (the operator's input)
@@ -215,7 +213,7 @@ Batch::Batch(Context &c_, const double kappa[2], MultiSpinor &B_, MultiSpinor &X
     throw std::runtime_error("batched_solve: the Krylov basis is FP32 or FP16");
   basis_bufs.reserve(m + 1);
   for (int i = 0; i <= m; i++) {
-    basis_bufs.push_back(new MultiBuf(c.g, p.basis, cap, nb, false));
+    basis_bufs.emplace_back(new MultiBuf(c.g, p.basis, cap, nb, false));
     V.push_back(basis_bufs.back()->m);
   }
   if (half()) {
@@ -562,7 +560,7 @@ TuneResult autotune_multi(Context &c, Prec p, int recon, int nrhs) {
   TuneResult best;
   best.ms = 1e30;
   int *d_n = nullptr;
-  QQCD_HIP(hipMalloc(&d_n, sizeof(int)));
+  pool_get(&d_n, sizeof(int));
   QQCD_HIP(hipMemcpy(d_n, &nrhs, sizeof(int), hipMemcpyHostToDevice));
   hipEvent_t e0, e1;
   QQCD_HIP(hipEventCreate(&e0));
@@ -597,12 +595,12 @@ TuneResult autotune_multi(Context &c, Prec p, int recon, int nrhs) {
       }
     }
   } catch (...) {
-    (void)hipFree(d_n);
+    pool_free(d_n);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     throw;
   }
-  (void)hipFree(d_n);
+  pool_free(d_n);
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   cache[key] = best;

@@ -36,6 +36,7 @@ extern "C" int qqcd_init(const int n[4], const int bc[4], int device) {
     delete g_ctx;
     g_ctx = nullptr;
   }
+  pool_trim();
   for (int m = 0; m < 4; m++)
     if (n[m] <= 0 || n[m] % 4 != 0)
       throw std::runtime_error("lattice extents must be positive multiples of 4 (2 blocks x 2 checkerboards)");
@@ -44,7 +45,7 @@ extern "C" int qqcd_init(const int n[4], const int bc[4], int device) {
   if (device < 0 || device >= ndev) throw std::runtime_error("no such HIP device");
   QQCD_HIP(hipSetDevice(device));
   lagfib_noalloc_setup(device);
-  Context *c = new Context();
+  std::unique_ptr<Context> c(new Context());
   c->device = device;
   Geom &g = c->g;
   for (int m = 0; m < 4; m++) {
@@ -59,8 +60,8 @@ extern "C" int qqcd_init(const int n[4], const int bc[4], int device) {
   set_bc(*c, bc);
   QQCD_HIP(hipStreamCreate(&c->stream));
   c->blas.reset(new Blas(c->stream));
-  for (double *&p : c->dref) QQCD_HIP(hipMalloc(&p, sizeof(double) * 6 * ref_ntotal(g) * 64));
-  g_ctx = c;
+  for (double *&p : c->dref) pool_get(&p, sizeof(double) * 6 * ref_ntotal(g) * 64);
+  g_ctx = c.release();
   API_END
 }
 
@@ -80,6 +81,7 @@ extern "C" int qqcd_finalize(void) {
   lagfib_release_device();
   delete g_ctx;
   g_ctx = nullptr;
+  pool_trim();
   API_END
 }
 
@@ -106,12 +108,12 @@ extern "C" int qqcd_gauge_load_canonical(const double *U, const double *coact) {
   set_coact(c, coact);
   const size_t n = (size_t)2 * 36 * c.g.V;
   double *d = nullptr;
-  QQCD_HIP(hipMalloc(&d, n * sizeof(double)));
+  pool_get(&d, n * sizeof(double));
   QQCD_HIP(hipMemcpyAsync(d, U, n * sizeof(double), hipMemcpyHostToDevice, c.stream));
   if (!c.U64.data) c.U64 = alloc_gauge(c.g, PREC_DOUBLE, 18);
   canon_to_gauge(c.g, d, c.U64, c.stream);
   QQCD_HIP(hipStreamSynchronize(c.stream));
-  (void)hipFree(d);
+  pool_free(d);
   c.u_host = nullptr;
   c.have_gauge = 1;
   c.gauge_gen++;
@@ -444,7 +446,7 @@ extern "C" int qqcd_bench_dslash_rot(int prec, int recon, int nbuf, int nwarm, i
 }
 
 static void canon_io(Context &c, const double *h, size_t n, double **d) {
-  QQCD_HIP(hipMalloc(d, n * sizeof(double)));
+  pool_get(d, n * sizeof(double));
   QQCD_HIP(hipMemcpyAsync(*d, h, n * sizeof(double), hipMemcpyHostToDevice, c.stream));
 }
 
@@ -465,12 +467,12 @@ extern "C" int qqcd_hop_canonical(const double *psi, double *out, int par_out, i
     QQCD_HIP(hipMemcpyAsync(out, dout, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
     QQCD_HIP(hipStreamSynchronize(c.stream));
   } catch (...) {
-    (void)hipFree(dp);
-    (void)hipFree(dout);
+    pool_free(dp);
+    pool_free(dout);
     throw;
   }
-  (void)hipFree(dp);
-  (void)hipFree(dout);
+  pool_free(dp);
+  pool_free(dout);
   API_END
 }
 
@@ -492,12 +494,12 @@ extern "C" int qqcd_schur_canonical(const double *psi, double *out, const double
     QQCD_HIP(hipMemcpyAsync(out, dout, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
     QQCD_HIP(hipStreamSynchronize(c.stream));
   } catch (...) {
-    (void)hipFree(dp);
-    (void)hipFree(dout);
+    pool_free(dp);
+    pool_free(dout);
     throw;
   }
-  (void)hipFree(dp);
-  (void)hipFree(dout);
+  pool_free(dp);
+  pool_free(dout);
   API_END
 }
 
@@ -526,11 +528,11 @@ extern "C" int qqcd_gauge_get_canonical(double *U) {
   if (!c.have_gauge) throw std::runtime_error("no gauge field loaded");
   const size_t n = (size_t)2 * 36 * c.g.V;
   double *d = nullptr;
-  QQCD_HIP(hipMalloc(&d, n * sizeof(double)));
+  pool_get(&d, n * sizeof(double));
   gauge_to_canon(c.g, c.U64, d, c.stream);
   QQCD_HIP(hipMemcpyAsync(U, d, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
   QQCD_HIP(hipStreamSynchronize(c.stream));
-  (void)hipFree(d);
+  pool_free(d);
   API_END
 }
 
@@ -544,11 +546,11 @@ extern "C" int qqcd_gauge_get_ref(double *u) {
   if (!c.have_gauge) throw std::runtime_error("no gauge field loaded");
   const size_t n = (size_t)18 * ref_ntotal(c.g) * 128;
   double *d = nullptr;
-  QQCD_HIP(hipMalloc(&d, n * sizeof(double)));
+  pool_get(&d, n * sizeof(double));
   gauge_to_ref(c.g, c.U64, d, c.stream);
   QQCD_HIP(hipMemcpyAsync(u, d, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
   QQCD_HIP(hipStreamSynchronize(c.stream));
-  (void)hipFree(d);
+  pool_free(d);
   API_END
 }
 

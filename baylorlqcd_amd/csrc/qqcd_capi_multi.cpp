@@ -36,13 +36,11 @@ BatchStats g_bst;
 struct DevArr {
   double *p = nullptr;
   DevArr(const double *h, size_t n, hipStream_t s) {
-    QQCD_HIP(hipMalloc(&p, n * sizeof(double)));
+    pool_get(&p, n * sizeof(double));
     if (h) QQCD_HIP(hipMemcpyAsync(p, h, n * sizeof(double), hipMemcpyHostToDevice, s));
     else QQCD_HIP(hipMemsetAsync(p, 0, n * sizeof(double), s));
   }
-  ~DevArr() {
-    if (p) (void)hipFree(p);
-  }
+  ~DevArr() { pool_free(p); }
 };
 
 void to_device(Context &c, const double *h, Spinor &s, int par) {
@@ -88,7 +86,7 @@ void multi_canonical(int which, int nrhs, int nact, int nb, int prec, int recon,
     mb.put(s.s, a.m, r);
   }
   int *d_n = nullptr;
-  QQCD_HIP(hipMalloc(&d_n, sizeof(int)));
+  pool_get(&d_n, sizeof(int));
   try {
     QQCD_HIP(hipMemcpyAsync(d_n, &nact, sizeof(int), hipMemcpyHostToDevice, c.stream));
     MultiTune t;
@@ -109,10 +107,10 @@ void multi_canonical(int which, int nrhs, int nact, int nb, int prec, int recon,
     }
     QQCD_HIP(hipStreamSynchronize(c.stream));
   } catch (...) {
-    (void)hipFree(d_n);
+    pool_free(d_n);
     throw;
   }
-  (void)hipFree(d_n);
+  pool_free(d_n);
 }
 
 BatchParams batch_params(const int GMRES[2], double tol, int nb_rhs) {
@@ -820,7 +818,7 @@ extern "C" int qqcd_bench_dslash_multi(int prec, int recon, int nrhs, int nact, 
     }
   }
   int *d_n = nullptr;
-  QQCD_HIP(hipMalloc(&d_n, sizeof(int)));
+  pool_get(&d_n, sizeof(int));
   hipEvent_t e0 = nullptr, e1 = nullptr;
   try {
     QQCD_HIP(hipMemcpy(d_n, &nact, sizeof(int), hipMemcpyHostToDevice));
@@ -837,12 +835,12 @@ extern "C" int qqcd_bench_dslash_multi(int prec, int recon, int nrhs, int nact, 
     QQCD_HIP(hipEventElapsedTime(&f, e0, e1));
     *ms = f / std::max(niter, 1);
   } catch (...) {
-    (void)hipFree(d_n);
+    pool_free(d_n);
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     throw;
   }
-  (void)hipFree(d_n);
+  pool_free(d_n);
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   API_END

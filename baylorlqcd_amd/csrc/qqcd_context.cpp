@@ -25,22 +25,30 @@ size_t Gauge::bytes() const {
   return (size_t)8 * (recon == 18 ? 9 : 6) * stride * (prec == PREC_DOUBLE ? 16 : prec == PREC_SINGLE ? 8 : 4);
 }
 
-Spinor alloc_spinor(const Geom &g, Prec p) {
+// the clears are queued on the library's stream, ahead of the buffer's uses
+static hipStream_t field_stream() { return g_ctx ? g_ctx->stream : nullptr; }
+
+Spinor alloc_spinor(const Geom &g, Prec p, bool clear) {
   Spinor s;
   s.prec = p;
   s.stride = g.stride;
-  QQCD_HIP(hipMalloc(&s.data, s.bytes()));
-  QQCD_HIP(hipMemset(s.data, 0, s.bytes()));
-  if (p == PREC_HALF) {
-    QQCD_HIP(hipMalloc(&s.norm, sizeof(float) * g.stride));
-    QQCD_HIP(hipMemset(s.norm, 0, sizeof(float) * g.stride));
+  try {
+    pool_get(&s.data, s.bytes());
+    if (p == PREC_HALF) pool_get(&s.norm, sizeof(float) * g.stride);
+    if (clear || g.stride != g.Vh) {
+      QQCD_HIP(hipMemsetAsync(s.data, 0, s.bytes(), field_stream()));
+      if (s.norm) QQCD_HIP(hipMemsetAsync(s.norm, 0, sizeof(float) * g.stride, field_stream()));
+    }
+  } catch (...) {
+    free_spinor(s);
+    throw;
   }
   return s;
 }
 
 void free_spinor(Spinor &s) {
-  if (s.data) (void)hipFree(s.data);
-  if (s.norm) (void)hipFree(s.norm);
+  pool_free(s.data);
+  pool_free(s.norm);
   s.data = nullptr;
   s.norm = nullptr;
 }
@@ -64,8 +72,7 @@ Context::~Context() {
   if (stream) (void)hipStreamSynchronize(stream);
   for (auto &kv : copies) free_gauge(kv.second.U);
   free_gauge(U64);
-  for (double *&p : dref)
-    if (p) (void)hipFree(p);
+  for (double *&p : dref) pool_free(p);
   blas.reset();
   if (stream) (void)hipStreamDestroy(stream);
 }
@@ -81,13 +88,13 @@ const Gauge &Context::gauge(Prec p, int recon) {
     if (!cp.U.data) cp.U = alloc_gauge(g, p, recon);
     // convert through the canonical FP64 staging on the device
     double *tmp = nullptr;
-    QQCD_HIP(hipMalloc(&tmp, sizeof(double) * 2 * 36 * g.V));
+    pool_get(&tmp, sizeof(double) * 2 * 36 * g.V);
     // unpack the master into canonical order, then repack
     extern void gauge_to_canon(const Geom &, const Gauge &, double *, hipStream_t);
     gauge_to_canon(g, U64, tmp, stream);
     canon_to_gauge(g, tmp, cp.U, stream);
     QQCD_HIP(hipStreamSynchronize(stream));
-    (void)hipFree(tmp);
+    pool_free(tmp);
     cp.gen = gauge_gen;
   }
   return cp.U;
@@ -123,12 +130,12 @@ void ensure_gauge(Context &c, const double *u_ref, const double *coact) {
   if (c.have_gauge && c.u_host == (const void *)u_ref) return;
   const size_t n = (size_t)18 * ref_ntotal(c.g) * 128;
   double *d = nullptr;
-  QQCD_HIP(hipMalloc(&d, n * sizeof(double)));
+  pool_get(&d, n * sizeof(double));
   QQCD_HIP(hipMemcpyAsync(d, u_ref, n * sizeof(double), hipMemcpyHostToDevice, c.stream));
   if (!c.U64.data) c.U64 = alloc_gauge(c.g, PREC_DOUBLE, 18);
   ref_to_gauge(c.g, d, c.U64, c.stream);
   QQCD_HIP(hipStreamSynchronize(c.stream));
-  (void)hipFree(d);
+  pool_free(d);
   c.u_host = u_ref;
   c.have_gauge = 1;
   c.gauge_gen++;

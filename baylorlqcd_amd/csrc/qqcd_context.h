@@ -9,6 +9,7 @@
 #include <memory>
 #include <vector>
 #include "qqcd_blas.h"
+#include "qqcd_pool.h"
 
 namespace qqcd {
 
@@ -42,7 +43,8 @@ struct Context {
 extern Context *g_ctx;
 Context &ctx();
 
-Spinor alloc_spinor(const Geom &g, Prec p);
+// zeroed, unless clear is false and no padding sites need to be
+Spinor alloc_spinor(const Geom &g, Prec p, bool clear = true);
 void free_spinor(Spinor &s);
 Gauge alloc_gauge(const Geom &g, Prec p, int recon);
 void free_gauge(Gauge &u);

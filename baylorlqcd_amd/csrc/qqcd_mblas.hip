@@ -668,36 +668,41 @@ MultiSpinor alloc_multi(const Geom &g, Prec p, int cap, int nb, bool norms) {
   m.lognb = 0;
   while ((1 << m.lognb) < nb) m.lognb++;
   m.stride = g.stride;
-  QQCD_HIP(hipMalloc(&m.data, (size_t)m.elems() * esize(p)));
-  QQCD_HIP(hipMemset(m.data, 0, (size_t)m.elems() * esize(p)));
-  if (p == PREC_HALF && norms) {
-    const size_t nn = (size_t)m.stride * nb * m.nblk();
-    QQCD_HIP(hipMalloc(&m.norm, nn * sizeof(float)));
-    QQCD_HIP(hipMemset(m.norm, 0, nn * sizeof(float)));
+  const hipStream_t s = ctx().stream;
+  try {
+    pool_get(&m.data, (size_t)m.elems() * esize(p));
+    QQCD_HIP(hipMemsetAsync(m.data, 0, (size_t)m.elems() * esize(p), s));
+    if (p == PREC_HALF && norms) {
+      const size_t nn = (size_t)m.stride * nb * m.nblk();
+      pool_get(&m.norm, nn * sizeof(float));
+      QQCD_HIP(hipMemsetAsync(m.norm, 0, nn * sizeof(float), s));
+    }
+  } catch (...) {
+    free_multi(m);
+    throw;
   }
   return m;
 }
 
 void free_multi(MultiSpinor &m) {
-  if (m.data) (void)hipFree(m.data);
-  if (m.norm) (void)hipFree(m.norm);
+  pool_free(m.data);
+  pool_free(m.norm);
   m.data = nullptr;
   m.norm = nullptr;
 }
 
 MBlas::MBlas(hipStream_t s, int cap_) : stream(s), cap(cap_) {}
-MBlas::~MBlas() {
-  if (part) (void)hipFree(part);
-}
+MBlas::~MBlas() { pool_free(part); }
 
 void MBlas::reserve(size_t n) {
   if (n <= part_cap) return;
   // only outside graph capture: the first call of each shape sizes the buffer
   if (part) {
     QQCD_HIP(hipStreamSynchronize(stream));
-    (void)hipFree(part);
+    pool_free(part);
+    part = nullptr;
   }
-  QQCD_HIP(hipMalloc(&part, n * sizeof(double)));
+  pool_get(&part, n * sizeof(double));
   part_cap = n;
 }
 

@@ -882,13 +882,13 @@ NNField alloc_nn(const Geom &g, int C) {
   NNField f;
   f.C = C;
   f.stride = g.stride;
-  QQCD_HIP(hipMalloc(&f.data, f.bytes()));
-  QQCD_HIP(hipMemset(f.data, 0, f.bytes()));
+  pool_get(&f.data, f.bytes());
+  QQCD_HIP(hipMemsetAsync(f.data, 0, f.bytes(), ctx().stream));
   return f;
 }
 
 void free_nn(NNField &f) {
-  if (f.data) (void)hipFree(f.data);
+  pool_free(f.data);
   f.data = nullptr;
 }
 

@@ -1,0 +1,33 @@
+// qqcd_pool.h -- device and pinned host buffers kept between calls.
+//
+// Every solve, operator call and field transfer needs a handful to several
+// hundred temporary fields of a few recurring sizes.  hipMalloc + hipFree of
+// one costs 100-300 us (hipFree waits for the device and unmaps), which for
+// the 50-300 fields of a solve was 60-90 ms: 30% of a 24-source noise loop
+// and half of an FP32 mixed solve at 16^3x32.  A freed buffer therefore goes
+// to a free list of its size and the next request of that size takes it.
+//
+//  * Order: a buffer may be freed while work on it is still queued on the
+//    context's stream; its next user queues on that same stream (the library
+//    has one) or on the null stream, which waits for it.
+//  * Bounds: the free lists hold at most a quarter of the device's memory
+//    (buffers beyond that are released at once); a failed hipMalloc releases
+//    them and tries again; qqcd_init and qqcd_finalize release them all.
+//  * Contents are undefined: a caller that needs zeros clears the buffer.
+//  * Calls from several threads are serialised by a mutex.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+
+namespace qqcd {
+
+void *pool_alloc(size_t bytes);
+void pool_free(void *p);
+void *pool_alloc_host(size_t bytes);  // pinned
+void pool_free_host(void *p);
+void pool_trim();  // releases every free buffer (waits for the device first)
+
+template <typename T> void pool_get(T **p, size_t bytes) { *p = static_cast<T *>(pool_alloc(bytes)); }
+
+}  // namespace qqcd

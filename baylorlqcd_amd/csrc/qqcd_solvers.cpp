@@ -116,14 +116,14 @@ struct DevHess {
   double *x = nullptr;    // paired steps: g2 (ld), the four scalars, the three coefficients
   explicit DevHess(int m_) : m(m_), ld(2 * (m_ + 1)) {
     const size_t n = (size_t)(ld + 1) * m;
-    QQCD_HIP(hipMalloc(&d, sizeof(double) * n));
-    QQCD_HIP(hipMalloc(&x, sizeof(double) * (ld + 8)));
-    QQCD_HIP(hipHostMalloc(&h, sizeof(double) * n, hipHostMallocDefault));
+    pool_get(&d, sizeof(double) * n);
+    pool_get(&x, sizeof(double) * (ld + 8));
+    h = static_cast<double *>(pool_alloc_host(sizeof(double) * n));
   }
   ~DevHess() {
-    if (d) (void)hipFree(d);
-    if (x) (void)hipFree(x);
-    if (h) (void)hipHostFree(h);
+    pool_free(d);
+    pool_free(x);
+    pool_free_host(h);
   }
   double *g2() { return x; }
   double *sc() { return x + ld; }
@@ -297,7 +297,7 @@ static void scaled_copy(Context &c, const Spinor &src, Spinor &dst, double s) {
 
 static void alloc_basis(Context &c, std::vector<Spinor> &V, int n, Prec p) {
   V.resize(n);
-  for (auto &s : V) s = alloc_spinor(c.g, p);
+  for (auto &s : V) s = alloc_spinor(c.g, p, false);  // every vector is written before it is read
 }
 static void free_basis(std::vector<Spinor> &V) {
   for (auto &s : V) free_spinor(s);
@@ -402,7 +402,7 @@ static void store_deflation(Context &c, Deflation *defl, const std::vector<Spino
   defl->H = Hnew;
   defl->V.resize(k + 1);
   for (int q = 0; q <= k; q++) {
-    defl->V[q] = alloc_spinor(c.g, p);
+    defl->V[q] = alloc_spinor(c.g, p, false);
     Vec d = vv(defl->V[q]);
     c.blas->copy(vv(V[q]), d);
   }

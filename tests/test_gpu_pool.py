@@ -1,0 +1,81 @@
+"""Buffers kept between calls: the device memory a program holds stops growing
+after the first pass over its calls, calls that take over used buffers give
+the results of fresh ones bit for bit, and finalize gives the memory back."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from baylorlqcd_amd import _lib, diracops, disconloops, inverters, lattice, quark
+
+pytestmark = pytest.mark.gpu
+
+BC = (1, 1, 1, -1)
+
+
+def free_bytes():
+    return torch.cuda.mem_get_info()[0]
+
+
+def calls(n, seed):
+    """One pass over calls that take fields of several sizes and precisions."""
+    co = O.coact_array()
+    rng = np.random.default_rng(seed)
+    L = int(np.prod(lattice.spinor_shape(n)))
+    b = np.zeros(L)
+    disconloops.z4source(b, None, seed, 0)
+    u = diracops.gauge_get_ref(n)
+    diracops.gauge_load(u, co)
+    x, h, g = np.zeros(L), np.zeros(L), np.zeros(L)
+    inverters.solve_mixed(b, x, (20, 5), 1e-10, 2, 2, 12, 0.0, 0, u, co, (0.14, 0.01), BC)
+    diracops.Hdbletm(h, u, None, b, 0, co, (0.14, 0.01), -1, BC)
+    inverters.gmresdr("", b, g, (20, 5), 1e-10, 0, u, None, -1, (0.14, 0.0), co, BC)
+    nz = disconloops.noise_loop(3, seed, (0.14, 0.0), (20, 4), tol=1e-10, coact=co, bc=BC, nb=2)
+    p = quark.propagator(3, (1, 2, 3, int(rng.integers(1, n[3] + 1))), (0.14, 0.01), (20, 4), solutions=True)
+    return [x, h, g, nz["traces"], *p["xe"]]
+
+
+# 4^4: vectors with padding-free strides down to two wavefronts; 12 x 4 x 4 x 4: 384 sites, 6 wavefronts
+@pytest.mark.parametrize("n", [(4, 4, 4, 4), (12, 4, 4, 4), (8, 8, 8, 16)])
+def test_reused_buffers(n):
+    held = []
+    lattice.init(n, BC)
+    try:
+        diracops.gauge_random(1, 0.1, 7, O.coact_array())
+        want = calls(n, 3)
+        calls(n, 4)
+        for _ in range(3):
+            held.append(free_bytes())
+            got = calls(n, 3)
+            for a, b in zip(got, want):
+                assert np.array_equal(a, b)
+    finally:
+        lattice.finalize()
+    assert abs(held[-1] - held[0]) < 16 << 20, held
+
+
+def test_finalize_returns_memory():
+    n = (8, 8, 8, 16)
+    lattice.init(n, BC)
+    lattice.finalize()
+    start = free_bytes()
+    lattice.init(n, BC)
+    diracops.gauge_random(1, 0.1, 7, O.coact_array())
+    nz = disconloops.noise_loop(8, 5, (0.14, 0.0), (30, 10), tol=1e-10, coact=O.coact_array(), bc=BC)
+    assert np.all(nz["res_full"] < 1e-9)
+    assert start - free_bytes() > 64 << 20  # the loop's fields are held for the next call
+    lattice.finalize()
+    assert start - free_bytes() < 16 << 20
+
+
+def test_failed_allocation_is_an_error():
+    """A lattice larger than the card: the error is reported and the library goes on."""
+    lattice.init((4, 4, 4, 4), BC)
+    try:
+        with pytest.raises(_lib.QQCDError):
+            lattice.init((128, 128, 128, 512), BC)
+    finally:
+        lattice.init((4, 4, 4, 4), BC)
+        diracops.gauge_random(0, 0.0, 1, O.coact_array())
+        assert np.isfinite(diracops.gauge_plaquette())
+        lattice.finalize()
