@@ -1,0 +1,505 @@
+// qqcd_arnoldi.hip -- see qqcd_arnoldi.h.
+#include "qqcd_arnoldi.h"
+
+#include <algorithm>
+#include <stdexcept>
+
+#include "qqcd_pool.h"
+
+namespace qqcd {
+
+typedef std::complex<double> zd;
+
+static constexpr int KV = 4;        // left vectors of a wavefront in the pass of dots
+static constexpr int DW = 8;        // wavefronts of its workgroups at most
+static constexpr int DGRID = 512;   // workgroups along the vector at most
+static constexpr int UB = 256;      // threads of an update workgroup
+
+struct VTab {
+  void *p[BlockArnoldi::NMAX];
+};
+
+// One lane moves 16 bytes of every vector: E complex numbers.
+template <typename T> struct Lane;
+template <> struct Lane<double> {
+  static constexpr int E = 1;
+  static __device__ __forceinline__ void ld(const void *p, long i, double2 (&e)[1]) { e[0] = ((const double2 *)p)[i]; }
+  static __device__ __forceinline__ void st(void *p, long i, const double2 (&e)[1]) { ((double2 *)p)[i] = e[0]; }
+};
+template <> struct Lane<float> {
+  static constexpr int E = 2;
+  static __device__ __forceinline__ void ld(const void *p, long i, double2 (&e)[2]) {
+    const float4 v = ((const float4 *)p)[i];
+    e[0] = make_double2(v.x, v.y);
+    e[1] = make_double2(v.z, v.w);
+  }
+  static __device__ __forceinline__ void st(void *p, long i, const double2 (&e)[2]) {
+    ((float4 *)p)[i] = make_float4((float)e[0].x, (float)e[0].y, (float)e[1].x, (float)e[1].y);
+  }
+};
+
+// part[(chunk * gridDim.x + block) * 2 KV S + 2 (q S + c) + {0, 1}] = <v_{KV chunk + q}, u_c>
+// over the block's lanes, u_c the last S of the nleft vectors.
+//
+// Bound by reading the basis once.  The wavefronts of a workgroup take KV
+// vectors each and the same stretch of the u_c, which so come from memory once
+// per workgroup (up to 32 vectors) and from the L1 for its other wavefronts;
+// KV S = 16 complex FP64 accumulators leave three wavefronts per SIMD.
+template <typename T, int S>
+__global__ void __launch_bounds__(64 * DW) k_bdot(long nu, VTab v, int nleft, double *part) {
+  constexpr int E = Lane<T>::E;
+  const int lane = threadIdx.x & 63;
+  const int chunk = blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int k0 = __builtin_amdgcn_readfirstlane(chunk * KV);
+  if (k0 >= nleft) return;
+  const void *a[KV], *u[S];
+#pragma unroll
+  for (int q = 0; q < KV; q++) a[q] = v.p[k0 + q < nleft ? k0 + q : nleft - 1];
+#pragma unroll
+  for (int c = 0; c < S; c++) u[c] = v.p[nleft - S + c];
+  double acc[2 * KV * S];
+#pragma unroll
+  for (int k = 0; k < 2 * KV * S; k++) acc[k] = 0;
+  for (long i = blockIdx.x * 64L + lane; i < nu; i += gridDim.x * 64L) {
+    double2 b[S][E], e[KV][E];
+#pragma unroll
+    for (int c = 0; c < S; c++) Lane<T>::ld(u[c], i, b[c]);
+#pragma unroll
+    for (int q = 0; q < KV; q++) Lane<T>::ld(a[q], i, e[q]);
+#pragma unroll
+    for (int q = 0; q < KV; q++)
+#pragma unroll
+      for (int c = 0; c < S; c++)
+#pragma unroll
+        for (int x = 0; x < E; x++) {
+          acc[2 * (q * S + c)] += e[q][x].x * b[c][x].x + e[q][x].y * b[c][x].y;
+          acc[2 * (q * S + c) + 1] += e[q][x].x * b[c][x].y - e[q][x].y * b[c][x].x;
+        }
+  }
+  double mine = 0;
+#pragma unroll
+  for (int k = 0; k < 2 * KV * S; k++) {
+    double s = acc[k];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (lane == k) mine = s;
+  }
+  if (lane < 2 * KV * S) part[((long)chunk * gridDim.x + blockIdx.x) * (2 * KV * S) + lane] = mine;
+}
+
+// sums[chunk * nq + q] = sum over the nb blocks, in a fixed order; one workgroup per chunk
+__global__ void __launch_bounds__(1024) k_bsum(int nb, int nq, const double *part, double *sums) {
+  __shared__ double sm[32][33];
+  const int q = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const double *p = part + (long)blockIdx.x * nb * nq + q;
+  double s = 0;
+  if (q < nq) {
+#pragma unroll 4
+    for (int b = g; b < nb; b += 32) s += p[(long)b * nq];
+  }
+  sm[g][q] = s;
+  __syncthreads();
+  // row g now sums column g
+  double c = sm[q][g];
+#pragma unroll
+  for (int o = 16; o > 0; o >>= 1) c += __shfl_xor(c, o, 32);
+  if (q == 0 && g < nq) sums[(long)blockIdx.x * nq + g] = c;
+}
+
+__device__ __forceinline__ double2 zmul(double2 a, double2 b) {
+  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+__device__ __forceinline__ double2 zsub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ double2 zcmul(double2 a, double2 b) {  // conj(a) b
+  return make_double2(a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x);
+}
+
+// The small algebra of a block, one workgroup: from the sums (rows 0..j: P,
+// rows j+1..j+s: G) the factor R, the update coefficients and the columns
+// j..j+s-1 of H, which go to the device matrix and to the host's slot.  again:
+// the vectors are the Q of this block, with P and R of the first pass in pr;
+// the total projections are P + P2 R and the total factor R2 R.
+template <int S>
+__global__ void __launch_bounds__(256) k_bcols(int j, int ld, int again, double least, const double2 *sums,
+                                               double2 *hd, double2 *pr, double2 *coef, double2 *hout, double *info) {
+  constexpr int SM = BlockArnoldi::SMAX, NM = BlockArnoldi::NMAX;
+  __shared__ double2 P[NM][S], C[NM][S], G[S][S], R[S][S], D[S][S], Pt[NM][S], Rt[S][S], col[S][NM + SM];
+  __shared__ double red[2][S];
+  __shared__ int good;
+  __shared__ double worst;
+  const int t = threadIdx.x, nv = j + 1;
+  for (int i = t; i < nv * S; i += 256) P[i / S][i % S] = sums[i];
+  for (int i = t; i < S * S; i += 256) G[i / S][i % S] = sums[(long)nv * S + i];
+  __syncthreads();
+  // G - P^H P, one entry per 16 threads
+  for (int e0 = 0; e0 < S * S; e0 += 16) {
+    const int e = e0 + (t >> 4), r = e / S, c = e % S;
+    double2 a = make_double2(0, 0);
+    if (e < S * S)
+      for (int k = t & 15; k < nv; k += 16) {
+        const double2 p = zcmul(P[k][r], P[k][c]);
+        a.x += p.x;
+        a.y += p.y;
+      }
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) {
+      a.x += __shfl_xor(a.x, o, 64);
+      a.y += __shfl_xor(a.y, o, 64);
+    }
+    if (e < S * S && (t & 15) == 0) R[r][c] = zsub(G[r][c], a);
+  }
+  __syncthreads();
+  if (t == 0) {
+    // Cholesky R^H R of the upper triangle, in place; D = R^-1 (upper)
+    double2 r[S][S], d[S][S];
+    double least_seen = 1.0;
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < S; i++)
+#pragma unroll
+      for (int k = 0; k < S; k++) {
+        r[i][k] = k >= i ? R[i][k] : make_double2(0, 0);
+        d[i][k] = make_double2(0, 0);
+      }
+    bool ok = true;
+#pragma unroll
+    for (int i = 0; i < S; i++) {
+      double p = r[i][i].x;
+#pragma unroll
+      for (int l = 0; l < i; l++) p -= r[l][i].x * r[l][i].x + r[l][i].y * r[l][i].y;
+      const double g = G[i][i].x;
+      ok = ok && p > least * g && p > 0;
+      const double h = ok ? sqrt(p) : 0.0, inv = ok ? 1.0 / h : 0.0;
+      if (ok) {
+        least_seen = fmin(least_seen, p / g);
+        n++;
+      }
+      r[i][i] = make_double2(h, 0);
+#pragma unroll
+      for (int k = i + 1; k < S; k++) {
+        double2 x = r[i][k];
+#pragma unroll
+        for (int l = 0; l < i; l++) x = zsub(x, zcmul(r[l][i], r[l][k]));
+        r[i][k] = make_double2(x.x * inv, x.y * inv);
+      }
+      // column i of the inverse
+      d[i][i] = make_double2(inv, 0);
+#pragma unroll
+      for (int l = i - 1; l >= 0; l--) {
+        double2 x = make_double2(0, 0);
+#pragma unroll
+        for (int q = l + 1; q <= i; q++) {
+          const double2 y = zmul(r[l][q], d[q][i]);
+          x.x += y.x;
+          x.y += y.y;
+        }
+        const double f = ok ? -d[l][l].x : 0.0;
+        d[l][i] = make_double2(x.x * f, x.y * f);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < S; i++)
+#pragma unroll
+      for (int k = 0; k < S; k++) {
+        R[i][k] = r[i][k];
+        D[i][k] = d[i][k];
+      }
+    good = n;
+    worst = least_seen;
+  }
+  __syncthreads();
+  // C = -P D, row by row; with `again` the totals P + P2 R, R2 R
+  double grow[S];
+#pragma unroll
+  for (int c = 0; c < S; c++) grow[c] = 0;
+  if (t < nv) {
+    const int k = t;
+#pragma unroll
+    for (int c = 0; c < S; c++) {
+      double2 a = make_double2(0, 0);
+      for (int l = 0; l <= c; l++) {
+        const double2 x = zmul(P[k][l], D[l][c]);
+        a.x -= x.x;
+        a.y -= x.y;
+      }
+      C[k][c] = a;
+      grow[c] += a.x * a.x + a.y * a.y;
+      double2 p = P[k][c];
+      if (again) {
+        p = pr[k * S + c];
+        for (int l = 0; l <= c; l++) {
+          const double2 x = zmul(P[k][l], pr[nv * S + l * S + c]);
+          p.x += x.x;
+          p.y += x.y;
+        }
+      }
+      Pt[k][c] = p;
+    }
+  }
+  if (t < S * S) {
+    const int r = t / S, c = t % S;
+    double2 x = R[r][c];
+    if (again) {
+      x = make_double2(0, 0);
+      for (int l = r; l <= c; l++) {
+        const double2 y = zmul(R[r][l], pr[nv * S + l * S + c]);
+        x.x += y.x;
+        x.y += y.y;
+      }
+    }
+    Rt[r][c] = x;
+  }
+  __syncthreads();
+  // rows of C sit in the first NMAX = 128 threads: two wavefronts
+#pragma unroll
+  for (int c = 0; c < S; c++) {
+    double s = grow[c];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (t < 128 && (t & 63) == 0) red[t >> 6][c] = s;
+  }
+  __syncthreads();
+  double most = 0;
+#pragma unroll
+  for (int c = 0; c < S; c++) most += red[0][c] + red[1][c];
+  for (int i = t; i < nv * S; i += 256) {
+    coef[i] = C[i / S][i % S];
+    pr[i] = Pt[i / S][i % S];
+  }
+  // the update walks the vectors four at a time
+  for (int i = nv * S + t; i < (nv + 3) / 4 * 4 * S; i += 256) coef[i] = make_double2(0, 0);
+  if (t < S * S) {
+    coef[NM * SM + t] = D[t / S][t % S];
+    pr[nv * S + t] = Rt[t / S][t % S];
+  }
+  // the columns, one after the other: row t of column j + i.  What the old
+  // columns contribute to all of them first (H_k has no rows past k + 1 <= j).
+  double2 old[S];
+#pragma unroll
+  for (int i = 0; i < S; i++) old[i] = make_double2(0, 0);
+  if (S > 1 && t <= j) {
+#pragma unroll 4
+    for (int k = 0; k < j; k++) {
+      const double2 h = hd[t + (long)ld * k];
+#pragma unroll
+      for (int i = 1; i < S; i++) {
+        const double2 x = zmul(Pt[k][i - 1], h);
+        old[i].x += x.x;
+        old[i].y += x.y;
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < S; i++) {
+    const int rows = j + i + 2;
+    if (t < ld) {
+      double2 h = make_double2(0, 0);
+      if (i < good && t < rows) {
+        // coef(u_{i+1}), u_1 first
+        if (t <= j) h = Pt[t][i];
+        else if (t - nv <= i) h = Rt[t - nv][i];
+        if (i > 0) {
+          // B q_i: less what u_i's other components contribute
+          h = zsub(zsub(h, old[i]), zmul(Pt[j][i - 1], col[0][t]));
+#pragma unroll
+          for (int l = 1; l < i; l++) h = zsub(h, zmul(Rt[l - 1][i - 1], col[l][t]));
+          const double inv = 1.0 / Rt[i - 1][i - 1].x;
+          h.x *= inv;
+          h.y *= inv;
+        }
+      }
+      col[i][t] = h;  // read by this thread only
+    }
+  }
+  for (int i = 0; i < S; i++)
+    if (t < ld) {
+      hd[t + (long)ld * (j + i)] = col[i][t];
+      hout[t + (long)ld * i] = col[i][t];
+    }
+  if (t == 0) {
+    info[0] = good;
+    info[1] = sqrt(most);
+    info[2] = worst;
+  }
+}
+
+// v_{nv+c} <- sum_l u_l D_lc + sum_k v_k C_kc, u_l = v_{nv+l} before: Q in place
+// of U.  Bound by reading the basis and U once and writing Q once (a lane's S
+// sums stay in registers over all nv vectors, four vectors' loads ahead); the
+// coefficients are wavefront-uniform and come through scalar loads.
+template <typename T, int S>
+__global__ void __launch_bounds__(UB) k_bupdate(long nu, VTab v, int nv, const double *__restrict__ coef) {
+  constexpr int E = Lane<T>::E;
+  const double *D = coef + 2 * BlockArnoldi::NMAX * BlockArnoldi::SMAX;
+  for (long i = blockIdx.x * (long)UB + threadIdx.x; i < nu; i += (long)gridDim.x * UB) {
+    double2 u[S][E], s[S][E];
+#pragma unroll
+    for (int c = 0; c < S; c++) Lane<T>::ld(v.p[nv + c], i, u[c]);
+#pragma unroll
+    for (int c = 0; c < S; c++)
+#pragma unroll
+      for (int x = 0; x < E; x++) {
+        s[c][x] = make_double2(0, 0);
+#pragma unroll
+        for (int l = 0; l <= c; l++) {
+          const double dr = D[2 * (l * S + c)], di = D[2 * (l * S + c) + 1];
+          s[c][x].x += dr * u[l][x].x - di * u[l][x].y;
+          s[c][x].y += dr * u[l][x].y + di * u[l][x].x;
+        }
+      }
+    for (int k = 0; k < nv; k += 4) {
+      double2 e[4][E];
+#pragma unroll
+      for (int q = 0; q < 4; q++) Lane<T>::ld(v.p[k + q < nv ? k + q : nv - 1], i, e[q]);
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int c = 0; c < S; c++) {
+          const double cr = coef[2 * ((k + q) * S + c)], ci = coef[2 * ((k + q) * S + c) + 1];
+#pragma unroll
+          for (int x = 0; x < E; x++) {
+            s[c][x].x += cr * e[q][x].x - ci * e[q][x].y;
+            s[c][x].y += cr * e[q][x].y + ci * e[q][x].x;
+          }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < S; c++) Lane<T>::st(v.p[nv + c], i, s[c]);
+  }
+}
+
+// ===================================================================== //
+
+static constexpr int CHUNKS = BlockArnoldi::NMAX / KV;
+
+BlockArnoldi::BlockArnoldi(hipStream_t s, int m_) : stream(s), m(m_), ld(m_ + 1) {
+  if (m < 1 || m + 1 > NMAX) throw std::runtime_error("BlockArnoldi: at most 127 steps");
+  const int slots = m;  // one per block at least
+  pool_get(&hd, sizeof(double) * 2 * ld * m);
+  pool_get(&part, sizeof(double) * 2 * KV * SMAX * DGRID * CHUNKS);
+  pool_get(&sums, sizeof(double) * 2 * KV * SMAX * CHUNKS);
+  pool_get(&pr, sizeof(double) * 2 * SMAX * (NMAX + SMAX));
+  pool_get(&coef, sizeof(double) * 2 * SMAX * (NMAX + SMAX));
+  hh = static_cast<double *>(pool_alloc_host(sizeof(double) * slot_len() * slots));
+}
+
+BlockArnoldi::~BlockArnoldi() {
+  (void)hipStreamSynchronize(stream);  // a queued block still writes to the pinned slots
+  pool_free(hd);
+  pool_free(part);
+  pool_free(sums);
+  pool_free(pr);
+  pool_free(coef);
+  pool_free_host(hh);
+}
+
+void BlockArnoldi::load(const zd *h, int ldh, int n, double sigma) {
+  if (n < 0 || n > m) throw std::runtime_error("BlockArnoldi: too many columns");
+  if (n == 0) return;
+  std::vector<zd> a((size_t)ld * n, 0.0);
+  for (int q = 0; q < n; q++)
+    for (int i = 0; i <= n; i++) a[i + (size_t)ld * q] = h[i + (size_t)ldh * q] - (i == q ? sigma : 0.0);
+  QQCD_HIP(hipMemcpyAsync(hd, a.data(), sizeof(zd) * a.size(), hipMemcpyHostToDevice, stream));
+  QQCD_HIP(hipStreamSynchronize(stream));
+}
+
+void BlockArnoldi::put(const zd *h, int j, double sigma) {
+  if (j < 0 || j >= m) throw std::runtime_error("BlockArnoldi: no such column");
+  std::vector<zd> a(ld, 0.0);
+  for (int i = 0; i <= j + 1; i++) a[i] = h[i] - (i == j ? sigma : 0.0);
+  QQCD_HIP(hipMemcpyAsync(hd + 2L * ld * j, a.data(), sizeof(zd) * ld, hipMemcpyHostToDevice, stream));
+  QQCD_HIP(hipStreamSynchronize(stream));
+}
+
+template <typename F> static void with_s(int s, F &&f) {
+  switch (s) {
+    case 1: f(std::integral_constant<int, 1>()); break;
+    case 2: f(std::integral_constant<int, 2>()); break;
+    case 3: f(std::integral_constant<int, 3>()); break;
+    case 4: f(std::integral_constant<int, 4>()); break;
+    default: throw std::runtime_error("BlockArnoldi: 1..4 steps a block");
+  }
+}
+
+void BlockArnoldi::run(const Vec *V, int j, int s, int slot, bool again) {
+  if (j < 0 || s < 1 || s > SMAX || j + s > m || slot < 0 || slot >= m) throw std::runtime_error("BlockArnoldi: bad block");
+  const int nleft = j + 1 + s;
+  VTab tab{};
+  for (int q = 0; q < nleft; q++) {
+    if (V[q].prec != V[0].prec || V[q].n != V[0].n) throw std::runtime_error("BlockArnoldi: mixed vectors");
+    tab.p[q] = V[q].data;
+  }
+  const long n = V[0].n;
+  double *slot_h = hh + slot_len() * slot;
+  auto go = [&](auto tag) {
+    typedef decltype(tag) T;
+    constexpr int E = Lane<T>::E;
+    if (n % E) throw std::runtime_error("BlockArnoldi: odd vector length");
+    const long nu = n / E;
+    const int chunks = (nleft + KV - 1) / KV, ny = (chunks + DW - 1) / DW, w = (chunks + ny - 1) / ny;
+    // about 3000 wavefronts in flight; no more workgroups than 64-lane stretches
+    const int gx = (int)std::max(1L, std::min({(nu + 63) / 64, (long)DGRID, 3072L / (long)(w * ny) + 1}));
+    const int gu = (int)std::min((nu + UB - 1) / UB, 2048L);
+    with_s(s, [&](auto SS) {
+      constexpr int S = decltype(SS)::value;
+      hipLaunchKernelGGL((k_bdot<T, S>), dim3(gx, ny), dim3(64 * w), 0, stream, nu, tab, nleft, part);
+      hipLaunchKernelGGL(k_bsum, dim3(chunks), dim3(1024), 0, stream, gx, 2 * KV * S, part, sums);
+      // a vector is taken while at least 1e-9 (FP64; FP32: 1e-10, its rounding squared being 4e-15) of its
+      // squared norm is left
+      hipLaunchKernelGGL((k_bcols<S>), dim3(1), dim3(256), 0, stream, j, ld, again ? 1 : 0,
+                         sizeof(T) == 8 ? 1e-9 : 1e-10, (const double2 *)sums, (double2 *)hd, (double2 *)pr,
+                         (double2 *)coef, (double2 *)slot_h, slot_h + 2L * SMAX * ld);
+      hipLaunchKernelGGL((k_bupdate<T, S>), dim3(gu), dim3(UB), 0, stream, nu, tab, j + 1, coef);
+    });
+    QQCD_HIP(hipGetLastError());
+  };
+  if (V[0].prec == PREC_DOUBLE) go(double());
+  else if (V[0].prec == PREC_SINGLE) go(float());
+  else throw std::runtime_error("BlockArnoldi: FP64 or FP32 vectors");
+}
+
+void BlockArnoldi::queue(const Vec *V, int j, int s, int slot) { run(V, j, s, slot, false); }
+void BlockArnoldi::queue_again(const Vec *V, int j, int s, int slot) { run(V, j, s, slot, true); }
+
+double BlockArnoldi::loss_of(const Vec *V, int n) {
+  if (n < 1 || n > NMAX || V[0].prec != PREC_DOUBLE) throw std::runtime_error("BlockArnoldi: FP64 vectors");
+  VTab tab{};
+  for (int q = 0; q < n; q++) tab.p[q] = V[q].data;
+  std::vector<zd> g((size_t)KV * SMAX * CHUNKS);
+  double f = 0;
+  // the upper triangle, SMAX columns at a time (the last columns again where n is not a multiple)
+  for (int c0 = 0; c0 < n; c0 += SMAX) {
+    const int nleft = std::min(n, c0 + SMAX), first = std::max(0, nleft - SMAX);
+    const int chunks = (nleft + KV - 1) / KV, ny = (chunks + DW - 1) / DW, w = (chunks + ny - 1) / ny;
+    const int s = nleft - first, gx = (int)std::min({(V[0].n + 63) / 64, (long)DGRID, 3072L / (w * ny) + 1});
+    with_s(s, [&](auto SS) {
+      constexpr int S = decltype(SS)::value;
+      hipLaunchKernelGGL((k_bdot<double, S>), dim3(gx, ny), dim3(64 * w), 0, stream, V[0].n, tab, nleft, part);
+      hipLaunchKernelGGL(k_bsum, dim3(chunks), dim3(1024), 0, stream, gx, 2 * KV * S, part, sums);
+    });
+    QQCD_HIP(hipGetLastError());
+    QQCD_HIP(hipMemcpyAsync(g.data(), sums, sizeof(zd) * nleft * s, hipMemcpyDeviceToHost, stream));
+    QQCD_HIP(hipStreamSynchronize(stream));
+    for (int q = 0; q < nleft; q++)
+      for (int c = std::max(c0, q); c < nleft; c++) {
+        const zd e = g[(size_t)q * s + c - first] - (q == c ? 1.0 : 0.0);
+        f += (q == c ? 1.0 : 2.0) * std::norm(e);
+      }
+  }
+  return std::sqrt(f);
+}
+
+int BlockArnoldi::fetch(int slot, int j, int s, double sigma, zd *H, int ldh) const {
+  const double *a = hh + slot_len() * slot, *info = a + 2L * SMAX * ld;
+  const int good = std::min(s, (int)info[0]);
+  for (int i = 0; i < good; i++)
+    for (int r = 0; r <= j + i + 1; r++)
+      H[r + (size_t)ldh * (j + i)] =
+          zd(a[2 * (r + (size_t)ld * i)], a[2 * (r + (size_t)ld * i) + 1]) + (r == j + i ? sigma : 0.0);
+  return good;
+}
+
+double BlockArnoldi::growth(int slot) const { return hh[slot_len() * slot + 2L * SMAX * ld + 1]; }
+double BlockArnoldi::pivot(int slot) const { return hh[slot_len() * slot + 2L * SMAX * ld + 2]; }
+
+}  // namespace qqcd

@@ -142,7 +142,7 @@ void ensure_gauge(Context &c, const double *u_ref, const double *coact) {
 }
 
 void schur_apply(Context &c, const Gauge &U, const double kappa[2], int idag, const Spinor &in, Spinor &out,
-                 Spinor &tmp_odd, Spinor *out32, bool only32) {
+                 Spinor &tmp_odd, Spinor *out32, bool only32, bool less_diag) {
   const double k = kappa[0], mu = kappa[1];
   Epilogue e1, e2;
   if (mu < 1e-8) {
@@ -156,8 +156,10 @@ void schur_apply(Context &c, const Gauge &U, const double kappa[2], int idag, co
     e2.a1 = 2.0 * mu / k;
     e2.b0 = -1.0 / (1.0 + a * a);
   }
+  if (less_diag) e2.a0 = 0;
+  const bool own = e2.a0 != 0 || e2.a1 != 0;
   dslash(c.g, U, in, tmp_odd, 1, idag, e1, nullptr, c.stream);
-  dslash(c.g, U, tmp_odd, out, 0, idag, e2, &in, c.stream, out32, only32);
+  dslash(c.g, U, tmp_odd, out, 0, idag, e2, own ? &in : nullptr, c.stream, out32, only32);
 }
 
 }  // namespace qqcd

@@ -22,6 +22,8 @@
 // early when its least-squares residual already meets the tolerance.
 #include "qqcd_solvers.h"
 
+#include "qqcd_arnoldi.h"
+
 #include <cmath>
 #include <memory>
 #include <stdexcept>
@@ -285,6 +287,64 @@ static void arnoldi_steps_dev(Context &c, LinOp &A, std::vector<Spinor> &V, int 
   e.e = nullptr;
 }
 
+// Arnoldi steps j .. j + want - 1 in blocks over an FP64 or FP32 basis
+// (qqcd_arnoldi.h), the columns into H; returns how many were made.  A block
+// reads the basis twice whatever its length, where a step of its own with the
+// DGKS test read it four times.
+//
+// Four steps a block: the smallest R_ii^2 / G_ii is 0.077 (two steps: 0.38), so
+// R^-1 costs a factor of 3.6 in rounding; the same Krylov steps as one at a
+// time in FP64 and FP32.  24^3x48 GMRES-DR(40,16): 522 ms one at a time,
+// 188 ms in blocks; 16^3x32 GMRES-DR(60,20) and GMRES-Proj(40): 279 -> 89 ms;
+// 16^3x32 FP32 mixed solve: 56.5 ms, 38.9 (blocks of two), 37.6 (four).
+//
+// keep (FP64): `loss` bounds ||E||, E = V^H V - 1 (Frobenius).  A block adds
+// V^H Q = -E P R^-1 twice and the rounding of G over what the cancellation
+// left, which at ||P R^-1|| = 0.8 is a factor of 1.5 a block.  Where the bound
+// passes 1e-8, the square root of the rounding unit, below which H is the
+// projection of A to rounding all the same (H. D. Simon, Math. Comp. 42 (1984)
+// 115, semiorthogonality), the block is orthogonalised a second time; a
+// restart past 1e-10 takes the true value instead, which is near rounding.
+// A block whose first vector cancels to below 9 digits is done step by step.
+static int arnoldi_blocks(Context &c, LinOp &A, std::vector<Spinor> &V, int j, int want, BlockArnoldi &ba, bool keep,
+                          double &loss, std::vector<zd> &H, int ldh, bool &ended) {
+  const int S = BlockArnoldi::SMAX;
+  std::vector<Vec> Vb = vecs(V, j + want + 1);
+  int n = 0;
+  for (int q = j; q < j + want; n++) {
+    const int s = std::min(S, j + want - q);
+    for (int i = 0; i < s; i++) A.apply_less(V[q + i], V[q + i + 1]);
+    ba.queue(Vb.data(), q, s, n);
+    q += s;
+  }
+  QQCD_HIP(hipStreamSynchronize(c.stream));
+  int q = j;
+  for (int b = 0; b < n; b++) {
+    const int s = std::min(S, j + want - q);
+    const int good = ba.fetch(b, q, s, A.sigma, H.data(), ldh);
+    const double g = ba.growth(b);
+    double after = std::hypot(loss * std::sqrt(1.0 + 2.0 * g * g), 1e-15 / ba.pivot(b));
+    if (keep && good == s && after > 1e-8) {
+      ba.queue_again(Vb.data(), q, s, b);
+      QQCD_HIP(hipStreamSynchronize(c.stream));
+      if (ba.fetch(b, q, s, A.sigma, H.data(), ldh) != s) return q - j;
+      after = std::max(loss, 1e-14);
+    }
+    loss = after;
+    q += good;
+    if (good == s) continue;
+    if (q == j) {
+      std::vector<zd> col(j + 2);
+      ended = arnoldi_step(c, A, V, j, col.data(), 1) == 0.0;
+      for (int i = 0; i <= j + 1; i++) H[i + (size_t)ldh * j] = col[i];
+      ba.put(col.data(), j, A.sigma);
+      q++;
+    }
+    break;
+  }
+  return q - j;
+}
+
 // dst = s * src across precisions (an FP16 destination through the conversion)
 static void scaled_copy(Context &c, const Spinor &src, Spinor &dst, double s) {
   if (dst.prec == PREC_HALF || src.prec == PREC_HALF) {
@@ -408,6 +468,38 @@ static void store_deflation(Context &c, Deflation *defl, const std::vector<Spino
   }
 }
 
+// whether a solve runs its Arnoldi steps in blocks: the basis in the work
+// precision, FP64 or FP32, an operator without its diagonal, no
+// preconditioner and no hook that wants every step
+static bool block_steps(const LinOp &A, int m, const LinOp *M, const StepHook *step_hook) {
+  return g_arnoldi_steps == 2 && g_step_graphs != 1 && A.apply_less && A.basis() == A.prec &&
+         (A.prec == PREC_DOUBLE || A.prec == PREC_SINGLE) && !M && !(step_hook && *step_hook) &&
+         m + 1 <= BlockArnoldi::NMAX;
+}
+
+// The least-squares residual after columns j + 1 .. j + got: true once it is
+// below goal with at least `more` of these steps taken, got then cut to the
+// first such column (every column's residual is looked at only in the block
+// that gets there, or where res wants them all).
+static bool first_enough(const std::vector<zd> &H, int ldh, const std::vector<zd> &cv, std::vector<zd> &y, int j,
+                         int &got, double goal, int more, std::vector<double> *res = nullptr) {
+  if (got < 1) return false;
+  auto at = [&](int q) { return dense::lsq(j + q + 1, j + q, H.data(), ldh, cv.data(), y.data()); };
+  const double last = at(got);
+  const bool done = last < goal && got >= more;
+  const int n = got;
+  if (!done && !res) return false;
+  for (int q = 1; q <= n; q++) {
+    const double r = q < n ? at(q) : last;
+    if (res) res->push_back(r);
+    if (done && r < goal && q >= more) {
+      got = q;
+      break;
+    }
+  }
+  return done;
+}
+
 SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int k, double tol, int itermin,
                    int maxiter, Deflation *defl, int reorth, LinOp *M, const CycleHook *hook,
                    const StepHook *step_hook) {
@@ -428,8 +520,12 @@ SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int 
   if (vp != p) work.reset(new SpinorBuf(c.g, p));
   // paired Arnoldi steps: one Gram-Schmidt pass, FP32 work over an FP16 basis
   if (g_arnoldi_steps == 2 && !reorth && !M && p == PREC_SINGLE && vp == PREC_HALF) work2.reset(new SpinorBuf(c.g, p));
+  const bool blocks = block_steps(A, m, M, step_hook);
   std::unique_ptr<DevHess> dh;
-  if (!reorth) dh.reset(new DevHess(m));
+  if (!reorth && !blocks) dh.reset(new DevHess(m));
+  std::unique_ptr<BlockArnoldi> ba;
+  if (blocks) ba.reset(new BlockArnoldi(c.stream, m));
+  double loss = 0;
   std::unique_ptr<StepGraphs> sg;
   if (dh && !M && g_step_graphs == 1) sg.reset(new StepGraphs);
   std::vector<zd> Zmat;
@@ -447,12 +543,23 @@ SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int 
   scaled_copy(c, r.s, V[0], 1.0 / rn);
   cv[0] = rn;
   int j = 0;
-  bool have_defl = false;
+  bool have_defl = false, restarted = false;  // V[0..k], Hnew: the deflation space of the last restart
   std::vector<zd> Hnew, cnew;
   for (;;) {
     // Arnoldi
     int jchk = j;
     while (j < m) {
+      if (ba) {
+        bool ended = false;
+        const int want = std::min(std::min(kCheck, m - j), std::max(1, maxiter - st.iters));
+        int got = arnoldi_blocks(c, A, V, j, want, *ba, reorth != 0, loss, H, ldh, ended);
+        const bool done = first_enough(H, ldh, cv, y, j, got, tol * r0, itermin - st.iters);
+        st.matvecs += got;
+        st.iters += got;
+        j += got;
+        if (done || ended || st.iters >= maxiter) break;
+        continue;
+      }
       if (dh) {
         if (sg || work2) {
           const int n = std::min(std::min(kCheck, m - j), std::max(1, maxiter - st.iters));
@@ -507,7 +614,9 @@ SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int 
     if (done) {
       st.converged = rn < tol * r0;
       // keep the harmonic Ritz space of the final cycle for later right-hand sides
-      if (defl && j > k && k > 0 && deflate(c, V, W, j, k, H, ldh, cv, y, Hnew, cnew)) {
+      // (or of the last restart, whose vectors are still V[0..k], where this cycle was too short)
+      if (defl && j > k && k > 0 && deflate(c, V, W, j, k, H, ldh, cv, y, Hnew, cnew)) restarted = true;
+      if (defl && restarted) {
         store_deflation(c, defl, V, k, Hnew, vp);
         have_defl = true;
       }
@@ -527,17 +636,24 @@ SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int 
         for (int i = 0; i <= k; i++) H[i + (size_t)ldh * q] = Hnew[i + (size_t)(k + 1) * q];
       for (int i = 0; i <= k; i++) cv[i] = cnew[i];
       j = k;
-      if (defl) {
-        store_deflation(c, defl, V, k, Hnew, vp);
-        have_defl = true;
+      restarted = true;
+      if (ba) {
+        ba->load(Hnew.data(), k + 1, k, A.sigma);
+        if (reorth && loss > 1e-10) loss = ba->loss_of(vecs(V, k + 1).data(), k + 1);
       }
     } else {
       // plain restart from the true residual
+      if (defl && restarted) {
+        store_deflation(c, defl, V, k, Hnew, vp);
+        have_defl = true;
+      }
+      restarted = false;
       scaled_copy(c, r.s, V[0], 1.0 / rn);
       std::fill(H.begin(), H.end(), zd(0.0));
       std::fill(cv.begin(), cv.end(), zd(0.0));
       cv[0] = rn;
       j = 0;
+      loss = 0;
     }
   }
 }
@@ -561,14 +677,15 @@ SolveStats gmresproj(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, co
   StepGraphs *sg = nullptr;
   // paired Arnoldi steps: one Gram-Schmidt pass, FP32 work over an FP16 basis
   const bool pairs = g_arnoldi_steps == 2 && !reorth && p == PREC_SINGLE && vp == PREC_HALF;
+  const bool blocks = block_steps(A, m, nullptr, nullptr);
+  const bool dev = !reorth && !blocks;
   if (ws) {
-    if (ws->m != m || ws->p != p || ws->vp != vp || (!reorth) != (ws->dh != nullptr) ||
-        pairs != (ws->work2 != nullptr)) {
+    if (ws->m != m || ws->p != p || ws->vp != vp || dev != (ws->dh != nullptr) || pairs != (ws->work2 != nullptr)) {
       ws->reset();
       alloc_basis(c, ws->V, m + 1, vp);
       if (vp != p) ws->work.reset(new SpinorBuf(c.g, p));
       if (pairs) ws->work2.reset(new SpinorBuf(c.g, p));
-      if (!reorth) ws->dh.reset(new DevHess(m));
+      if (dev) ws->dh.reset(new DevHess(m));
       ws->m = m;
       ws->p = p;
       ws->vp = vp;
@@ -584,7 +701,7 @@ SolveStats gmresproj(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, co
     alloc_basis(c, Vown, m + 1, vp);
     if (vp != p) work_own.reset(new SpinorBuf(c.g, p));
     if (pairs) work2_own.reset(new SpinorBuf(c.g, p));
-    if (!reorth) dh_own.reset(new DevHess(m));
+    if (dev) dh_own.reset(new DevHess(m));
     if (dh_own && g_step_graphs == 1) sg_own.reset(new StepGraphs);
     work = work_own.get();
     work2 = work2_own.get();
@@ -592,6 +709,8 @@ SolveStats gmresproj(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, co
     sg = sg_own.get();
   }
   std::vector<Spinor> &V = *Vp;
+  std::unique_ptr<BlockArnoldi> ba;
+  if (blocks) ba.reset(new BlockArnoldi(c.stream, m));
   SpinorBuf r(c.g, p);
   double rn = residual(c, A, b, x, r.s, st);
   const double r0 = rn;
@@ -624,7 +743,21 @@ SolveStats gmresproj(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, co
     scaled_copy(c, r.s, V[0], 1.0 / rn);
     cv[0] = rn;
     int j = 0, jchk = 0;
+    double loss = 0;
     while (j < m) {
+      if (ba) {
+        bool ended = false;
+        const int want = std::min(std::min(kCheck, m - j), std::max(1, maxiter - st.iters));
+        int got = arnoldi_blocks(c, A, V, j, want, *ba, reorth != 0, loss, H, ldh, ended);
+        std::vector<double> res;
+        const bool done = first_enough(H, ldh, cv, y, j, got, tol * r0, itermin - st.iters, hist ? &res : nullptr);
+        for (size_t q = 0; q < res.size(); q++) hist->emplace_back(st.matvecs + 1 + (int)q, res[q]);
+        st.matvecs += got;
+        st.iters += got;
+        j += got;
+        if (done || ended || st.iters >= maxiter) break;
+        continue;
+      }
       if (dh) {
         if (sg || work2) {
           const int n = std::min(std::min(kCheck, m - j), std::max(1, maxiter - st.iters));
@@ -799,6 +932,18 @@ MixedStats solve_mixed(Context &c, const double kappa[2], const Spinor &b, Spino
         spinor_copy_convert(c.g, out_lo->s, r, c.stream);
       }
     };
+    if (work == PREC_SINGLE && (op_prec == PREC_SINGLE || direct32)) {
+      o.sigma = Alo->diag();
+      o.apply_less = [&, direct32](const Spinor &a, Spinor &r) {
+        const Spinor *in = &a;
+        if (a.prec != op_prec) {
+          spinor_copy_convert(c.g, a, in_lo->s, c.stream);
+          in = &in_lo->s;
+        }
+        if (direct32) (*Alo)(*in, out_lo->s, &r, true, true);
+        else (*Alo)(*in, r, nullptr, false, true);
+      };
+    }
     if (direct32) {
       // r1 = A a in FP32 and, rounded to FP16 by the same launch, the input
       // of r2 = A r1: the operator reads its input in FP16, so r2 is A

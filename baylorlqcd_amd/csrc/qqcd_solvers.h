@@ -23,6 +23,11 @@ struct LinOp {
   // optional: r1 = A a, r2 = A r1 in one call (an operator that rounds its
   // input to a lower storage precision can then pass its own rounded r1 on)
   std::function<void(const Spinor &, Spinor &, Spinor &)> apply_sq;
+  // optional: r = (A - sigma) a, the operator without its multiple of the
+  // identity: the same Krylov space, without the cancellation of that part
+  // in every orthogonalisation
+  std::function<void(const Spinor &, Spinor &)> apply_less;
+  double sigma = 0;
   Prec basis() const { return store < 0 ? prec : (Prec)store; }
 };
 
@@ -38,13 +43,17 @@ struct SchurOp {
     kappa[0] = k[0];
     kappa[1] = k[1];
   }
-  void operator()(const Spinor &in, Spinor &out, Spinor *out32 = nullptr, bool only32 = false) {
-    schur_apply(c, U, kappa, idag, in, out, tmp.s, out32, only32);
+  void operator()(const Spinor &in, Spinor &out, Spinor *out32 = nullptr, bool only32 = false,
+                  bool less_diag = false) {
+    schur_apply(c, U, kappa, idag, in, out, tmp.s, out32, only32, less_diag);
   }
+  double diag() const { return 1.0 / (kappa[0] * kappa[0]); }
   LinOp op() {
     LinOp o;
     o.prec = tmp.s.prec;
     o.apply = [this](const Spinor &a, Spinor &b) { (*this)(a, b); };
+    o.apply_less = [this](const Spinor &a, Spinor &b) { (*this)(a, b, nullptr, false, true); };
+    o.sigma = diag();
     return o;
   }
 };

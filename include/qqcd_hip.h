@@ -426,7 +426,9 @@ int qqcd_batch_set(int reorth, int use_graph, double inner_tol, int inner_cycles
  * of both in one pass each over the basis, column j + 1 of the Hessenberg
  * matrix from the Arnoldi relation -- where one Gram-Schmidt pass (and, in
  * the batched solver, the two-slot operator and an even cycle length)
- * allows it; 1 one step at a time.  Tuning aid; no reference counterpart. */
+ * allows it; 1 one step at a time.  The single-right-hand-side solvers over
+ * an FP64 or FP32 basis run four steps per pair of passes with 2, one with 1.
+ * Tuning aid; no reference counterpart. */
 int qqcd_set_arnoldi_steps(int steps);
 
 /* Paired Arnoldi steps of the batched solver: 1 (the default) takes the norm
