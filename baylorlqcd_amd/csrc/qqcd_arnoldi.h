@@ -1,4 +1,4 @@
-// qqcd_arnoldi.h -- Arnoldi steps in blocks of s over an FP64 or FP32 basis.
+// qqcd_arnoldi.h -- Arnoldi steps in blocks of s over an FP64, FP32 or FP16 basis.
 //
 // With B = A - sigma (the operator without its identity part, the same Krylov
 // space) and u_i = B^i v_j, i = 1..s, one pass over the basis forms the
@@ -33,6 +33,8 @@ class BlockArnoldi {
   // queue block `slot` (0..): V[j+1..j+s] hold B^i V[j] and become the next s
   // basis vectors.  No synchronisation.
   void queue(const Vec *V, int j, int s, int slot);
+  // the same over an FP16 basis with per-site norms; the B^i V[j] are the FP32 U[0..s-1]
+  void queue_half(const Vec *V, const Vec *U, int j, int s, int slot);
   // the same vectors orthogonalised once more, the columns corrected
   void queue_again(const Vec *V, int j, int s, int slot);
   // after the stream has been waited for: columns j.. of H (of A) from block
@@ -55,6 +57,7 @@ class BlockArnoldi {
   double *sums = nullptr;  // their totals: left vectors x s, complex
   double *pr = nullptr;    // P and R of the last block (for queue_again)
   double *coef = nullptr;  // update coefficients: C (NMAX x SMAX), D (SMAX x SMAX), complex
+  float *coef32 = nullptr;  // the same in FP32
   double *hh = nullptr;    // pinned: slots of SMAX columns of ld, then 4 numbers
   long slot_len() const { return 2L * SMAX * ld + 4; }
 };

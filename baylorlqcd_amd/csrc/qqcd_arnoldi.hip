@@ -45,6 +45,7 @@ template <> struct Lane<float> {
 // vectors each and the same stretch of the u_c, which so come from memory once
 // per workgroup (up to 32 vectors) and from the L1 for its other wavefronts;
 // KV S = 16 complex FP64 accumulators leave three wavefronts per SIMD.
+// 24^3x48, FP64, S = 4 over 32 vectors on average: 419 us, 5.4 TB/s.
 template <typename T, int S>
 __global__ void __launch_bounds__(64 * DW) k_bdot(long nu, VTab v, int nleft, double *part) {
   constexpr int E = Lane<T>::E;
@@ -115,13 +116,14 @@ __device__ __forceinline__ double2 zcmul(double2 a, double2 b) {  // conj(a) b
 }
 
 // The small algebra of a block, one workgroup: from the sums (rows 0..j: P,
-// rows j+1..j+s: G) the factor R, the update coefficients and the columns
+// rows g0..g0+s-1: G) the factor R, the update coefficients and the columns
 // j..j+s-1 of H, which go to the device matrix and to the host's slot.  again:
 // the vectors are the Q of this block, with P and R of the first pass in pr;
 // the total projections are P + P2 R and the total factor R2 R.
 template <int S>
-__global__ void __launch_bounds__(256) k_bcols(int j, int ld, int again, double least, const double2 *sums,
-                                               double2 *hd, double2 *pr, double2 *coef, double2 *hout, double *info) {
+__global__ void __launch_bounds__(256) k_bcols(int j, int ld, int again, int g0, double least, const double2 *sums,
+                                               double2 *hd, double2 *pr, double2 *coef, float2 *coef32, double2 *hout,
+                                               double *info) {
   constexpr int SM = BlockArnoldi::SMAX, NM = BlockArnoldi::NMAX;
   __shared__ double2 P[NM][S], C[NM][S], G[S][S], R[S][S], D[S][S], Pt[NM][S], Rt[S][S], col[S][NM + SM];
   __shared__ double red[2][S];
@@ -129,7 +131,7 @@ __global__ void __launch_bounds__(256) k_bcols(int j, int ld, int again, double 
   __shared__ double worst;
   const int t = threadIdx.x, nv = j + 1;
   for (int i = t; i < nv * S; i += 256) P[i / S][i % S] = sums[i];
-  for (int i = t; i < S * S; i += 256) G[i / S][i % S] = sums[(long)nv * S + i];
+  for (int i = t; i < S * S; i += 256) G[i / S][i % S] = sums[(long)g0 * S + i];
   __syncthreads();
   // G - P^H P, one entry per 16 threads
   for (int e0 = 0; e0 < S * S; e0 += 16) {
@@ -263,13 +265,20 @@ __global__ void __launch_bounds__(256) k_bcols(int j, int ld, int again, double 
 #pragma unroll
   for (int c = 0; c < S; c++) most += red[0][c] + red[1][c];
   for (int i = t; i < nv * S; i += 256) {
-    coef[i] = C[i / S][i % S];
+    const double2 x = C[i / S][i % S];
+    coef[i] = x;
+    coef32[i] = make_float2((float)x.x, (float)x.y);
     pr[i] = Pt[i / S][i % S];
   }
   // the update walks the vectors four at a time
-  for (int i = nv * S + t; i < (nv + 3) / 4 * 4 * S; i += 256) coef[i] = make_double2(0, 0);
+  for (int i = nv * S + t; i < (nv + 3) / 4 * 4 * S; i += 256) {
+    coef[i] = make_double2(0, 0);
+    coef32[i] = make_float2(0, 0);
+  }
   if (t < S * S) {
-    coef[NM * SM + t] = D[t / S][t % S];
+    const double2 x = D[t / S][t % S];
+    coef[NM * SM + t] = x;
+    coef32[NM * SM + t] = make_float2((float)x.x, (float)x.y);
     pr[nv * S + t] = Rt[t / S][t % S];
   }
   // the columns, one after the other: row t of column j + i.  What the old
@@ -326,7 +335,8 @@ __global__ void __launch_bounds__(256) k_bcols(int j, int ld, int again, double 
 // v_{nv+c} <- sum_l u_l D_lc + sum_k v_k C_kc, u_l = v_{nv+l} before: Q in place
 // of U.  Bound by reading the basis and U once and writing Q once (a lane's S
 // sums stay in registers over all nv vectors, four vectors' loads ahead); the
-// coefficients are wavefront-uniform and come through scalar loads.
+// coefficients are wavefront-uniform and come through scalar loads.  24^3x48,
+// FP64, S = 4: 448 us, 5.1 TB/s.
 template <typename T, int S>
 __global__ void __launch_bounds__(UB) k_bupdate(long nu, VTab v, int nv, const double *__restrict__ coef) {
   constexpr int E = Lane<T>::E;
@@ -368,9 +378,182 @@ __global__ void __launch_bounds__(UB) k_bupdate(long nu, VTab v, int nv, const d
   }
 }
 
+// ---- an FP16 basis with per-site norms, the block's u_c in FP32 ----------
+
+struct NTab {
+  float *n[BlockArnoldi::NMAX];
+};
+struct UTab {
+  const void *p[BlockArnoldi::SMAX];
+};
+typedef f16 h2v __attribute__((ext_vector_type(2)));
+typedef f16 h8v __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ void ld4(const void *p, long i, float2 (&e)[4]) {
+  const float4 a = ((const float4 *)p)[2 * i], b = ((const float4 *)p)[2 * i + 1];
+  e[0] = make_float2(a.x, a.y);
+  e[1] = make_float2(a.z, a.w);
+  e[2] = make_float2(b.x, b.y);
+  e[3] = make_float2(b.z, b.w);
+}
+// k_bdot for an FP16 basis: the chunks of KV basis vectors, and after them one
+// of the u_c themselves (G).  A lane takes four consecutive sites and walks
+// their 12 component runs (nq = stride / 4 site quads), so each vector's norms
+// are read once; 16 bytes of a vector a lane.  Sums in FP32 within a lane (the
+// basis carries 11 bits), in FP64 across lanes.
+template <int S>
+__global__ void __launch_bounds__(64 * DW) k_bdot_h(long nq, VTab v, NTab vn, UTab ut, int nv, double *part) {
+  const int lane = threadIdx.x & 63, cv = (nv + KV - 1) / KV;
+  const int chunk = __builtin_amdgcn_readfirstlane(blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6));
+  if (chunk > cv) return;
+  float af[2 * KV * S];
+#pragma unroll
+  for (int k = 0; k < 2 * KV * S; k++) af[k] = 0.f;
+  auto add = [&](const float2(&e)[4], const float2(&b)[S][4], int q) {
+#pragma unroll
+    for (int c = 0; c < S; c++)
+#pragma unroll
+      for (int x = 0; x < 4; x++) {
+        af[2 * (q * S + c)] += e[x].x * b[c][x].x + e[x].y * b[c][x].y;
+        af[2 * (q * S + c) + 1] += e[x].x * b[c][x].y - e[x].y * b[c][x].x;
+      }
+  };
+  if (chunk < cv) {
+    const int k0 = chunk * KV;
+    const void *pv[KV];
+#pragma unroll
+    for (int k = 0; k < KV; k++) pv[k] = v.p[k0 + k < nv ? k0 + k : nv - 1];
+    for (long q = blockIdx.x * 64L + lane; q < nq; q += gridDim.x * 64L) {
+      float4 m[KV], ub[2 * S];
+      h8v vb[KV];
+      auto fetch = [&](long i) {
+#pragma unroll
+        for (int k = 0; k < KV; k++) vb[k] = ((const h8v *)pv[k])[i];
+#pragma unroll
+        for (int c = 0; c < S; c++) {
+          ub[2 * c] = ((const float4 *)ut.p[c])[2 * i];
+          ub[2 * c + 1] = ((const float4 *)ut.p[c])[2 * i + 1];
+        }
+      };
+      fetch(q);
+#pragma unroll
+      for (int k = 0; k < KV; k++) m[k] = *(const float4 *)(vn.n[k0 + k < nv ? k0 + k : nv - 1] + 4 * q);
+      for (int r = 0; r < 12; r++) {
+        float2 b[S][4];
+        h8v vc[KV];
+#pragma unroll
+        for (int c = 0; c < S; c++) {
+          b[c][0] = make_float2(ub[2 * c].x, ub[2 * c].y);
+          b[c][1] = make_float2(ub[2 * c].z, ub[2 * c].w);
+          b[c][2] = make_float2(ub[2 * c + 1].x, ub[2 * c + 1].y);
+          b[c][3] = make_float2(ub[2 * c + 1].z, ub[2 * c + 1].w);
+        }
+#pragma unroll
+        for (int k = 0; k < KV; k++) vc[k] = vb[k];
+        if (r < 11) fetch((r + 1) * nq + q);  // ahead of this run's arithmetic
+#pragma unroll
+        for (int k = 0; k < KV; k++) {
+          float2 e[4];
+          e[0] = make_float2(m[k].x * (float)vc[k][0], m[k].x * (float)vc[k][1]);
+          e[1] = make_float2(m[k].y * (float)vc[k][2], m[k].y * (float)vc[k][3]);
+          e[2] = make_float2(m[k].z * (float)vc[k][4], m[k].z * (float)vc[k][5]);
+          e[3] = make_float2(m[k].w * (float)vc[k][6], m[k].w * (float)vc[k][7]);
+          add(e, b, k);
+        }
+      }
+    }
+  } else {
+    for (long q = blockIdx.x * 64L + lane; q < nq; q += gridDim.x * 64L)
+      for (int r = 0; r < 12; r++) {
+        float2 b[S][4];
+#pragma unroll
+        for (int c = 0; c < S; c++) ld4(ut.p[c], r * nq + q, b[c]);
+#pragma unroll
+        for (int k = 0; k < S; k++) add(b[k], b, k);
+      }
+  }
+  double mine = 0;
+#pragma unroll
+  for (int k = 0; k < 2 * KV * S; k++) {
+    double s = (double)af[k];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (lane == k) mine = s;
+  }
+  if (lane < 2 * KV * S) part[((long)chunk * gridDim.x + blockIdx.x) * (2 * KV * S) + lane] = mine;
+}
+
+// k_bupdate for an FP16 basis, one lane per site: the S new vectors of a site
+// in registers (24 S floats), rounded to the basis's format at the end (the
+// site's 24 reals over their largest magnitude, that magnitude as its norm).
+// Reads the basis and the u_c once, writes the new vectors once: 244 us at
+// 32^3x64 and 14.5 vectors, 5.7 TB/s.
+template <int S>
+__global__ void __launch_bounds__(UB) k_bupdate_h(long stride, VTab v, NTab vn, UTab ut, int nv,
+                                                  const float *__restrict__ coef) {
+  const float *D = coef + 2 * BlockArnoldi::NMAX * BlockArnoldi::SMAX;
+  const long i = blockIdx.x * (long)UB + threadIdx.x;
+  if (i >= stride) return;
+  float2 s[S][12];
+#pragma unroll
+  for (int r = 0; r < 12; r++) {
+    float2 u[S];
+#pragma unroll
+    for (int c = 0; c < S; c++) u[c] = ((const float2 *)ut.p[c])[r * stride + i];
+#pragma unroll
+    for (int c = 0; c < S; c++) {
+      s[c][r] = make_float2(0, 0);
+#pragma unroll
+      for (int l = 0; l <= c; l++) {
+        const float dr = D[2 * (l * S + c)], di = D[2 * (l * S + c) + 1];
+        s[c][r].x += dr * u[l].x - di * u[l].y;
+        s[c][r].y += dr * u[l].y + di * u[l].x;
+      }
+    }
+  }
+  for (int k = 0; k < nv; k++) {
+    const float m = vn.n[k][i];
+    const h2v *p = (const h2v *)v.p[k] + i;
+    h2v h[12];
+#pragma unroll
+    for (int r = 0; r < 12; r++) h[r] = p[r * stride];
+    float cr[S], ci[S];
+#pragma unroll
+    for (int c = 0; c < S; c++) {
+      cr[c] = m * coef[2 * (k * S + c)];
+      ci[c] = m * coef[2 * (k * S + c) + 1];
+    }
+#pragma unroll
+    for (int r = 0; r < 12; r++) {
+      const float x = (float)h[r].x, y = (float)h[r].y;
+#pragma unroll
+      for (int c = 0; c < S; c++) {
+        s[c][r].x += cr[c] * x - ci[c] * y;
+        s[c][r].y += cr[c] * y + ci[c] * x;
+      }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < S; c++) {
+    float m = 0.f;
+#pragma unroll
+    for (int r = 0; r < 12; r++) m = fmaxf(m, fmaxf(fabsf(s[c][r].x), fabsf(s[c][r].y)));
+    const float f = m > 0.f ? 1.f / m : 0.f;
+    h2v *o = (h2v *)v.p[nv + c] + i;
+#pragma unroll
+    for (int r = 0; r < 12; r++) {
+      h2v h;
+      h.x = (f16)(s[c][r].x * f);
+      h.y = (f16)(s[c][r].y * f);
+      o[r * stride] = h;
+    }
+    vn.n[nv + c][i] = m;
+  }
+}
+
 // ===================================================================== //
 
-static constexpr int CHUNKS = BlockArnoldi::NMAX / KV;
+static constexpr int CHUNKS = BlockArnoldi::NMAX / KV + 1;
 
 BlockArnoldi::BlockArnoldi(hipStream_t s, int m_) : stream(s), m(m_), ld(m_ + 1) {
   if (m < 1 || m + 1 > NMAX) throw std::runtime_error("BlockArnoldi: at most 127 steps");
@@ -380,6 +563,7 @@ BlockArnoldi::BlockArnoldi(hipStream_t s, int m_) : stream(s), m(m_), ld(m_ + 1)
   pool_get(&sums, sizeof(double) * 2 * KV * SMAX * CHUNKS);
   pool_get(&pr, sizeof(double) * 2 * SMAX * (NMAX + SMAX));
   pool_get(&coef, sizeof(double) * 2 * SMAX * (NMAX + SMAX));
+  pool_get(&coef32, sizeof(float) * 2 * SMAX * (NMAX + SMAX));
   hh = static_cast<double *>(pool_alloc_host(sizeof(double) * slot_len() * slots));
 }
 
@@ -390,6 +574,7 @@ BlockArnoldi::~BlockArnoldi() {
   pool_free(sums);
   pool_free(pr);
   pool_free(coef);
+  pool_free(coef32);
   pool_free_host(hh);
 }
 
@@ -446,9 +631,9 @@ void BlockArnoldi::run(const Vec *V, int j, int s, int slot, bool again) {
       hipLaunchKernelGGL(k_bsum, dim3(chunks), dim3(1024), 0, stream, gx, 2 * KV * S, part, sums);
       // a vector is taken while at least 1e-9 (FP64; FP32: 1e-10, its rounding squared being 4e-15) of its
       // squared norm is left
-      hipLaunchKernelGGL((k_bcols<S>), dim3(1), dim3(256), 0, stream, j, ld, again ? 1 : 0,
+      hipLaunchKernelGGL((k_bcols<S>), dim3(1), dim3(256), 0, stream, j, ld, again ? 1 : 0, j + 1,
                          sizeof(T) == 8 ? 1e-9 : 1e-10, (const double2 *)sums, (double2 *)hd, (double2 *)pr,
-                         (double2 *)coef, (double2 *)slot_h, slot_h + 2L * SMAX * ld);
+                         (double2 *)coef, (float2 *)coef32, (double2 *)slot_h, slot_h + 2L * SMAX * ld);
       hipLaunchKernelGGL((k_bupdate<T, S>), dim3(gu), dim3(UB), 0, stream, nu, tab, j + 1, coef);
     });
     QQCD_HIP(hipGetLastError());
@@ -456,6 +641,39 @@ void BlockArnoldi::run(const Vec *V, int j, int s, int slot, bool again) {
   if (V[0].prec == PREC_DOUBLE) go(double());
   else if (V[0].prec == PREC_SINGLE) go(float());
   else throw std::runtime_error("BlockArnoldi: FP64 or FP32 vectors");
+}
+
+void BlockArnoldi::queue_half(const Vec *V, const Vec *U, int j, int s, int slot) {
+  if (j < 0 || s < 1 || s > SMAX || j + s > m || slot < 0 || slot >= m) throw std::runtime_error("BlockArnoldi: bad block");
+  VTab tab{};
+  NTab nt{};
+  UTab ut{};
+  for (int q = 0; q <= j + s; q++) {
+    if (V[q].prec != PREC_HALF || !V[q].norm || V[q].n != V[0].n) throw std::runtime_error("BlockArnoldi: FP16 basis");
+    tab.p[q] = V[q].data;
+    nt.n[q] = const_cast<float *>(V[q].norm);
+  }
+  for (int c = 0; c < s; c++) {
+    if (U[c].prec != PREC_SINGLE || U[c].n != V[0].n) throw std::runtime_error("BlockArnoldi: FP32 work vectors");
+    ut.p[c] = U[c].data;
+  }
+  const long stride = V[0].n / 12, nq = stride / 4;
+  if (V[0].n % 48) throw std::runtime_error("BlockArnoldi: not a checkerboard field");
+  const int nv = j + 1, cv = (nv + KV - 1) / KV, chunks = cv + 1, ny = (chunks + DW - 1) / DW, w = (chunks + ny - 1) / ny;
+  const int gx = (int)std::max(1L, std::min({(nq + 63) / 64, (long)DGRID, 3072L / (long)(w * ny) + 1}));
+  double *slot_h = hh + slot_len() * slot;
+  with_s(s, [&](auto SS) {
+    constexpr int S = decltype(SS)::value;
+    hipLaunchKernelGGL((k_bdot_h<S>), dim3(gx, ny), dim3(64 * w), 0, stream, nq, tab, nt, ut, nv, part);
+    hipLaunchKernelGGL(k_bsum, dim3(chunks), dim3(1024), 0, stream, gx, 2 * KV * S, part, sums);
+    // FP32 sums over vectors of an FP16 operator: below 1e-6 of its squared norm a vector is their rounding
+    hipLaunchKernelGGL((k_bcols<S>), dim3(1), dim3(256), 0, stream, j, ld, 0, cv * KV, 1e-6, (const double2 *)sums,
+                       (double2 *)hd, (double2 *)pr, (double2 *)coef, (float2 *)coef32, (double2 *)slot_h,
+                       slot_h + 2L * SMAX * ld);
+    hipLaunchKernelGGL((k_bupdate_h<S>), dim3((unsigned)((stride + UB - 1) / UB)), dim3(UB), 0, stream, stride, tab, nt,
+                       ut, nv, coef32);
+  });
+  QQCD_HIP(hipGetLastError());
 }
 
 void BlockArnoldi::queue(const Vec *V, int j, int s, int slot) { run(V, j, s, slot, false); }

@@ -115,21 +115,15 @@ struct DevHess {
   int m, ld;              // ld = 2 (m + 1) doubles per column
   double *d = nullptr;    // m columns of complex <V_i, w>, then m squared norms
   double *h = nullptr;    // pinned host copy
-  double *x = nullptr;    // paired steps: g2 (ld), the four scalars, the three coefficients
   explicit DevHess(int m_) : m(m_), ld(2 * (m_ + 1)) {
     const size_t n = (size_t)(ld + 1) * m;
     pool_get(&d, sizeof(double) * n);
-    pool_get(&x, sizeof(double) * (ld + 8));
     h = static_cast<double *>(pool_alloc_host(sizeof(double) * n));
   }
   ~DevHess() {
     pool_free(d);
-    pool_free(x);
     pool_free_host(h);
   }
-  double *g2() { return x; }
-  double *sc() { return x + ld; }
-  double *cb() { return x + ld + 4; }
   DevHess(const DevHess &) = delete;
   DevHess &operator=(const DevHess &) = delete;
   double *col(int j) { return d + (size_t)ld * j; }
@@ -168,43 +162,12 @@ static void arnoldi_step_dev(Context &c, LinOp &A, std::vector<Spinor> &V, int j
   else c.blas->rscale_dev(w, dh.n2(j));
 }
 
-// Arnoldi steps j and j + 1 in one pair (FP16 basis with per-site norms, FP32
-// work vectors w1, w2): u1 = A v_j, u2 = A u1, the dots of both against
-// V_0..V_j in one pass over the basis, both updates in another, column j + 1
-// of H from the Arnoldi relation (pair_columns); then v_{j+1} = u1' / ||u1'||
-// and v_{j+2} from the part of A v_{j+1} orthogonal to v_0..v_{j+1}.  Half
-// the passes over the basis of two single steps.  The derivation of column
-// j + 1 uses the orthonormality of V_j, which the FP16 basis holds to its
-// rounding, as the single-step passes do.
 static int g_arnoldi_steps = 2;
 void set_arnoldi_steps(int steps) {
   if (steps != 1 && steps != 2) throw std::runtime_error("Arnoldi steps per Gram-Schmidt pass: 1 or 2");
   g_arnoldi_steps = steps;
 }
 int arnoldi_steps() { return g_arnoldi_steps; }
-
-static void arnoldi_pair_dev(Context &c, LinOp &A, std::vector<Spinor> &V, int j, DevHess &dh, Spinor &w1,
-                             Spinor &w2) {
-  if (A.apply_sq) {
-    A.apply_sq(V[j], w1, w2);
-  } else {
-    A.apply(V[j], w1);
-    A.apply(w1, w2);
-  }
-  Vec a1 = vv(w1), a2 = vv(w2);
-  std::vector<Vec> Vb = vecs(V, j + 1);
-  c.blas->pair_dot_dev(j + 1, Vb.data(), a1, a2, dh.col(j), dh.g2());
-  c.blas->pair_axpy_dev(j + 1, dh.col(j), dh.g2(), Vb.data(), a1, a2, dh.sc());
-  pair_columns(dh.d, dh.ld, dh.m, j, dh.g2(), dh.sc(), dh.cb(), c.stream);
-  if (V[j + 1].prec == PREC_HALF && V[j + 1].norm && V[j + 2].prec == PREC_HALF && V[j + 2].norm &&
-      w1.prec == PREC_SINGLE && w2.prec == PREC_SINGLE) {
-    c.blas->pair_comb_basis(c.g.Vh, dh.cb(), w1, w2, dh.n2(j), V[j + 1], V[j + 2], dh.n2(j + 1));
-    return;
-  }
-  c.blas->pair_comb_dev(dh.cb(), a1, a2, dh.n2(j + 1));
-  spinor_convert_rnorm(c.g, w1, V[j + 1], dh.n2(j), c.stream);
-  spinor_convert_rnorm(c.g, w2, V[j + 2], dh.n2(j + 1), c.stream);
-}
 
 // Groups of synchronisation-free steps replayed from HIP graphs: a group
 // [j0, j0 + n) that already ran on the same vectors is launched as one
@@ -242,20 +205,16 @@ struct StepGraphs {
 };
 
 static void arnoldi_steps_dev(Context &c, LinOp &A, std::vector<Spinor> &V, int j0, int n, DevHess &dh,
-                              Spinor *work, StepGraphs *sg, Spinor *work2 = nullptr) {
-  // in pairs when a second work vector is given and the group is whole pairs
+                              Spinor *work, StepGraphs *sg) {
   auto run = [&]() {
-    if (work && work2 && j0 % 2 == 0 && n % 2 == 0)
-      for (int j = j0; j < j0 + n; j += 2) arnoldi_pair_dev(c, A, V, j, dh, *work, *work2);
-    else
-      for (int j = j0; j < j0 + n; j++) arnoldi_step_dev(c, A, V, j, dh, nullptr, nullptr, work);
+    for (int j = j0; j < j0 + n; j++) arnoldi_step_dev(c, A, V, j, dh, nullptr, nullptr, work);
   };
   if (!sg) {
     run();
     return;
   }
   std::vector<const void *> key{(const void *)(intptr_t)j0, (const void *)(intptr_t)n, work ? work->data : nullptr,
-                                work2 ? work2->data : nullptr, dh.d};
+                                dh.d};
   for (int q = 0; q <= j0 + n; q++) {
     key.push_back(V[q].data);
     key.push_back(V[q].norm);
@@ -287,8 +246,9 @@ static void arnoldi_steps_dev(Context &c, LinOp &A, std::vector<Spinor> &V, int 
   e.e = nullptr;
 }
 
-// Arnoldi steps j .. j + want - 1 in blocks over an FP64 or FP32 basis
-// (qqcd_arnoldi.h), the columns into H; returns how many were made.  A block
+// Arnoldi steps j .. j + want - 1 in blocks (qqcd_arnoldi.h), the columns into
+// H; returns how many were made.  work: over an FP16 basis, the FP32 vectors of
+// a block.  A block
 // reads the basis twice whatever its length, where a step of its own with the
 // DGKS test read it four times.
 //
@@ -307,14 +267,22 @@ static void arnoldi_steps_dev(Context &c, LinOp &A, std::vector<Spinor> &V, int 
 // restart past 1e-10 takes the true value instead, which is near rounding.
 // A block whose first vector cancels to below 9 digits is done step by step.
 static int arnoldi_blocks(Context &c, LinOp &A, std::vector<Spinor> &V, int j, int want, BlockArnoldi &ba, bool keep,
-                          double &loss, std::vector<zd> &H, int ldh, bool &ended) {
+                          double &loss, std::vector<zd> &H, int ldh, bool &ended,
+                          const std::vector<std::unique_ptr<SpinorBuf>> &work) {
   const int S = BlockArnoldi::SMAX;
   std::vector<Vec> Vb = vecs(V, j + want + 1);
   int n = 0;
   for (int q = j; q < j + want; n++) {
     const int s = std::min(S, j + want - q);
-    for (int i = 0; i < s; i++) A.apply_less(V[q + i], V[q + i + 1]);
-    ba.queue(Vb.data(), q, s, n);
+    Spinor *u[BlockArnoldi::SMAX];
+    Vec uv[BlockArnoldi::SMAX];
+    for (int i = 0; i < s; i++) {
+      u[i] = work.empty() ? &V[q + i + 1] : &work[i]->s;
+      uv[i] = vv(*u[i]);
+    }
+    A.apply_less(V[q], u, s);
+    if (work.empty()) ba.queue(Vb.data(), q, s, n);
+    else ba.queue_half(Vb.data(), uv, q, s, n);
     q += s;
   }
   QQCD_HIP(hipStreamSynchronize(c.stream));
@@ -335,7 +303,7 @@ static int arnoldi_blocks(Context &c, LinOp &A, std::vector<Spinor> &V, int j, i
     if (good == s) continue;
     if (q == j) {
       std::vector<zd> col(j + 2);
-      ended = arnoldi_step(c, A, V, j, col.data(), 1) == 0.0;
+      ended = arnoldi_step(c, A, V, j, col.data(), keep, nullptr, nullptr, work.empty() ? nullptr : &work[0]->s) == 0.0;
       for (int i = 0; i <= j + 1; i++) H[i + (size_t)ldh * j] = col[i];
       ba.put(col.data(), j, A.sigma);
       q++;
@@ -373,8 +341,7 @@ ProjWork::~ProjWork() { reset(); }
 void ProjWork::reset() {
   sg.reset();  // the graphs name the buffers: they go first
   dh.reset();
-  work.reset();
-  work2.reset();
+  work.clear();
   free_basis(V);
   m = 0;
 }
@@ -469,12 +436,20 @@ static void store_deflation(Context &c, Deflation *defl, const std::vector<Spino
 }
 
 // whether a solve runs its Arnoldi steps in blocks: the basis in the work
-// precision, FP64 or FP32, an operator without its diagonal, no
-// preconditioner and no hook that wants every step
-static bool block_steps(const LinOp &A, int m, const LinOp *M, const StepHook *step_hook) {
-  return g_arnoldi_steps == 2 && g_step_graphs != 1 && A.apply_less && A.basis() == A.prec &&
-         (A.prec == PREC_DOUBLE || A.prec == PREC_SINGLE) && !M && !(step_hook && *step_hook) &&
+// precision (FP64, FP32), or in FP16 under FP32 with one Gram-Schmidt pass, an
+// operator without its diagonal, no preconditioner and no hook that wants
+// every step
+static bool block_steps(const LinOp &A, int m, int reorth, const LinOp *M, const StepHook *step_hook) {
+  const bool own = A.basis() == A.prec && (A.prec == PREC_DOUBLE || A.prec == PREC_SINGLE);
+  const bool half = A.basis() == PREC_HALF && A.prec == PREC_SINGLE && !reorth;
+  return g_arnoldi_steps == 2 && A.apply_less && (own || half) && !M && !(step_hook && *step_hook) &&
          m + 1 <= BlockArnoldi::NMAX;
+}
+
+// the work-precision vectors of a solve whose basis is stored lower: one, or a block's
+static void alloc_work(Context &c, std::vector<std::unique_ptr<SpinorBuf>> &work, bool lower, bool blocks, Prec p) {
+  work.clear();
+  for (int i = 0; lower && i < (blocks ? BlockArnoldi::SMAX : 1); i++) work.emplace_back(new SpinorBuf(c.g, p));
 }
 
 // The least-squares residual after columns j + 1 .. j + got: true once it is
@@ -516,11 +491,9 @@ SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int 
     alloc_basis(c, Z, m, p);
     alloc_basis(c, ZW, k, p);
   }
-  std::unique_ptr<SpinorBuf> work, work2;
-  if (vp != p) work.reset(new SpinorBuf(c.g, p));
-  // paired Arnoldi steps: one Gram-Schmidt pass, FP32 work over an FP16 basis
-  if (g_arnoldi_steps == 2 && !reorth && !M && p == PREC_SINGLE && vp == PREC_HALF) work2.reset(new SpinorBuf(c.g, p));
-  const bool blocks = block_steps(A, m, M, step_hook);
+  const bool blocks = block_steps(A, m, reorth, M, step_hook);
+  std::vector<std::unique_ptr<SpinorBuf>> work;
+  alloc_work(c, work, vp != p, blocks, p);
   std::unique_ptr<DevHess> dh;
   if (!reorth && !blocks) dh.reset(new DevHess(m));
   std::unique_ptr<BlockArnoldi> ba;
@@ -552,7 +525,7 @@ SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int 
       if (ba) {
         bool ended = false;
         const int want = std::min(std::min(kCheck, m - j), std::max(1, maxiter - st.iters));
-        int got = arnoldi_blocks(c, A, V, j, want, *ba, reorth != 0, loss, H, ldh, ended);
+        int got = arnoldi_blocks(c, A, V, j, want, *ba, reorth != 0, loss, H, ldh, ended, work);
         const bool done = first_enough(H, ldh, cv, y, j, got, tol * r0, itermin - st.iters);
         st.matvecs += got;
         st.iters += got;
@@ -561,14 +534,14 @@ SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int 
         continue;
       }
       if (dh) {
-        if (sg || work2) {
+        if (sg) {
           const int n = std::min(std::min(kCheck, m - j), std::max(1, maxiter - st.iters));
-          arnoldi_steps_dev(c, A, V, j, n, *dh, work ? &work->s : nullptr, sg.get(), work2 ? &work2->s : nullptr);
+          arnoldi_steps_dev(c, A, V, j, n, *dh, work.empty() ? nullptr : &work[0]->s, sg.get());
           st.matvecs += n;
           st.iters += n;
           j += n;
         } else {
-          arnoldi_step_dev(c, A, V, j, *dh, M, M ? &Z : nullptr, work ? &work->s : nullptr);
+          arnoldi_step_dev(c, A, V, j, *dh, M, M ? &Z : nullptr, work.empty() ? nullptr : &work[0]->s);
           st.matvecs++;
           st.iters++;
           j++;
@@ -584,7 +557,8 @@ SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int 
         if ((est < tol * r0 && st.iters >= itermin) || st.iters >= maxiter) break;
         continue;
       }
-      const double hn = arnoldi_step(c, A, V, j, col.data(), reorth, M, M ? &Z : nullptr, work ? &work->s : nullptr);
+      const double hn = arnoldi_step(c, A, V, j, col.data(), reorth, M, M ? &Z : nullptr,
+                                     work.empty() ? nullptr : &work[0]->s);
       st.matvecs++;
       st.iters++;
       for (int i = 0; i <= j + 1; i++) H[i + (size_t)ldh * j] = col[i];
@@ -668,23 +642,20 @@ SolveStats gmresproj(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, co
   // or the precisions change)
   std::vector<Spinor> Vown;
   BasisGuard g1{Vown};
-  std::unique_ptr<SpinorBuf> work_own, work2_own;
+  std::vector<std::unique_ptr<SpinorBuf>> work_own;
   std::unique_ptr<DevHess> dh_own;
   std::unique_ptr<StepGraphs> sg_own;
   std::vector<Spinor> *Vp = &Vown;
-  SpinorBuf *work = nullptr, *work2 = nullptr;
+  std::vector<std::unique_ptr<SpinorBuf>> *wp = &work_own;
   DevHess *dh = nullptr;
   StepGraphs *sg = nullptr;
-  // paired Arnoldi steps: one Gram-Schmidt pass, FP32 work over an FP16 basis
-  const bool pairs = g_arnoldi_steps == 2 && !reorth && p == PREC_SINGLE && vp == PREC_HALF;
-  const bool blocks = block_steps(A, m, nullptr, nullptr);
+  const bool blocks = block_steps(A, m, reorth, nullptr, nullptr);
   const bool dev = !reorth && !blocks;
   if (ws) {
-    if (ws->m != m || ws->p != p || ws->vp != vp || dev != (ws->dh != nullptr) || pairs != (ws->work2 != nullptr)) {
+    if (ws->m != m || ws->p != p || ws->vp != vp || dev != (ws->dh != nullptr)) {
       ws->reset();
       alloc_basis(c, ws->V, m + 1, vp);
-      if (vp != p) ws->work.reset(new SpinorBuf(c.g, p));
-      if (pairs) ws->work2.reset(new SpinorBuf(c.g, p));
+      alloc_work(c, ws->work, vp != p, blocks, p);
       if (dev) ws->dh.reset(new DevHess(m));
       ws->m = m;
       ws->p = p;
@@ -693,21 +664,19 @@ SolveStats gmresproj(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, co
     if (ws->dh && g_step_graphs && !ws->sg) ws->sg.reset(new StepGraphs);
     if (!g_step_graphs) ws->sg.reset();
     Vp = &ws->V;
-    work = ws->work.get();
-    work2 = ws->work2.get();
+    wp = &ws->work;
     dh = ws->dh.get();
     sg = ws->sg.get();
   } else {
     alloc_basis(c, Vown, m + 1, vp);
-    if (vp != p) work_own.reset(new SpinorBuf(c.g, p));
-    if (pairs) work2_own.reset(new SpinorBuf(c.g, p));
+    alloc_work(c, work_own, vp != p, blocks, p);
     if (dev) dh_own.reset(new DevHess(m));
     if (dh_own && g_step_graphs == 1) sg_own.reset(new StepGraphs);
-    work = work_own.get();
-    work2 = work2_own.get();
     dh = dh_own.get();
     sg = sg_own.get();
   }
+  const std::vector<std::unique_ptr<SpinorBuf>> &work = *wp;
+  Spinor *const w0 = work.empty() ? nullptr : &work[0]->s;
   std::vector<Spinor> &V = *Vp;
   std::unique_ptr<BlockArnoldi> ba;
   if (blocks) ba.reset(new BlockArnoldi(c.stream, m));
@@ -748,7 +717,7 @@ SolveStats gmresproj(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, co
       if (ba) {
         bool ended = false;
         const int want = std::min(std::min(kCheck, m - j), std::max(1, maxiter - st.iters));
-        int got = arnoldi_blocks(c, A, V, j, want, *ba, reorth != 0, loss, H, ldh, ended);
+        int got = arnoldi_blocks(c, A, V, j, want, *ba, reorth != 0, loss, H, ldh, ended, work);
         std::vector<double> res;
         const bool done = first_enough(H, ldh, cv, y, j, got, tol * r0, itermin - st.iters, hist ? &res : nullptr);
         for (size_t q = 0; q < res.size(); q++) hist->emplace_back(st.matvecs + 1 + (int)q, res[q]);
@@ -759,14 +728,14 @@ SolveStats gmresproj(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, co
         continue;
       }
       if (dh) {
-        if (sg || work2) {
+        if (sg) {
           const int n = std::min(std::min(kCheck, m - j), std::max(1, maxiter - st.iters));
-          arnoldi_steps_dev(c, A, V, j, n, *dh, work ? &work->s : nullptr, sg, work2 ? &work2->s : nullptr);
+          arnoldi_steps_dev(c, A, V, j, n, *dh, w0, sg);
           st.matvecs += n;
           st.iters += n;
           j += n;
         } else {
-          arnoldi_step_dev(c, A, V, j, *dh, nullptr, nullptr, work ? &work->s : nullptr);
+          arnoldi_step_dev(c, A, V, j, *dh, nullptr, nullptr, w0);
           st.matvecs++;
           st.iters++;
           j++;
@@ -786,7 +755,7 @@ SolveStats gmresproj(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, co
         if ((est < tol * r0 && st.iters >= itermin) || st.iters >= maxiter) break;
         continue;
       }
-      const double hn = arnoldi_step(c, A, V, j, col.data(), reorth, nullptr, nullptr, work ? &work->s : nullptr);
+      const double hn = arnoldi_step(c, A, V, j, col.data(), reorth, nullptr, nullptr, w0);
       st.matvecs++;
       st.iters++;
       for (int i = 0; i <= j + 1; i++) H[i + (size_t)ldh * j] = col[i];
@@ -934,29 +903,25 @@ MixedStats solve_mixed(Context &c, const double kappa[2], const Spinor &b, Spino
     };
     if (work == PREC_SINGLE && (op_prec == PREC_SINGLE || direct32)) {
       o.sigma = Alo->diag();
-      o.apply_less = [&, direct32](const Spinor &a, Spinor &r) {
+      o.apply_less = [&, direct32](const Spinor &a, Spinor *const *r, int n) {
         const Spinor *in = &a;
         if (a.prec != op_prec) {
           spinor_copy_convert(c.g, a, in_lo->s, c.stream);
           in = &in_lo->s;
         }
-        if (direct32) (*Alo)(*in, out_lo->s, &r, true, true);
-        else (*Alo)(*in, r, nullptr, false, true);
-      };
-    }
-    if (direct32) {
-      // r1 = A a in FP32 and, rounded to FP16 by the same launch, the input
-      // of r2 = A r1: the operator reads its input in FP16, so r2 is A
-      // applied to r1 as the operator sees it
-      o.apply_sq = [&](const Spinor &a, Spinor &r1, Spinor &r2) {
-        if (r1.prec != PREC_SINGLE || r2.prec != PREC_SINGLE) throw std::runtime_error("apply_sq: FP32 results");
-        const Spinor *in = &a;
-        if (a.prec != op_prec) {
-          spinor_copy_convert(c.g, a, in_lo->s, c.stream);
-          in = &in_lo->s;
+        for (int i = 0; i < n; i++) {
+          if (r[i]->prec != PREC_SINGLE) throw std::runtime_error("apply_less: FP32 results");
+          if (direct32) {
+            // in FP32 and, rounded to FP16 by the same launch, the input of
+            // the next: the operator reads its input in FP16 in any case
+            Spinor &lo = in == &out_lo->s ? in_lo->s : out_lo->s;
+            (*Alo)(*in, lo, r[i], i + 1 == n, true);
+            in = &lo;
+          } else {
+            (*Alo)(*in, *r[i], nullptr, false, true);
+            in = r[i];
+          }
         }
-        (*Alo)(*in, out_lo->s, &r1, false);
-        (*Alo)(out_lo->s, in_lo->s, &r2, true);
       };
     }
     return o;

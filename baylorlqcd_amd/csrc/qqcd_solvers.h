@@ -20,13 +20,11 @@ struct LinOp {
   Prec prec = PREC_DOUBLE;
   int store = -1;
   std::function<void(const Spinor &, Spinor &)> apply;
-  // optional: r1 = A a, r2 = A r1 in one call (an operator that rounds its
-  // input to a lower storage precision can then pass its own rounded r1 on)
-  std::function<void(const Spinor &, Spinor &, Spinor &)> apply_sq;
-  // optional: r = (A - sigma) a, the operator without its multiple of the
-  // identity: the same Krylov space, without the cancellation of that part
-  // in every orthogonalisation
-  std::function<void(const Spinor &, Spinor &)> apply_less;
+  // optional: r[i] = (A - sigma)^(i+1) a, i < n: the operator without its
+  // multiple of the identity, which gives the same Krylov space without the
+  // cancellation of that part in every orthogonalisation.  (An operator that
+  // rounds its input to a lower storage precision passes its own rounded r[i] on.)
+  std::function<void(const Spinor &a, Spinor *const *r, int n)> apply_less;
   double sigma = 0;
   Prec basis() const { return store < 0 ? prec : (Prec)store; }
 };
@@ -52,7 +50,9 @@ struct SchurOp {
     LinOp o;
     o.prec = tmp.s.prec;
     o.apply = [this](const Spinor &a, Spinor &b) { (*this)(a, b); };
-    o.apply_less = [this](const Spinor &a, Spinor &b) { (*this)(a, b, nullptr, false, true); };
+    o.apply_less = [this](const Spinor &a, Spinor *const *r, int n) {
+      for (int i = 0; i < n; i++) (*this)(i ? *r[i - 1] : a, *r[i], nullptr, false, true);
+    };
     o.sigma = diag();
     return o;
   }
@@ -113,7 +113,7 @@ struct StepGraphs;
 // same operator; reset() whenever that operator is replaced.
 struct ProjWork {
   std::vector<Spinor> V;
-  std::unique_ptr<SpinorBuf> work, work2;
+  std::vector<std::unique_ptr<SpinorBuf>> work;
   std::unique_ptr<DevHess> dh;
   std::unique_ptr<StepGraphs> sg;
   int m = 0;
@@ -161,8 +161,8 @@ namespace qqcd {
 // graphs: 0 never, 1 in every solve, 2 (the default) only where the basis is
 // kept between calls (ProjWork), so that a capture serves many solves
 void set_step_graphs(int mode);
-// Arnoldi steps per Gram-Schmidt pass over an FP16 basis (single-RHS
-// solvers): 2 (the default) in pairs, 1 one at a time
+// Arnoldi steps per Gram-Schmidt pass: 2 (the default) in blocks of four (the
+// batched solver: in pairs), 1 one at a time
 void set_arnoldi_steps(int steps);
 int arnoldi_steps();
 

@@ -129,12 +129,13 @@ def test_invariant_start(prec):
         lattice.finalize()
 
 
-@pytest.mark.parametrize("basis,prec,recon", [(1, 1, 18), (1, 1, 12), (1, 2, 12)])
-@pytest.mark.parametrize("gm", [(40, 16), (21, 6)])
-def test_mixed_fp32_basis(basis, prec, recon, gm):
-    """Blocks over an FP32 basis, operator in FP32 or FP16: the FP64 residual is met, in about the steps of
-    one at a time (an inner solve may end a check later)."""
-    n, kap = (8, 8, 8, 16), (0.125, 0.01)
+@pytest.mark.parametrize("basis,prec,recon", [(1, 1, 18), (1, 1, 12), (1, 2, 12), (2, 2, 12), (2, 2, 18), (2, 1, 18)])
+@pytest.mark.parametrize("n,gm", [((8, 8, 8, 16), (40, 16)), ((8, 8, 8, 16), (21, 6)), ((4, 4, 4, 4), (10, 3)),
+                                  ((12, 4, 8, 4), (60, 20))])
+def test_mixed_low_basis(basis, prec, recon, n, gm):
+    """Blocks over an FP32 or FP16 basis, operator in FP32 or FP16: the FP64 residual is met, in about the steps
+    of one at a time (an inner solve may end a check later)."""
+    kap = (0.125, 0.01)
     U, u, co = setup(n)
     try:
         psi, phi = rhs(n, 6)
@@ -148,4 +149,8 @@ def test_mixed_fp32_basis(basis, prec, recon, gm):
         lattice.finalize()
     assert residual(n, U, kap, psi, blk[1]) < 1e-10
     assert np.linalg.norm(blk[1] - one[1]) < 1e-8 * np.linalg.norm(one[1])
-    assert abs(blk[0] - one[0]) <= 0.15 * one[0] + 8, (one[0], blk[0])
+    # not more steps, to an inner check's granularity per outer step; fewer only where the inner target (1e-6 with
+    # the FP32 operator) is below what an FP16 basis carries (11 bits), so that inner solves run to their cap
+    assert blk[0] <= 1.15 * one[0] + 8, (one[0], blk[0])
+    if (basis, prec) != (2, 1):
+        assert blk[0] >= 0.85 * one[0] - 8, (one[0], blk[0])

@@ -35,7 +35,7 @@ def calls(n, seed):
     return [x, h, g, nz["traces"], *p["xe"]]
 
 
-# 4^4: vectors with padding-free strides down to two wavefronts; 12 x 4 x 4 x 4: 384 sites, 6 wavefronts
+# checkerboards of 2, 6 and 64 wavefronts of sites
 @pytest.mark.parametrize("n", [(4, 4, 4, 4), (12, 4, 4, 4), (8, 8, 8, 16)])
 def test_reused_buffers(n):
     held = []
