@@ -23,6 +23,7 @@
 #include "qqcd_solvers.h"
 
 #include "qqcd_arnoldi.h"
+#include "qqcd_bicgstab.h"
 
 #include <cmath>
 #include <memory>
@@ -788,6 +789,7 @@ SolveStats bicgstab(Context &c, LinOp &A, const Spinor &b, Spinor &x, double tol
   SolveStats st;
   const Prec p = A.prec;
   SpinorBuf r(c.g, p), rhat(c.g, p), pp(c.g, p), v(c.g, p), t(c.g, p);
+  if (p != PREC_DOUBLE) throw std::runtime_error("bicgstab: FP64 operator expected");
   Vec R = vv(r.s), Rh = vv(rhat.s), P = vv(pp.s), Vv = vv(v.s), T = vv(t.s), X = vv(x);
   double rn = residual(c, A, b, x, r.s, st);
   const double r0 = rn;
@@ -795,33 +797,36 @@ SolveStats bicgstab(Context &c, LinOp &A, const Spinor &b, Spinor &x, double tol
     st.converged = 1;
     return st;
   }
+  BiCGStabDev bi(c.stream, R.n);
+  const double goal = tol * r0;
   for (;;) {
-    c.blas->copy(R, Rh);
-    c.blas->zero(P);
-    c.blas->zero(Vv);
-    zd rho = 1.0, alpha = 1.0, omega = 1.0;
-    double rr = rn;
-    while (!((rr < tol * r0 && st.iters >= itermin) || st.iters >= maxiter)) {
-      const zd oldrho = rho;
-      rho = c.blas->dot(Rh, R);
-      const zd beta = (rho / oldrho) * (alpha / omega);
-      // p = r + beta (p - omega v)
-      c.blas->axpby(-beta * omega, Vv, beta, P, false);
-      c.blas->axpby(1.0, R, 1.0, P, false);
-      A.apply(pp.s, v.s);
-      st.matvecs++;
-      alpha = rho / c.blas->dot(Rh, Vv);
-      c.blas->axpby(-alpha, Vv, 1.0, R, false);
-      A.apply(r.s, t.s);
-      st.matvecs++;
-      const zd top = c.blas->dot(T, R);
-      const double bot = c.blas->norm2(T);
-      omega = top / bot;
-      c.blas->axpby(omega, R, 1.0, X, false);
-      c.blas->axpby(alpha, P, 1.0, X, false);
-      rr = std::sqrt(c.blas->axpby(-omega, T, 1.0, R, true));
-      st.iters++;
-      if (hook && *hook) (*hook)(st.iters, rr, r0);
+    bi.reset(R, Rh, P, Vv, rn, goal, st.iters, itermin, maxiter);
+    const double from = rn;
+    const int first = st.iters;
+    double rr = rn, seen[BiCGStabDev::AHEAD];
+    int ahead = 4;
+    bool ended = (rn < goal && st.iters >= itermin) || st.iters >= maxiter || !std::isfinite(rn);
+    while (!ended) {
+      for (int k = 0; k < ahead; k++) {
+        bi.start(R, Vv, P);
+        A.apply(pp.s, v.s);
+        bi.middle(Rh, Vv, R);
+        A.apply(r.s, t.s);
+        bi.finish(Rh, P, T, R, X);
+      }
+      QQCD_HIP(hipStreamSynchronize(c.stream));
+      const int n = bi.fetch(st.iters, seen, &ended);
+      for (int k = 0; k < n; k++) {
+        st.iters++;
+        st.matvecs += 2;
+        rr = seen[k];
+        if (hook && *hook) (*hook)(st.iters, rr, r0);
+      }
+      // queue up to most of the iterations that are left at the rate so far:
+      // those queued past the end still apply the operator
+      const double rate = std::log(from / rr) / std::max(1, st.iters - first), left = std::log(rr / goal);
+      ahead = rate > 0 && left > 0 ? (int)std::min(0.7 * left / rate, 16.0) : 2;
+      ahead = std::max(2, ahead);
     }
     // confirm on the true residual
     rn = residual(c, A, b, x, r.s, st);
