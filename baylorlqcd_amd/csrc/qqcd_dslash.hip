@@ -797,6 +797,160 @@ __global__ void __launch_bounds__(256) k_dslash_pipe(const DslashArgs a) {
   dslash_site_pipe<S, L, RECON, SIG, NT, false, D>(a, h, a.out, a.out_norm, a.x, a.x_norm, i, 0, 0);
 }
 
+// ---- one hop per wavefront (fields that stay in the caches) ---------------
+//
+// k_dslash_pipe gives a site to one lane: at 4096 sites that is 64 wavefronts
+// on a chip of 1024 SIMDs, each making its eight hops' trips to memory two at
+// a time.  Here the eight wavefronts of a workgroup take one hop each of the
+// same 64 sites, so all trips of a site are made at once; they leave the
+// hops' half spinors U (1 +/- g) psi (scaled) in LDS, and six of them then
+// form the sum and the epilogue, two coupled spins of one colour each.  Every
+// value of a hop passes through LDS once (2.1 KB a site in FP64, 9 us of the
+// chip's LDS rate at 24^3x48).
+template <int SIG, int K, typename R>
+__device__ __forceinline__ void hop_half(const cx<R> u[9], const cx<R> p[12], cx<R> w[6]) {
+  constexpr int MU = K >> 1;
+  constexpr bool FWD = !(K & 1);
+  cx<R> hh[6];
+  if constexpr (MU == 3) {
+#pragma unroll
+    for (int c = 0; c < 6; c++) hh[c] = p[c];
+  } else {
+    project<MU>(p, R(FWD ? SIG : -SIG), hh);
+  }
+  if (FWD) {
+    mv(u, hh, w);
+    mv(u, hh + 3, w + 3);
+  } else {
+    mdv(u, hh, w);
+    mdv(u, hh + 3, w + 3);
+  }
+}
+
+template <typename S, typename L, int RECON, int SIG, int K, typename R>
+__device__ __forceinline__ void hop_to_lds(const DslashArgs &a, const HopIn &h, int i, int x, int y, int z, int t,
+                                           cx<R> (*ws)[64], int lane) {
+  constexpr int NC = RECON == 18 ? 9 : 6;
+  constexpr int NP = (K >> 1) == 3 ? 6 : 12;
+  HopRaw<S, L, RECON> r;
+  hop_fetch<S, L, RECON, SIG, false, false, K>(a, h, i, x, y, z, t, 0, 0, r);
+  cx<R> u[9], p[12], w[6];
+#pragma unroll
+  for (int k = 0; k < NC; k++) u[k] = mk<R>((R)r.u[k].x, (R)r.u[k].y);
+  if constexpr (RECON == 12) recon_row2(u);
+#pragma unroll
+  for (int k = 0; k < NP; k++) p[k] = mk<R>((R)r.p[k].x, (R)r.p[k].y);
+  hop_half<SIG, K>(u, p, w);
+  R f = (R)a.scl[K >> 1] * (R)r.edge * ((K >> 1) == 3 ? R(2) : R(1));
+  if constexpr (std::is_same<S, f16>::value) f *= (R)r.nrm;
+#pragma unroll
+  for (int k = 0; k < 6; k++) ws[k][lane] = f * w[k];
+}
+
+template <typename S, typename L, int RECON, int SIG>
+__global__ void __launch_bounds__(512) k_dslash_split(const DslashArgs a) {
+  typedef typename SIO<S>::R R;
+  typedef typename V2<S>::T SE;
+  __shared__ cx<R> ws[8][6][64];
+  __shared__ float mx[6][64];
+  int blk = blockIdx.x;
+  if (a.xcd_remap) {
+    const int nb = gridDim.x, per = (nb + 7) / 8;
+    const int xcd = blk & 7, k = blk >> 3;
+    const int full = nb - 8 * (per - 1);
+    blk = xcd < full ? xcd * per + k : full * per + (xcd - full) * (per - 1) + k;
+  }
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l = blk * 64 + lane;
+  const bool in = l < a.Vh;
+  const int i = site_of(a, in ? l : a.Vh - 1);  // lanes past the end repeat the last site and store nothing
+  const int nx = a.n[0], ny = a.n[1], nz = a.n[2];
+  const int r2 = 2 * i;
+  const int x0 = r2 % nx;
+  int q = r2 / nx;
+  const int y = q % ny;
+  q /= ny;
+  const int z = q % nz;
+  const int t = q / nz;
+  const int x = x0 + ((a.par + y + z + t) & 1);
+  const HopIn h{a.in, a.in_norm, a.links, a.sstride, a.lstride};
+  switch (wave) {
+#define HOPCASE(K) \
+  case K: hop_to_lds<S, L, RECON, SIG, K>(a, h, i, x, y, z, t, ws[K], lane); break;
+    HOPCASE(0) HOPCASE(1) HOPCASE(2) HOPCASE(3) HOPCASE(4) HOPCASE(5) HOPCASE(6) HOPCASE(7)
+#undef HOPCASE
+  }
+  __syncthreads();
+  // wavefront 3 s + c: spins s and s + 2 of colour c
+  const int s = wave / 3, c = wave - 3 * s;
+  cx<R> o0 = mk<R>(0, 0), o2 = mk<R>(0, 0);
+  const uint32_t srun = (uint32_t)h.sstride * (uint32_t)sizeof(SE);
+  if (wave < 6) {
+    SE x0r{}, x2r{};
+    float xn = 1.f;
+    if (a.has_x) {
+      const __amdgpu_buffer_rsrc_t xrs = make_rsrc(a.x, 12 * srun);
+      x0r = bld<SE, 0>(xrs, (uint32_t)i * (uint32_t)sizeof(SE), (3 * s + c) * srun);
+      x2r = bld<SE, 0>(xrs, (uint32_t)i * (uint32_t)sizeof(SE), (6 + 3 * s + c) * srun);
+      if constexpr (std::is_same<S, f16>::value) xn = a.x_norm[i];
+    }
+    // the sums of spins s (upper) and s + 2 (lower) from the half spinors:
+    // see accum() for the reconstruction
+    const int own = 3 * s + c, oth = 3 - 3 * s + c;
+    const R e = s ? R(-1) : R(1);
+    cx<R> up = mk<R>(0, 0), dn = mk<R>(0, 0);
+#pragma unroll
+    for (int K = 0; K < 6; K++) {
+      const R sg = ((K & 1) ? -SIG : SIG) > 0 ? R(1) : R(-1);
+      up = up + ws[K][own][lane];
+      if (K < 2) fma_acc(dn, sg, ws[K][oth][lane]);
+      else if (K < 4) fma_acc_i(dn, -e * sg, ws[K][oth][lane]);
+      else fma_acc(dn, e * sg, ws[K][own][lane]);
+    }
+    up = up + ws[SIG > 0 ? 6 : 7][own][lane];
+    dn = dn + ws[SIG > 0 ? 7 : 6][own][lane];
+    const R b0 = (R)a.b0, b1 = (R)a.b1;
+    o0 = b0 * up + b1 * dn;
+    o2 = b0 * dn - b1 * up;
+    if (a.has_x) {
+      const R a0 = (R)a.a0, a1 = (R)a.a1;
+      const cx<R> xa = mk<R>((R)xn * (R)x0r.x, (R)xn * (R)x0r.y), xb = mk<R>((R)xn * (R)x2r.x, (R)xn * (R)x2r.y);
+      o0 = o0 + a0 * xa + a1 * xb;
+      o2 = o2 + a0 * xb - a1 * xa;
+    }
+  }
+  auto put = [&](auto tag, void *dst, R f) {
+    typedef decltype(tag) E;
+    typedef typename V2<E>::T EE;
+    const uint32_t run = (uint32_t)h.sstride * (uint32_t)sizeof(EE);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(dst, 12 * run);
+    EE v, w;
+    v.x = (E)(f * o0.re);
+    v.y = (E)(f * o0.im);
+    w.x = (E)(f * o2.re);
+    w.y = (E)(f * o2.im);
+    bst<EE, 0>(v, rs, (uint32_t)i * (uint32_t)sizeof(EE), (3 * s + c) * run);
+    bst<EE, 0>(w, rs, (uint32_t)i * (uint32_t)sizeof(EE), (6 + 3 * s + c) * run);
+  };
+  if constexpr (std::is_same<S, f16>::value) {
+    // the site's largest magnitude is spread over six wavefronts
+    if (wave < 6) mx[wave][lane] = fmaxf(fmaxf(fabsf(o0.re), fabsf(o0.im)), fmaxf(fabsf(o2.re), fabsf(o2.im)));
+    __syncthreads();
+    if (wave < 6 && in) {
+      if (!a.skip16) {
+        float m = 0.f;
+#pragma unroll
+        for (int k = 0; k < 6; k++) m = fmaxf(m, mx[k][lane]);
+        if (wave == 0) a.out_norm[i] = m;
+        put(f16(), a.out, m > 0.f ? 1.f / m : 0.f);
+      }
+      if (a.out32) put(float(), a.out32, 1.f);
+    }
+  } else {
+    if (wave < 6 && in) put(S(), a.out, R(1));
+  }
+}
+
 // Several right-hand sides, RHS-innermost in blocks of nb = 2^lognb
 // (element (rhs r, component k, site j) of a field at
 // ((r/nb * 12 + k) * stride + j) * nb + r%nb).  A work tile is 256 lanes of
@@ -1267,8 +1421,33 @@ static bool launch_t(const DslashArgs &a0, int sig, hipStream_t s) {
       }
     a.order = ((t.order == 1 || t.order == 2) && bz > 1 && ext % bz == 0) ? t.order : 0;
     a.bz = a.order ? bz : 1;
-    if (sig > 0) launch_pipe<S, L, RECON, 1>(a, t.depth, t.nt, nb, s);
-    else launch_pipe<S, L, RECON, -1>(a, t.depth, t.nt, nb, s);
+    int nt = t.nt;
+    if (t.automatic()) {
+      // Where the links, input and output stay in the 256 MB last-level cache
+      // from one launch to the next, streaming past the caches costs 5-30%
+      // (16^3x32 FP32/18 12.1 us streamed, 10.6 not; 24^3x48 FP32/12 47.8,
+      // 37.4; but 24^3x48 FP64, 509 MB, 105.6, 124.1), and the form with one
+      // hop per wavefront is the faster one there (8^3x16 FP64 7.9 us pipelined,
+      // 4.5; 12x8x20x28 10.6, 8.3; 16^3x32 19.5, 17.6; 20^3x40 47.2, 40.6;
+      // 24^3x48 FP32/12 37.4, 33.2), in checkerboard order.  FP16 fields, half
+      // of whose time is arithmetic, gain from it up to 20^3x40 (16^3x32 7.5
+      // us, 7.1; 20^3x40 14.6, 13.3) and lose at 24^3x48 (23.5, 24.6).
+      const double bytes = 8.0 * a.lstride * (RECON == 18 ? 9 : 6) * sizeof(typename V2<L>::T) +
+                           24.0 * a.sstride * sizeof(typename V2<S>::T);
+      if (bytes <= 256e6) {
+        nt = 0;
+        if (!std::is_same<S, f16>::value || a.Vh <= 200000) {
+          a.order = 0;
+          const dim3 gs((a.Vh + 63) / 64);
+          if (sig > 0) hipLaunchKernelGGL((k_dslash_split<S, L, RECON, 1>), gs, dim3(512), 0, s, a);
+          else hipLaunchKernelGGL((k_dslash_split<S, L, RECON, -1>), gs, dim3(512), 0, s, a);
+          QQCD_HIP(hipGetLastError());
+          return true;
+        }
+      }
+    }
+    if (sig > 0) launch_pipe<S, L, RECON, 1>(a, t.depth, nt, nb, s);
+    else launch_pipe<S, L, RECON, -1>(a, t.depth, nt, nb, s);
     QQCD_HIP(hipGetLastError());
     return true;
   }

@@ -116,6 +116,9 @@ struct DslashTune {
   int bz = 0;
   int depth = 2;
   int nt = 1;
+  // left at its default, the launch also picks by size between this shape and
+  // the one-hop-per-wavefront kernel without streaming
+  bool automatic() const { return order == 1 && bz == 0 && depth == 2 && nt == 1; }
 };
 void set_dslash_tune(const DslashTune &t);
 // overrides of the multi-RHS launch shape for every call (-1: the caller's)

@@ -641,8 +641,10 @@ int qqcd_set_xcd_remap(int on);
  * hops' loads ahead; order 1 sweeps blocks of bz z-planes in t, order 2
  * blocks of bz t-slices in z (bz 0: the largest of 16, 8, 4, 2 dividing the
  * blocked extent; order 0: the checkerboard index); nt 1
- * streams links and output past the L2.  Default (1, 0, 2, 1).  Tuning aid;
- * no reference counterpart. */
+ * streams links and output past the L2.  Default (1, 0, 2, 1), with which
+ * fields that stay in the last-level cache (links, input and output below 256
+ * MB) are not streamed and take a kernel with one hop per wavefront instead.
+ * Tuning aid; no reference counterpart. */
 int qqcd_set_dslash_tune(int order, int bz, int depth, int nt);
 
 /* ---- host dense linear algebra of the solvers (verification hooks) ------
