@@ -23,11 +23,18 @@ struct VTab {
 template <typename T> struct Lane;
 template <> struct Lane<double> {
   static constexpr int E = 1;
+  typedef double2 Raw;
+  static __device__ __forceinline__ void split(Raw v, double2 (&e)[1]) { e[0] = v; }
   static __device__ __forceinline__ void ld(const void *p, long i, double2 (&e)[1]) { e[0] = ((const double2 *)p)[i]; }
   static __device__ __forceinline__ void st(void *p, long i, const double2 (&e)[1]) { ((double2 *)p)[i] = e[0]; }
 };
 template <> struct Lane<float> {
   static constexpr int E = 2;
+  typedef float4 Raw;
+  static __device__ __forceinline__ void split(Raw v, double2 (&e)[2]) {
+    e[0] = make_double2(v.x, v.y);
+    e[1] = make_double2(v.z, v.w);
+  }
   static __device__ __forceinline__ void ld(const void *p, long i, double2 (&e)[2]) {
     const float4 v = ((const float4 *)p)[i];
     e[0] = make_double2(v.x, v.y);
@@ -45,7 +52,9 @@ template <> struct Lane<float> {
 // vectors each and the same stretch of the u_c, which so come from memory once
 // per workgroup (up to 32 vectors) and from the L1 for its other wavefronts;
 // KV S = 16 complex FP64 accumulators leave three wavefronts per SIMD.
-// 24^3x48, FP64, S = 4 over 32 vectors on average: 419 us, 5.4 TB/s.
+// The next stretch is loaded ahead of a stretch's arithmetic (FP32 vectors, whose
+// products are formed in FP64, 16^3x32: 83.6 -> 44.2 us; FP64 3%).  24^3x48, FP64,
+// S = 4 over 31 vectors on average: 358 us, 5.5 TB/s.
 template <typename T, int S>
 __global__ void __launch_bounds__(64 * DW) k_bdot(long nu, VTab v, int nleft, double *part) {
   constexpr int E = Lane<T>::E;
@@ -61,12 +70,24 @@ __global__ void __launch_bounds__(64 * DW) k_bdot(long nu, VTab v, int nleft, do
   double acc[2 * KV * S];
 #pragma unroll
   for (int k = 0; k < 2 * KV * S; k++) acc[k] = 0;
-  for (long i = blockIdx.x * 64L + lane; i < nu; i += gridDim.x * 64L) {
+  typedef typename Lane<T>::Raw Raw;
+  const long step = gridDim.x * 64L;
+  Raw rb[S], re[KV];
+  auto fetch = [&](long i) {
+#pragma unroll
+    for (int c = 0; c < S; c++) rb[c] = ((const Raw *)u[c])[i];
+#pragma unroll
+    for (int q = 0; q < KV; q++) re[q] = ((const Raw *)a[q])[i];
+  };
+  long i = blockIdx.x * 64L + lane;
+  if (i < nu) fetch(i);
+  for (; i < nu; i += step) {
     double2 b[S][E], e[KV][E];
 #pragma unroll
-    for (int c = 0; c < S; c++) Lane<T>::ld(u[c], i, b[c]);
+    for (int c = 0; c < S; c++) Lane<T>::split(rb[c], b[c]);
 #pragma unroll
-    for (int q = 0; q < KV; q++) Lane<T>::ld(a[q], i, e[q]);
+    for (int q = 0; q < KV; q++) Lane<T>::split(re[q], e[q]);
+    if (i + step < nu) fetch(i + step);  // ahead of this stretch's arithmetic
 #pragma unroll
     for (int q = 0; q < KV; q++)
 #pragma unroll
