@@ -101,7 +101,7 @@ struct HbArgs {
   long stride;
   int n[4];
   int Vh;
-  int par, mu;
+  int par;
   double beta;
   uint64_t seed;
   int sweep;
@@ -111,54 +111,84 @@ __device__ __forceinline__ int nb_index(const int n[4], int x[4]) {
   return (x[0] + n[0] * (x[1] + n[1] * (x[2] + n[2] * x[3]))) >> 1;
 }
 
-__global__ void __launch_bounds__(128) k_heatbath(HbArgs a) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.Vh) return;
+// Three wavefronts share 64 sites: each forms the two staples of one other
+// direction, the first then adds the six in their order and draws the new
+// link.  Bound by reading 18 links a site (860 MB a launch on 24^3x48, half of
+// it distinct), so each XCD takes one contiguous run of sites, and by the
+// registers of the products: forward and backward staple are formed one after
+// the other, which leaves three wavefronts a SIMD.  us a launch, against one
+// lane a site with all six staples (204 registers and 296 B of scratch):
+// 8^3x16 14.8 | 23.0, 12x8x20x28 18.4 | 26.6, 16^3x32 35 | 45, 24^3x48 133 |
+// 216.  Bounds for two or four wavefronts a SIMD: 16^3x32 39 and 42.
+template <int MU> __global__ void __launch_bounds__(192, 3) k_heatbath(HbArgs a) {
+  __shared__ double sm[4][18][64];
+  const int nb = gridDim.x, per = (nb + 7) / 8;
+  const int xcd = blockIdx.x & 7, kb = blockIdx.x >> 3;
+  const int full = nb - 8 * (per - 1);  // XCDs that get `per` workgroups
+  const int blk = xcd < full ? xcd * per + kb : full * per + (xcd - full) * (per - 1) + kb;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = blk * 64 + lane, ic = i < a.Vh ? i : a.Vh - 1;
   const int *n = a.n;
+  const int mu = MU, par = a.par, opar = par ^ 1;
   int x[4];
   {
-    const int r = 2 * i;
-    const int x0 = r % n[0];
-    int q = r / n[0];
+    const unsigned r = 2u * (unsigned)ic;
+    const unsigned x0 = r % n[0];
+    unsigned q = r / n[0];
     x[1] = q % n[1];
     q /= n[1];
     x[2] = q % n[2];
     x[3] = q / n[2];
-    x[0] = x0 + ((a.par + x[1] + x[2] + x[3]) & 1);
+    x[0] = x0 + ((par + x[1] + x[2] + x[3]) & 1);
   }
-  const int mu = a.mu, par = a.par, opar = par ^ 1;
-  // staple sum A: U_mu(x) A closes the 6 plaquettes containing U_mu(x)
-  M3 A;
+  // staple sum A: U_mu(x) A closes the 6 plaquettes containing U_mu(x); this wavefront's direction nu
+  M3 A, B;
+  {
+    const int nu = wv + (wv >= MU);
+    int xpm[4] = {x[0], x[1], x[2], x[3]};
+    xpm[MU] = x[MU] + 1 == n[MU] ? 0 : x[MU] + 1;
+    int xpn[4], xmn[4], xpmmn[4];
 #pragma unroll
-  for (int k = 0; k < 9; k++) A.a[k] = z{0, 0};
-  int xpm[4] = {x[0], x[1], x[2], x[3]};
-  xpm[mu] = (xpm[mu] + 1) % n[mu];
-  const int i_pm = nb_index(n, xpm);
-  for (int nu = 0; nu < 4; nu++) {
-    if (nu == mu) continue;
-    int xpn[4] = {x[0], x[1], x[2], x[3]}, xmn[4] = {x[0], x[1], x[2], x[3]};
-    int xpmmn[4] = {xpm[0], xpm[1], xpm[2], xpm[3]};
-    xpn[nu] = (xpn[nu] + 1) % n[nu];
-    xmn[nu] = (xmn[nu] + n[nu] - 1) % n[nu];
-    xpmmn[nu] = (xpmmn[nu] + n[nu] - 1) % n[nu];
+    for (int m = 0; m < 4; m++) {
+      const int up = x[m] + 1 == n[m] ? 0 : x[m] + 1, dn = x[m] == 0 ? n[m] - 1 : x[m] - 1;
+      xpn[m] = m == nu ? up : x[m];
+      xmn[m] = m == nu ? dn : x[m];
+      xpmmn[m] = m == nu ? dn : xpm[m];
+    }
     // forward: U_nu(x+mu) U_mu(x+nu)^dag U_nu(x)^dag
-    const M3 a1 = ld(a.U, a.stride, opar, nu, i_pm);
+    const M3 a1 = ld(a.U, a.stride, opar, nu, nb_index(n, xpm));
     const M3 a2 = ld(a.U, a.stride, opar, mu, nb_index(n, xpn));
-    const M3 a3 = ld(a.U, a.stride, par, nu, i);
-    const M3 f = muld(muld(a1, a2), a3);
+    const M3 a3 = ld(a.U, a.stride, par, nu, ic);
+    A = muld(muld(a1, a2), a3);
+    __builtin_amdgcn_sched_barrier(0);
     // backward: U_nu(x+mu-nu)^dag U_mu(x-nu)^dag U_nu(x-nu)
     const M3 b1 = ld(a.U, a.stride, par, nu, nb_index(n, xpmmn));
     const M3 b2 = ld(a.U, a.stride, opar, mu, nb_index(n, xmn));
     const M3 b3 = ld(a.U, a.stride, opar, nu, nb_index(n, xmn));
-    const M3 bk = dmul(b1, dmul(b2, b3));  // b1^dag (b2^dag b3)
-#pragma unroll
-    for (int k = 0; k < 9; k++) A.a[k] = A.a[k] + f.a[k] + bk.a[k];
+    B = dmul(b1, dmul(b2, b3));  // b1^dag (b2^dag b3)
   }
+  if (wv > 0) {
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+      sm[2 * wv - 2][2 * k][lane] = A.a[k].re;
+      sm[2 * wv - 2][2 * k + 1][lane] = A.a[k].im;
+      sm[2 * wv - 1][2 * k][lane] = B.a[k].re;
+      sm[2 * wv - 1][2 * k + 1][lane] = B.a[k].im;
+    }
+  }
+  __syncthreads();
+  if (wv > 0 || i >= a.Vh) return;
+#pragma unroll
+  for (int k = 0; k < 9; k++) A.a[k] = A.a[k] + B.a[k];
+#pragma unroll
+  for (int w = 0; w < 4; w++)
+#pragma unroll
+    for (int k = 0; k < 9; k++) A.a[k] = A.a[k] + z{sm[w][2 * k][lane], sm[w][2 * k + 1][lane]};
   M3 U = ld(a.U, a.stride, par, mu, i);
   Rng rng{smix(a.seed ^ smix(((uint64_t)a.sweep * 8 + (uint64_t)(par * 4 + mu)) * 0x100000000ull + (uint64_t)i))};
-  const int sub[3][2] = {{0, 1}, {1, 2}, {0, 2}};
+#pragma unroll
   for (int s = 0; s < 3; s++) {
-    const int p = sub[s][0], q = sub[s][1];
+    const int p = s == 1 ? 1 : 0, q = s == 0 ? 1 : 2;
     const M3 W = mul(U, A);
     const z wpp = W.a[3 * p + p], wpq = W.a[3 * p + q], wqp = W.a[3 * q + p], wqq = W.a[3 * q + q];
     // SU(2) part of the 2x2 block: w = a0 + i a.sigma
@@ -201,16 +231,23 @@ __global__ void __launch_bounds__(128) k_heatbath(HbArgs a) {
   }
   // re-unitarise
   double nrm = 0;
+#pragma unroll
   for (int c = 0; c < 3; c++) nrm += U.a[c].re * U.a[c].re + U.a[c].im * U.a[c].im;
   nrm = 1.0 / sqrt(nrm);
+#pragma unroll
   for (int c = 0; c < 3; c++) U.a[c] = nrm * U.a[c];
   z d{0, 0};
+#pragma unroll
   for (int c = 0; c < 3; c++) d = d + cjmul(U.a[c], U.a[3 + c]);
+#pragma unroll
   for (int c = 0; c < 3; c++) U.a[3 + c] = U.a[3 + c] - cmul(d, U.a[c]);
   nrm = 0;
+#pragma unroll
   for (int c = 0; c < 3; c++) nrm += U.a[3 + c].re * U.a[3 + c].re + U.a[3 + c].im * U.a[3 + c].im;
   nrm = 1.0 / sqrt(nrm);
+#pragma unroll
   for (int c = 0; c < 3; c++) U.a[3 + c] = nrm * U.a[3 + c];
+#pragma unroll
   for (int c = 0; c < 3; c++) {
     const int e = (c + 1) % 3, f = (c + 2) % 3;
     const z t = cmul(U.a[e], U.a[3 + f]) - cmul(U.a[f], U.a[3 + e]);
@@ -298,19 +335,20 @@ void heatbath(Context &c, double beta, int nsweep, uint64_t seed, int hot_start)
   a.Vh = (int)g.Vh;
   a.beta = beta;
   a.seed = seed;
-  const int nb = (int)((g.Vh + 127) / 128);
+  const int nb = (int)((g.Vh + 63) / 64);
   // the sweep index keys the random stream: a hot or cold start begins a new
   // chain at sweep 0, a continuation carries on from the chain's last sweep
   if (hot_start >= 0) c.hb_sweep = 0;
   for (int sw = 0; sw < nsweep; sw++) {
     a.sweep = c.hb_sweep++;
-    for (int par = 0; par < 2; par++)
-      for (int mu = 0; mu < 4; mu++) {
-        a.par = par;
-        a.mu = mu;
-        hipLaunchKernelGGL(k_heatbath, dim3(nb), dim3(128), 0, c.stream, a);
-        QQCD_HIP(hipGetLastError());
-      }
+    for (int par = 0; par < 2; par++) {
+      a.par = par;
+      hipLaunchKernelGGL(k_heatbath<0>, dim3(nb), dim3(192), 0, c.stream, a);
+      hipLaunchKernelGGL(k_heatbath<1>, dim3(nb), dim3(192), 0, c.stream, a);
+      hipLaunchKernelGGL(k_heatbath<2>, dim3(nb), dim3(192), 0, c.stream, a);
+      hipLaunchKernelGGL(k_heatbath<3>, dim3(nb), dim3(192), 0, c.stream, a);
+      QQCD_HIP(hipGetLastError());
+    }
   }
   QQCD_HIP(hipStreamSynchronize(c.stream));
   c.u_host = nullptr;
