@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <stdexcept>
 
+#include "qqcd_blockalg.h"
 #include "qqcd_pool.h"
 
 namespace qqcd {
@@ -128,229 +129,53 @@ __global__ void __launch_bounds__(1024) k_bsum(int nb, int nq, const double *par
   if (q == 0 && g < nq) sums[(long)blockIdx.x * nq + g] = c;
 }
 
-__device__ __forceinline__ double2 zmul(double2 a, double2 b) {
-  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ __forceinline__ double2 zsub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ double2 zcmul(double2 a, double2 b) {  // conj(a) b
-  return make_double2(a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x);
-}
+// what block_columns reads and writes for one right-hand side
+template <int S> struct BlockIO {
+  const double2 *sums;
+  double2 *hd, *pr, *c;
+  float2 *c32;
+  double2 *hout;
+  double *inf;
+  int ld, g0, nv;
+  static constexpr int SM = BlockArnoldi::SMAX, NM = BlockArnoldi::NMAX;
+  __device__ double2 p(int k, int c_) const { return sums[k * S + c_]; }
+  __device__ double2 g(int r, int c_) const { return sums[(long)(g0 + r) * S + c_]; }
+  __device__ double2 p1(int k, int c_) const { return pr[k * S + c_]; }
+  __device__ double2 r1(int l, int c_) const { return pr[nv * S + l * S + c_]; }
+  __device__ void coef(int k, int c_, double2 x, double2 pt) {
+    const int i = k * S + c_;
+    c[i] = x;
+    c32[i] = make_float2((float)x.x, (float)x.y);
+    pr[i] = pt;
+    // the update walks the vectors four at a time
+    if (k == nv - 1)
+      for (int q = nv; q < (nv + 3) / 4 * 4; q++) {
+        c[q * S + c_] = make_double2(0, 0);
+        c32[q * S + c_] = make_float2(0, 0);
+      }
+  }
+  __device__ void factor(int r, int c_, double2 d, double2 rt) {
+    c[NM * SM + r * S + c_] = d;
+    c32[NM * SM + r * S + c_] = make_float2((float)d.x, (float)d.y);
+    pr[nv * S + r * S + c_] = rt;
+  }
+  __device__ double2 h(int row, int col) const { return hd[row + (long)ld * col]; }
+  __device__ void put(int row, int col, int i, double2 x) {
+    hd[row + (long)ld * col] = x;
+    hout[row + (long)ld * i] = x;
+  }
+  __device__ void info(int good, double growth, double pivot) {
+    inf[0] = good;
+    inf[1] = growth;
+    inf[2] = pivot;
+  }
+};
 
-// The small algebra of a block, one workgroup: from the sums (rows 0..j: P,
-// rows g0..g0+s-1: G) the factor R, the update coefficients and the columns
-// j..j+s-1 of H, which go to the device matrix and to the host's slot.  again:
-// the vectors are the Q of this block, with P and R of the first pass in pr;
-// the total projections are P + P2 R and the total factor R2 R.
 template <int S>
 __global__ void __launch_bounds__(256) k_bcols(int j, int ld, int again, int g0, double least, const double2 *sums,
                                                double2 *hd, double2 *pr, double2 *coef, float2 *coef32, double2 *hout,
                                                double *info) {
-  constexpr int SM = BlockArnoldi::SMAX, NM = BlockArnoldi::NMAX;
-  __shared__ double2 P[NM][S], C[NM][S], G[S][S], R[S][S], D[S][S], Pt[NM][S], Rt[S][S], col[S][NM + SM];
-  __shared__ double red[2][S];
-  __shared__ int good;
-  __shared__ double worst;
-  const int t = threadIdx.x, nv = j + 1;
-  for (int i = t; i < nv * S; i += 256) P[i / S][i % S] = sums[i];
-  for (int i = t; i < S * S; i += 256) G[i / S][i % S] = sums[(long)g0 * S + i];
-  __syncthreads();
-  // G - P^H P, one entry per 16 threads
-  for (int e0 = 0; e0 < S * S; e0 += 16) {
-    const int e = e0 + (t >> 4), r = e / S, c = e % S;
-    double2 a = make_double2(0, 0);
-    if (e < S * S)
-      for (int k = t & 15; k < nv; k += 16) {
-        const double2 p = zcmul(P[k][r], P[k][c]);
-        a.x += p.x;
-        a.y += p.y;
-      }
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) {
-      a.x += __shfl_xor(a.x, o, 64);
-      a.y += __shfl_xor(a.y, o, 64);
-    }
-    if (e < S * S && (t & 15) == 0) R[r][c] = zsub(G[r][c], a);
-  }
-  __syncthreads();
-  if (t == 0) {
-    // Cholesky R^H R of the upper triangle, in place; D = R^-1 (upper)
-    double2 r[S][S], d[S][S];
-    double least_seen = 1.0;
-    int n = 0;
-#pragma unroll
-    for (int i = 0; i < S; i++)
-#pragma unroll
-      for (int k = 0; k < S; k++) {
-        r[i][k] = k >= i ? R[i][k] : make_double2(0, 0);
-        d[i][k] = make_double2(0, 0);
-      }
-    bool ok = true;
-#pragma unroll
-    for (int i = 0; i < S; i++) {
-      double p = r[i][i].x;
-#pragma unroll
-      for (int l = 0; l < i; l++) p -= r[l][i].x * r[l][i].x + r[l][i].y * r[l][i].y;
-      const double g = G[i][i].x;
-      ok = ok && p > least * g && p > 0;
-      const double h = ok ? sqrt(p) : 0.0, inv = ok ? 1.0 / h : 0.0;
-      if (ok) {
-        least_seen = fmin(least_seen, p / g);
-        n++;
-      }
-      r[i][i] = make_double2(h, 0);
-#pragma unroll
-      for (int k = i + 1; k < S; k++) {
-        double2 x = r[i][k];
-#pragma unroll
-        for (int l = 0; l < i; l++) x = zsub(x, zcmul(r[l][i], r[l][k]));
-        r[i][k] = make_double2(x.x * inv, x.y * inv);
-      }
-      // column i of the inverse
-      d[i][i] = make_double2(inv, 0);
-#pragma unroll
-      for (int l = i - 1; l >= 0; l--) {
-        double2 x = make_double2(0, 0);
-#pragma unroll
-        for (int q = l + 1; q <= i; q++) {
-          const double2 y = zmul(r[l][q], d[q][i]);
-          x.x += y.x;
-          x.y += y.y;
-        }
-        const double f = ok ? -d[l][l].x : 0.0;
-        d[l][i] = make_double2(x.x * f, x.y * f);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < S; i++)
-#pragma unroll
-      for (int k = 0; k < S; k++) {
-        R[i][k] = r[i][k];
-        D[i][k] = d[i][k];
-      }
-    good = n;
-    worst = least_seen;
-  }
-  __syncthreads();
-  // C = -P D, row by row; with `again` the totals P + P2 R, R2 R
-  double grow[S];
-#pragma unroll
-  for (int c = 0; c < S; c++) grow[c] = 0;
-  if (t < nv) {
-    const int k = t;
-#pragma unroll
-    for (int c = 0; c < S; c++) {
-      double2 a = make_double2(0, 0);
-      for (int l = 0; l <= c; l++) {
-        const double2 x = zmul(P[k][l], D[l][c]);
-        a.x -= x.x;
-        a.y -= x.y;
-      }
-      C[k][c] = a;
-      grow[c] += a.x * a.x + a.y * a.y;
-      double2 p = P[k][c];
-      if (again) {
-        p = pr[k * S + c];
-        for (int l = 0; l <= c; l++) {
-          const double2 x = zmul(P[k][l], pr[nv * S + l * S + c]);
-          p.x += x.x;
-          p.y += x.y;
-        }
-      }
-      Pt[k][c] = p;
-    }
-  }
-  if (t < S * S) {
-    const int r = t / S, c = t % S;
-    double2 x = R[r][c];
-    if (again) {
-      x = make_double2(0, 0);
-      for (int l = r; l <= c; l++) {
-        const double2 y = zmul(R[r][l], pr[nv * S + l * S + c]);
-        x.x += y.x;
-        x.y += y.y;
-      }
-    }
-    Rt[r][c] = x;
-  }
-  __syncthreads();
-  // rows of C sit in the first NMAX = 128 threads: two wavefronts
-#pragma unroll
-  for (int c = 0; c < S; c++) {
-    double s = grow[c];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (t < 128 && (t & 63) == 0) red[t >> 6][c] = s;
-  }
-  __syncthreads();
-  double most = 0;
-#pragma unroll
-  for (int c = 0; c < S; c++) most += red[0][c] + red[1][c];
-  for (int i = t; i < nv * S; i += 256) {
-    const double2 x = C[i / S][i % S];
-    coef[i] = x;
-    coef32[i] = make_float2((float)x.x, (float)x.y);
-    pr[i] = Pt[i / S][i % S];
-  }
-  // the update walks the vectors four at a time
-  for (int i = nv * S + t; i < (nv + 3) / 4 * 4 * S; i += 256) {
-    coef[i] = make_double2(0, 0);
-    coef32[i] = make_float2(0, 0);
-  }
-  if (t < S * S) {
-    const double2 x = D[t / S][t % S];
-    coef[NM * SM + t] = x;
-    coef32[NM * SM + t] = make_float2((float)x.x, (float)x.y);
-    pr[nv * S + t] = Rt[t / S][t % S];
-  }
-  // the columns, one after the other: row t of column j + i.  What the old
-  // columns contribute to all of them first (H_k has no rows past k + 1 <= j).
-  double2 old[S];
-#pragma unroll
-  for (int i = 0; i < S; i++) old[i] = make_double2(0, 0);
-  if (S > 1 && t <= j) {
-#pragma unroll 4
-    for (int k = 0; k < j; k++) {
-      const double2 h = hd[t + (long)ld * k];
-#pragma unroll
-      for (int i = 1; i < S; i++) {
-        const double2 x = zmul(Pt[k][i - 1], h);
-        old[i].x += x.x;
-        old[i].y += x.y;
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < S; i++) {
-    const int rows = j + i + 2;
-    if (t < ld) {
-      double2 h = make_double2(0, 0);
-      if (i < good && t < rows) {
-        // coef(u_{i+1}), u_1 first
-        if (t <= j) h = Pt[t][i];
-        else if (t - nv <= i) h = Rt[t - nv][i];
-        if (i > 0) {
-          // B q_i: less what u_i's other components contribute
-          h = zsub(zsub(h, old[i]), zmul(Pt[j][i - 1], col[0][t]));
-#pragma unroll
-          for (int l = 1; l < i; l++) h = zsub(h, zmul(Rt[l - 1][i - 1], col[l][t]));
-          const double inv = 1.0 / Rt[i - 1][i - 1].x;
-          h.x *= inv;
-          h.y *= inv;
-        }
-      }
-      col[i][t] = h;  // read by this thread only
-    }
-  }
-  for (int i = 0; i < S; i++)
-    if (t < ld) {
-      hd[t + (long)ld * (j + i)] = col[i][t];
-      hout[t + (long)ld * i] = col[i][t];
-    }
-  if (t == 0) {
-    info[0] = good;
-    info[1] = sqrt(most);
-    info[2] = worst;
-  }
+  block_columns<S>(BlockIO<S>{sums, hd, pr, coef, coef32, hout, info, ld, g0, j + 1}, j, ld, again, least);
 }
 
 // v_{nv+c} <- sum_l u_l D_lc + sum_k v_k C_kc, u_l = v_{nv+l} before: Q in place

@@ -20,7 +20,7 @@ MultiSchur::MultiSchur(Context &c_, Prec p, int recon, const double k[2], int ca
   kappa[1] = k[1];
 }
 
-void MultiSchur::operator()(const MultiSpinor &in, MultiSpinor &out, const int *nact) {
+void MultiSchur::operator()(const MultiSpinor &in, MultiSpinor &out, const int *nact, bool less_diag) {
   const double k = kappa[0], mu = kappa[1];
   Epilogue e1, e2;
   if (mu < 1e-8) {
@@ -33,8 +33,10 @@ void MultiSchur::operator()(const MultiSpinor &in, MultiSpinor &out, const int *
     e2.a1 = 2.0 * mu / k;
     e2.b0 = -1.0 / (1.0 + a * a);
   }
+  if (less_diag) e2.a0 = 0;
+  const bool own = e2.a0 != 0 || e2.a1 != 0;
   dslash_multi(c.g, U, in, mid(), 1, idag, e1, nullptr, nact, tune, c.stream);
-  dslash_multi(c.g, U, mid(), out, 0, idag, e2, &in, nact, tune, c.stream);
+  dslash_multi(c.g, U, mid(), out, 0, idag, e2, own ? &in : nullptr, nact, tune, c.stream);
 }
 
 bool MultiSchur::can_scale() const { return dslash_multi_can_scale(c.g, tmp.m.prec, tmp.m.nb, tune); }
@@ -129,9 +131,15 @@ class Batch {
   // of the update pass and the per-slot coefficients of the next vector
   bool paired = false;
   std::unique_ptr<MultiBuf> U2f;
+  // blocks of four steps (MBlas::block): B^1..B^4 v_j in Wf, U2f, U3f, U4f,
+  // the next block's FP32 input in Qf; H is then that of B = A - sigma
+  bool quads = false;
+  double sigma = 0.0;
+  std::unique_ptr<MultiBuf> U3f, U4f;
   // device state: ints [0] n_outer, [1] n_inner, [2] any, [3, 3+cap) flags
   DevBuf<int> di;
-  DevBuf<double> h1, h2, n2a, n2b, nf, H, coef, coef2, n2, ssc, sbc, sself;
+  DevBuf<double> h1, h2, n2a, n2b, nf, H, coef, coef2, n2, ssc, sbc, bsum;
+  DevBuf<float> bcoef;
   HostBuf<double> hH, hc, hcoef, hcoef2, hn2;
   std::vector<double> bn, rn, tgt;  // per slot: ||b||, current ||r||, inner target
   BatchStats st;
@@ -158,6 +166,7 @@ class Batch {
   void swap_slots(int a, int b, bool inner_fields);
   void arnoldi_step(int j);
   void arnoldi_block(int j);
+  void arnoldi_quad(int j, int s);
   void arnoldi_cycle();
   void inner();
   void outer_residual();
@@ -194,7 +203,8 @@ Batch::Batch(Context &c_, const double kappa[2], MultiSpinor &B_, MultiSpinor &X
       n2(B_.cap),
       ssc((size_t)4 * B_.cap),
       sbc((size_t)4 * B_.cap),
-      sself((size_t)4 * B_.cap),
+      bsum((size_t)8 * (p_.m + 2) * B_.cap),
+      bcoef((size_t)8 * (p_.m + 2) * B_.cap),
       hH((size_t)2 * p_.m * (p_.m + 1) * B_.cap),
       hc((size_t)2 * (p_.m + 1) * B_.cap),
       hcoef((size_t)2 * (p_.m + 1) * B_.cap),
@@ -221,8 +231,14 @@ Batch::Batch(Context &c_, const double kappa[2], MultiSpinor &B_, MultiSpinor &X
     Qf.reset(new MultiBuf(c.g, PREC_SINGLE, cap, nb));
     fused = p.fuse_norm && A32.can_scale();
     hs = std::sqrt(12.0 * (double)c.g.stride);
-    paired = fused && p.sstep == 2 && p.reorth == 0 && m % 2 == 0;
-    if (paired) U2f.reset(new MultiBuf(c.g, PREC_SINGLE, cap, nb));
+    quads = p.sstep == 2 && p.reorth == 0 && p.pair_norms && MBlas::can_block(m, B.nblk());
+    paired = !quads && fused && p.sstep == 2 && p.reorth == 0 && m % 2 == 0;
+    if (quads) {
+      sigma = A32.diag();
+      U3f.reset(new MultiBuf(c.g, PREC_SINGLE, cap, nb));
+      U4f.reset(new MultiBuf(c.g, PREC_SINGLE, cap, nb));
+    }
+    if (paired || quads) U2f.reset(new MultiBuf(c.g, PREC_SINGLE, cap, nb));
   }
   A32.set_half_mid(p.half_mid != 0);
   mb.reserve(mb.need());
@@ -302,23 +318,27 @@ void Batch::arnoldi_block(int j) {
   if (j == 0) A32(rin, u1, nin);
   else A32.scaled(rin, u1, nin, nf.p, &V[j], hs);
   A32(u1, u2, nin);
-  if (p.pair_norms) {
-    mb.dot2(j + 1, V.data(), u1, u2, nin, h1.p, h2.p, sself.p);
-    pythag_scalars(j + 1, h1.p, h2.p, sself.p, ssc.p, nin, cap, c.stream);
-    sstep_columns(H.p, m + 1, j, h1.p, h2.p, ssc.p, sbc.p, nin, cap, hs, c.stream);
-    mb.axpy2_next(j + 1, V.data(), h1.p, h2.p, u1, u2, sbc.p, rin, V[j + 1], nin, nf.p);
-  } else {
-    mb.dot2(j + 1, V.data(), u1, u2, nin, h1.p, h2.p);
-    mb.axpy2(j + 1, V.data(), h1.p, h2.p, u1, u2, nin, ssc.p);
-    sstep_columns(H.p, m + 1, j, h1.p, h2.p, ssc.p, sbc.p, nin, cap, hs, c.stream);
-    mb.next2(u1, u2, rin, V[j + 1], sbc.p, nin, nf.p);
-  }
+  mb.dot2(j + 1, V.data(), u1, u2, nin, h1.p, h2.p);
+  mb.axpy2(j + 1, V.data(), h1.p, h2.p, u1, u2, nin, ssc.p);
+  sstep_columns(H.p, m + 1, j, h1.p, h2.p, ssc.p, sbc.p, nin, cap, hs, c.stream);
+  mb.next2(u1, u2, rin, V[j + 1], sbc.p, nin, nf.p);
   set_subdiag(H.p, m + 1, j + 1, nf.p, nin, cap, c.stream);
+}
+
+// Arnoldi steps j .. j + s - 1 of every active inner slot in one block: two
+// reads of the basis for up to four steps; device-only (capturable)
+void Batch::arnoldi_quad(int j, int s) {
+  int *nin = d_nin();
+  MultiSpinor *u[4] = {&Wf->m, &U2f->m, &U3f->m, &U4f->m};
+  for (int i = 0; i < s; i++) A32(i ? *u[i - 1] : Qf->m, *u[i], nin, true);
+  mb.block(j, s, V.data(), u, Qf->m, H.p, m + 1, bsum.p, bcoef.p, nin);
 }
 
 void Batch::arnoldi_cycle() {
   auto run_steps = [&]() {
-    if (paired)
+    if (quads)
+      for (int j = 0; j < m; j += 4) arnoldi_quad(j, std::min(4, m - j));
+    else if (paired)
       for (int j = 0; j < m; j += 2) arnoldi_block(j);
     else
       for (int j = 0; j < m; j++) arnoldi_step(j);
@@ -417,6 +437,9 @@ void Batch::inner() {
           jj = j + 1;
           break;
         }
+      // back from B = A - sigma to A (a column that a block gave up is zero)
+      for (int j = 0; j < jj && sigma != 0.0; j++)
+        if (Hs[j + 1 + (size_t)ldh * j] != zd(0.0)) Hs[j + (size_t)ldh * j] += sigma;
       std::fill(cs.begin(), cs.end(), zd(0.0));
       cs[0] = beta[s];
       std::fill(y.begin(), y.end(), zd(0.0));

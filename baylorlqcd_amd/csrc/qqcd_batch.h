@@ -23,7 +23,9 @@ struct MultiSchur {
              int idag_ = 0);
   void set_half_mid(bool on);
   MultiSpinor &mid() { return tmp16 ? tmp16->m : tmp.m; }
-  void operator()(const MultiSpinor &in, MultiSpinor &out, const int *nact);
+  // less_diag: out - in/k^2, the operator without its multiple of the identity
+  void operator()(const MultiSpinor &in, MultiSpinor &out, const int *nact, bool less_diag = false);
+  double diag() const { return 1.0 / (kappa[0] * kappa[0]); }
   // out = A in / ||in|| per slot (n2: ||in||^2 per slot in device memory, 0
   // where it is not positive) and side = hs in / ||in|| as an FP16 field
   // without norms, both in the second hop's epilogue: the normalisation of
@@ -63,16 +65,11 @@ struct BatchParams {
   // FP16 basis: fold each Arnoldi step's normalisation into the next
   // operator application where the launch form allows it
   int fuse_norm = 1;
-  // Arnoldi steps per Gram-Schmidt pass over the basis: 2 runs the steps in
-  // pairs (u1 = A v_j, u2 = A u1, one pass over V for both sets of dots and
-  // one for both updates, column j + 1 from the Arnoldi relation) where the
-  // FP16 basis, the normalising operator, one Gram-Schmidt pass and an even
-  // m allow it; 1 one step at a time
+  // Arnoldi steps per Gram-Schmidt pass over an FP16 basis (one pass): 2 runs
+  // them in blocks -- of four (MBlas::block), or with pair_norms 0, where the
+  // normalising operator and an even m allow it, of two, whose norms come from
+  // the updated vectors in a third pass; 1 one step at a time
   int sstep = 2;
-  // paired steps: 1 takes the norm and inner product of the updated vectors
-  // from those of u1, u2 (formed in the pass of dots) less the projections,
-  // so the update pass also writes the next basis vector and operator input;
-  // 0 computes them from the updated vectors, with a third pass for those two
   int pair_norms = 1;
   // the inner operator's intermediate (odd-checkerboard) field in FP16 with
   // norms where the two-slot kernel runs (1), or in FP32 (0)

@@ -15,6 +15,7 @@
 #include <stdexcept>
 #include <type_traits>
 
+#include "qqcd_blockalg.h"
 #include "qqcd_multi.h"
 
 namespace qqcd {
@@ -379,14 +380,13 @@ __global__ void k_arnoldi_column(double *H, int ldh, int j, const double *h1, co
 // ---- two-step Arnoldi block (FP16 basis V, FP32 W1 = A v_j, W2 = A W1) ----
 // Per-lane sums in FP32 (the basis carries 11 bits), across lanes in FP64.
 
-// part[((c * cap + slot) * gx + bx]: c < 2K <V_k, W1>, then 2K + c <V_k, W2>;
-// SELF: then ||W1||^2, Re <W1, W2>, Im <W1, W2>, ||W2||^2
-template <int K, bool SELF>
+// part[((c * cap + slot) * gx + bx]: c < 2K <V_k, W1>, then 2K + c <V_k, W2>
+template <int K>
 __global__ void __launch_bounds__(MB) k_mdot2(MShape a, MPtr v, const void *w1, const void *w2, double *part) {
   const int nact = *a.nact, nb = 1 << a.lognb, blk = blockIdx.y;
   if ((blk << a.lognb) >= nact) return;
   const int rr = threadIdx.x & (nb - 1), slot = (blk << a.lognb) + rr;
-  constexpr int NV = 4 * K + (SELF ? 4 : 0);
+  constexpr int NV = 4 * K;
   float af[NV];
 #pragma unroll
   for (int k = 0; k < NV; k++) af[k] = 0.f;
@@ -407,12 +407,6 @@ __global__ void __launch_bounds__(MB) k_mdot2(MShape a, MPtr v, const void *w1, 
         af[2 * k + 1] += xx * b1[1] - xy * b1[0];
         af[2 * K + 2 * k] += xx * b2[0] + xy * b2[1];
         af[2 * K + 2 * k + 1] += xx * b2[1] - xy * b2[0];
-      }
-      if (SELF) {
-        af[4 * K] += b1[0] * b1[0] + b1[1] * b1[1];
-        af[4 * K + 1] += b1[0] * b2[0] + b1[1] * b2[1];
-        af[4 * K + 2] += b1[0] * b2[1] - b1[1] * b2[0];
-        af[4 * K + 3] += b2[0] * b2[0] + b2[1] * b2[1];
       }
     }
   }
@@ -471,91 +465,6 @@ __global__ void __launch_bounds__(MB) k_maxpy2(MShape a, MPtr v, const double *g
     }
   }
   if (LAST) slot_sum<4>(acc, a.lognb, part, a.cap, blk << a.lognb, a.gx);
-}
-
-// The last chunk of axpy2 with next2 folded in: W1' = W1 - sum_k g1_k V_k and
-// W2' likewise stay in registers, R = b0 W2' + (b1 + i b2) W1' (FP32) and
-// H = b3 W1' (FP16) are stored, with partials of ||R||^2 of the stored values.
-// The coefficients b come before the pass, from norms and inner products of
-// W1', W2' formed from those of W1, W2 and the projections (pythag_scalars).
-template <int K>
-__global__ void __launch_bounds__(MB) k_maxpy2n(MShape a, MPtr v, const double *g1, const double *g2, int q0,
-                                                const void *w1, const void *w2, void *rout, void *hout,
-                                                const double *b, double *part) {
-  const int nact = *a.nact, nb = 1 << a.lognb, blk = blockIdx.y;
-  if ((blk << a.lognb) >= nact) return;
-  const int rr = threadIdx.x & (nb - 1), slot = (blk << a.lognb) + rr;
-  double acc[1] = {0.0};
-  if (slot < nact) {
-    float c1r[K], c1i[K], c2r[K], c2i[K];
-    const double f = a.hinv;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-      const long o = 2 * ((long)(q0 + k) * a.cap + slot);
-      c1r[k] = (float)(f * g1[o]);
-      c1i[k] = (float)(f * g1[o + 1]);
-      c2r[k] = (float)(f * g2[o]);
-      c2i[k] = (float)(f * g2[o + 1]);
-    }
-    const float s2 = (float)b[4 * slot], s1r = (float)b[4 * slot + 1], s1i = (float)b[4 * slot + 2],
-                sv = (float)b[4 * slot + 3];
-    const int per = MB >> a.lognb;
-    const long base = (long)blk * a.blk_elems;
-    typedef typename E2<float>::raw f2;
-    typedef typename E2<f16>::raw h2;
-    float nr = 0.f;
-    for (long p = (long)blockIdx.x * per + (threadIdx.x >> a.lognb); p < a.rows; p += (long)a.gx * per) {
-      const long e = base + (p << a.lognb) + rr;
-      f2 b1 = E2<float>::ldr(w1, e), b2 = E2<float>::ldr(w2, e);
-      typename E2<f16>::raw xr[K];
-#pragma unroll
-      for (int k = 0; k < K; k++) xr[k] = E2<f16>::ldr(v.p[k], e);
-      pin_loads(xr);
-#pragma unroll
-      for (int k = 0; k < K; k++) {
-        const float xx = (float)xr[k][0], xy = (float)xr[k][1];
-        b1[0] -= c1r[k] * xx - c1i[k] * xy;
-        b1[1] -= c1r[k] * xy + c1i[k] * xx;
-        b2[0] -= c2r[k] * xx - c2i[k] * xy;
-        b2[1] -= c2r[k] * xy + c2i[k] * xx;
-      }
-      f2 r;
-      r[0] = s2 * b2[0] + (s1r * b1[0] - s1i * b1[1]);
-      r[1] = s2 * b2[1] + (s1r * b1[1] + s1i * b1[0]);
-      ((f2 *)rout)[e] = r;
-      h2 hv;
-      hv[0] = (f16)(sv * b1[0]);
-      hv[1] = (f16)(sv * b1[1]);
-      ((h2 *)hout)[e] = hv;
-      nr += r[0] * r[0] + r[1] * r[1];
-    }
-    acc[0] = (double)nr;
-  }
-  slot_sum<1>(acc, a.lognb, part, a.cap, blk << a.lognb, a.gx);
-}
-
-// One thread per slot: sc = (||W1'||^2, Re <W1', W2'>, Im <W1', W2'>,
-// ||W2'||^2) of W1' = W1 - V g1, W2' = W2 - V g2 from self = the same four of
-// W1, W2 and the projections g = <V_k, W> (V orthonormal: ||W1'||^2 = ||W1||^2
-// - sum |g1_k|^2, <W1', W2'> = <W1, W2> - sum conj(g1_k) g2_k).
-__global__ void k_pythag_scalars(int nq, const double *g1, const double *g2, const double *self, double *sc,
-                                 const int *nact, int cap) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= cap || r >= *nact) return;
-  double n1 = 0.0, cr = 0.0, ci = 0.0, n2 = 0.0;
-  for (int q = 0; q < nq; q++) {
-    const long o = 2 * ((long)q * cap + r);
-    const double ar = g1[o], ai = g1[o + 1], br = g2[o], bi = g2[o + 1];
-    n1 += ar * ar + ai * ai;
-    n2 += br * br + bi * bi;
-    cr += ar * br + ai * bi;
-    ci += ar * bi - ai * br;
-  }
-  const double p1 = self[r] - n1;
-  sc[r] = p1 > 0.0 ? p1 : 0.0;
-  sc[cap + r] = self[cap + r] - cr;
-  sc[2 * cap + r] = self[2 * cap + r] - ci;
-  sc[3 * cap + r] = self[3 * cap + r] - n2;
 }
 
 // R = b0 W2 + (b1 + i b2) W1 in FP32, H = b3 W1 in FP16 (b per slot, 4 doubles),
@@ -654,6 +563,228 @@ __global__ void k_set_subdiag(double *H, int ldh, int j, const double *n2, const
   H[2 * (((long)j * ldh + j + 1) * cap + r) + 1] = 0.0;
 }
 
+// ---- blocks of up to four Arnoldi steps (FP16 basis V, FP32 u_c = B^c v_j) ----
+
+static constexpr int BQ = 6;     // basis fields of a wavefront in the pass of dots
+static constexpr int BWV = 8;    // its wavefronts at most: 7 BQ fields and the u_c
+static constexpr int BCH = (BWV - 1) * BQ;  // basis fields of one launch of the pass
+struct BTab {
+  void *p[128];
+};
+struct BUTab {
+  const void *p[4];
+};
+
+// part[((2 (q S + c) + {0, 1}) cap + slot) gx + bx]: <V_{q0+q}, u_c> for q < nq, then (with a wavefront more)
+// <u_q, u_c>.
+//
+// Bound by reading the basis: the wavefronts of a workgroup take BQ fields each (the last one the u_c) of the same
+// 64 elements, so the u_c come from memory once and from the L1 for the other wavefronts.  Sums in FP32 within a lane
+// (the basis carries 11 bits), in FP64 across lanes; two elements are in flight, one is worked on.  16^3x32, 23
+// sources, 1..37 basis vectors: 591 us a block of four with 6 fields a wavefront, 631 with 8 (141 registers), 606
+// with 4; with the update below 1.23 ms for four steps, where two pairs of steps took about 1.5.
+template <int S>
+__global__ void __launch_bounds__(64 * BWV) k_mbdot(MShape a, BTab v, BUTab ut, int q0, int nq, double *part) {
+  const int nact = *a.nact, nb = 1 << a.lognb, blk = blockIdx.y;
+  if ((blk << a.lognb) >= nact) return;
+  const int lane = threadIdx.x & 63, rr = lane & (nb - 1), slot = (blk << a.lognb) + rr;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = (nq + BQ - 1) / BQ, k0 = wv * BQ;
+  typedef typename E2<float>::raw f2;
+  typedef typename E2<f16>::raw h2;
+  // the 64 elements of a wavefront are consecutive: a uniform address and the lane (12 stride is a multiple of 64)
+  const long base = (long)blk * a.blk_elems, groups = a.rows >> (6 - a.lognb);
+  float af[2 * BQ * S];
+#pragma unroll
+  for (int k = 0; k < 2 * BQ * S; k++) af[k] = 0.f;
+  auto add = [&](float x, float y, const f2(&u)[S], int q) {
+#pragma unroll
+    for (int c = 0; c < S; c++) {
+      float &re = af[2 * (q * S + c)], &im = af[2 * (q * S + c) + 1];
+      re = fmaf(y, u[c][1], fmaf(x, u[c][0], re));
+      im = fmaf(-y, u[c][0], fmaf(x, u[c][1], im));
+    }
+  };
+  int left = S;
+  if (wv < nw) {
+    left = nq - k0 < BQ ? nq - k0 : BQ;
+    if (slot < nact) {
+      const h2 *vp[BQ];
+      const f2 *up[S];
+#pragma unroll
+      for (int k = 0; k < BQ; k++) vp[k] = (const h2 *)v.p[q0 + (k < left ? k0 + k : nq - 1)] + base;
+#pragma unroll
+      for (int c = 0; c < S; c++) up[c] = (const f2 *)ut.p[c] + base;
+      const unsigned l4 = (threadIdx.x & 63) * 4u;
+      h2 x[2][BQ];
+      f2 u[2][S];
+      auto fetch = [&](int h, long g) {
+#pragma unroll
+        for (int k = 0; k < BQ; k++) x[h][k] = *(const h2 *)((const char *)(vp[k] + g * 64) + l4);
+#pragma unroll
+        for (int c = 0; c < S; c++) u[h][c] = *(const f2 *)((const char *)(up[c] + g * 64) + 2 * l4);
+      };
+      auto work = [&](int h) {
+#pragma unroll
+        for (int k = 0; k < BQ; k++) add((float)x[h][k][0], (float)x[h][k][1], u[h], k);
+      };
+      long g = blockIdx.x;
+      const long st = a.gx;
+      fetch(0, g);
+      for (; g + 2 * st < groups; g += 2 * st) {
+        fetch(1, g + st);
+        work(0);
+        fetch(0, g + 2 * st);
+        work(1);
+      }
+      if (g + st < groups) {
+        fetch(1, g + st);
+        work(0);
+        work(1);
+      } else {
+        work(0);
+      }
+    }
+    const float f = (float)a.hinv;
+#pragma unroll
+    for (int k = 0; k < 2 * BQ * S; k++) af[k] *= f;
+  } else if (slot < nact) {
+    for (long g = blockIdx.x; g < groups; g += a.gx) {
+      f2 u[S];
+#pragma unroll
+      for (int c = 0; c < S; c++) u[c] = ((const f2 *)ut.p[c] + base + g * 64)[lane];
+#pragma unroll
+      for (int q = 0; q < S; q++) add(u[q][0], u[q][1], u, q);
+    }
+  }
+  const int first = wv < nw ? k0 : nq;
+#pragma unroll
+  for (int k = 0; k < 2 * BQ * S; k++) {
+    double s = (double)af[k];
+    for (int o = 32; o >= nb; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (k < 2 * left * S && lane < nb && slot < nact)
+      part[((long)(2 * first * S + k) * a.cap + slot) * a.gx + blockIdx.x] = s;
+  }
+}
+
+// block_columns for slot blockIdx.x: sums complex [(q S + c) cap + slot], H as the batched Hessenberg matrix (of B),
+// coefficients (FP32) [((k S + c) cap + slot)], C for the stored (scaled) basis fields, then D
+template <int S> struct MBlockIO {
+  const double2 *sums;
+  double2 *H;
+  float2 *cf;
+  int ldh, cap, slot, nv;
+  double hinv;
+  __device__ double2 p(int k, int c) const { return sums[(long)(k * S + c) * cap + slot]; }
+  __device__ double2 g(int r, int c) const { return sums[(long)((nv + r) * S + c) * cap + slot]; }
+  __device__ double2 p1(int, int) const { return make_double2(0, 0); }
+  __device__ double2 r1(int, int) const { return make_double2(0, 0); }
+  __device__ void coef(int k, int c, double2 x, double2) {
+    cf[(long)(k * S + c) * cap + slot] = make_float2((float)(hinv * x.x), (float)(hinv * x.y));
+  }
+  __device__ void factor(int r, int c, double2 d, double2) {
+    cf[(long)((nv + r) * S + c) * cap + slot] = make_float2((float)d.x, (float)d.y);
+  }
+  __device__ double2 h(int row, int col) const { return H[((long)col * ldh + row) * cap + slot]; }
+  __device__ void put(int row, int col, int, double2 x) { H[((long)col * ldh + row) * cap + slot] = x; }
+  __device__ void info(int, double, double) {}
+};
+template <int S>
+__global__ void __launch_bounds__(256) k_mbcols(int j, int ldh, int cap, const int *nact, double hinv,
+                                                const double2 *sums, double2 *H, float2 *cf) {
+  const int slot = blockIdx.x;
+  if (slot >= *nact) return;
+  // FP32 sums of an operator with an FP16 intermediate: below 1e-6 of its squared norm a vector is their rounding
+  block_columns<S>(MBlockIO<S>{sums, H, cf, ldh, cap, slot, j + 1, hinv}, j, ldh, 0, 1e-6);
+}
+
+// V_{nq+c} = hs (sum_l D_lc u_l + sum_k C_kc V_k) in FP16, the last one in FP32 (unscaled) too: the next block's
+// operator input.  Bound by reading the basis and the u_c once.  A slot's coefficients come from LDS, where the lanes
+// of other sites share them, and a lane takes two sites per read of them; where they do not fit (wide slot blocks over
+// a large basis) each lane reads its slot's from the cache.  16^3x32, 23 sources, 1..37 basis vectors: 635 us a block
+// of four, 3.9 TB/s.
+template <int S, bool LDS>
+__global__ void __launch_bounds__(MB) k_mbupd(MShape a, BTab v, BUTab ut, int nq, const float2 *cf, void *rout) {
+  extern __shared__ float2 cs[];  // [nq + S][nb][S]
+  const int nact = *a.nact, nb = 1 << a.lognb, blk = blockIdx.y;
+  if ((blk << a.lognb) >= nact) return;
+  const int rr = threadIdx.x & (nb - 1), slot = (blk << a.lognb) + rr;
+  if constexpr (LDS) {
+    for (int i = threadIdx.x >> a.lognb; i < (nq + S) * S; i += MB >> a.lognb)
+      cs[(((i / S) << a.lognb) + rr) * S + i % S] = slot < nact ? cf[(long)i * a.cap + slot] : make_float2(0.f, 0.f);
+    __syncthreads();
+  }
+  if (slot >= nact) return;
+  auto coef = [&](int k, float2(&z)[S]) {
+#pragma unroll
+    for (int c = 0; c < S; c++) z[c] = LDS ? cs[((k << a.lognb) + rr) * S + c] : cf[(long)(k * S + c) * a.cap + slot];
+  };
+  typedef typename E2<float>::raw f2;
+  typedef typename E2<f16>::raw h2;
+  const float hs = (float)a.hs;
+  auto mac = [](f2 &s, float2 z, float x, float y) {
+    s[0] = fmaf(-z.y, y, fmaf(z.x, x, s[0]));
+    s[1] = fmaf(z.y, x, fmaf(z.x, y, s[1]));
+  };
+  const long base = (long)blk * a.blk_elems, n = a.rows << a.lognb, step = (long)a.gx * MB;
+  for (long q0 = (long)blockIdx.x * MB; q0 + threadIdx.x < n; q0 += 2 * step) {
+    const bool two = q0 + step + threadIdx.x < n;
+    const long e0 = base + q0, e1 = two ? e0 + step : e0;
+    f2 s0[S], s1[S];
+    {
+      f2 u0[S], u1[S];
+#pragma unroll
+      for (int c = 0; c < S; c++) {
+        u0[c] = ((const f2 *)ut.p[c] + e0)[threadIdx.x];
+        u1[c] = ((const f2 *)ut.p[c] + e1)[threadIdx.x];
+      }
+#pragma unroll
+      for (int c = 0; c < S; c++) s0[c][0] = s0[c][1] = s1[c][0] = s1[c][1] = 0.f;
+#pragma unroll
+      for (int l = 0; l < S; l++) {
+        float2 d[S];
+        coef(nq + l, d);
+#pragma unroll
+        for (int c = l; c < S; c++) {
+          mac(s0[c], d[c], u0[l][0], u0[l][1]);
+          mac(s1[c], d[c], u1[l][0], u1[l][1]);
+        }
+      }
+    }
+    for (int k0 = 0; k0 < nq; k0 += 4) {
+      h2 x0[4], x1[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const h2 *q = (const h2 *)v.p[k0 + k < nq ? k0 + k : nq - 1];
+        x0[k] = (q + e0)[threadIdx.x];
+        x1[k] = (q + e1)[threadIdx.x];
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        if (k0 + k >= nq) break;
+        float2 z[S];
+        coef(k0 + k, z);
+#pragma unroll
+        for (int c = 0; c < S; c++) {
+          mac(s0[c], z[c], (float)x0[k][0], (float)x0[k][1]);
+          mac(s1[c], z[c], (float)x1[k][0], (float)x1[k][1]);
+        }
+      }
+    }
+    auto put = [&](long e, const f2(&s)[S]) {
+#pragma unroll
+      for (int c = 0; c < S; c++) {
+        h2 h;
+        h[0] = (f16)(hs * s[c][0]);
+        h[1] = (f16)(hs * s[c][1]);
+        ((h2 *)v.p[nq + c] + e)[threadIdx.x] = h;
+      }
+      ((f2 *)rout + e)[threadIdx.x] = s[S - 1];
+    };
+    put(e0, s0);
+    if (two) put(e1, s1);
+  }
+}
+
 // ===================================================================== //
 
 static size_t esize(Prec p) { return p == PREC_DOUBLE ? 16 : p == PREC_SINGLE ? 8 : 4; }
@@ -716,7 +847,9 @@ static int gx_of(long rows, int nb, int nblk) {
 // (MAXK complex dots and a norm, or MAXK2 complex dots with each of two
 // fields): sized once, before any capture, so that no later pass moves the
 // buffer a captured graph names
-size_t MBlas::need() const { return (size_t)2048 * std::max(2 * MAXK + 2, 4 * MAXK2 + 4) * cap + 64; }
+size_t MBlas::need() const {
+  return std::max((size_t)2048 * std::max(2 * MAXK + 2, 4 * MAXK2 + 4) * cap, (size_t)8 * (BCH + 4) * 1024 * std::min(cap, 64)) + 64;
+}
 
 static MShape shape(const MultiSpinor &W, const int *nact) {
   MShape a;
@@ -981,7 +1114,7 @@ static void basis_fields(int nq, const MultiSpinor *V, const MultiSpinor &W, std
 }
 
 void MBlas::dot2(int nq, const MultiSpinor *V, const MultiSpinor &W1, const MultiSpinor &W2, const int *nact,
-                 double *g1, double *g2, double *self) {
+                 double *g1, double *g2) {
   if (W1.prec != PREC_SINGLE || W2.prec != PREC_SINGLE) throw std::runtime_error("MBlas::dot2: FP32 W1, W2");
   same_layout2(W1, W2, "MBlas::dot2");
   std::vector<const void *> vp;
@@ -990,71 +1123,84 @@ void MBlas::dot2(int nq, const MultiSpinor *V, const MultiSpinor &W1, const Mult
   reserve((size_t)a.gx * (4 * MAXK2 + 4) * W1.cap);
   for (int q0 = 0, K; q0 < nq; q0 += K) {
     K = chunk_len(nq, q0, MAXK2);
-    const bool with_self = self && q0 == 0;
     MPtr pk{};
     for (int k = 0; k < K; k++) pk.p[k] = vp[q0 + k];
     dim3 grid(a.gx, W1.nblk());
     with_k<MAXK2>(K, [&](auto kk) {
       constexpr int KK = decltype(kk)::value;
-      if (with_self)
-        hipLaunchKernelGGL((k_mdot2<KK, true>), grid, dim3(MB), 0, stream, a, pk, W1.data, W2.data, part);
-      else
-        hipLaunchKernelGGL((k_mdot2<KK, false>), grid, dim3(MB), 0, stream, a, pk, W1.data, W2.data, part);
+      hipLaunchKernelGGL(k_mdot2<KK>, grid, dim3(MB), 0, stream, a, pk, W1.data, W2.data, part);
     });
     QQCD_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_mfinal, dim3(W1.cap, 2 * K), dim3(64), 0, stream, 2 * K, W1.cap, a.gx, nact,
                        (const double *)part, g1, q0, 1);
     hipLaunchKernelGGL(k_mfinal, dim3(W1.cap, 2 * K), dim3(64), 0, stream, 2 * K, W1.cap, a.gx, nact,
                        (const double *)part + (size_t)2 * K * W1.cap * a.gx, g2, q0, 1);
-    if (with_self)
-      hipLaunchKernelGGL(k_mfinal, dim3(W1.cap, 4), dim3(64), 0, stream, 4, W1.cap, a.gx, nact,
-                         (const double *)part + (size_t)4 * K * W1.cap * a.gx, self, 0, 0);
     QQCD_HIP(hipGetLastError());
   }
 }
 
-void MBlas::axpy2_next(int nq, const MultiSpinor *V, const double *g1, const double *g2, MultiSpinor &W1,
-                       MultiSpinor &W2, const double *b, MultiSpinor &R, MultiSpinor &H, const int *nact, double *nr) {
-  if (W1.prec != PREC_SINGLE || W2.prec != PREC_SINGLE || R.prec != PREC_SINGLE)
-    throw std::runtime_error("MBlas::axpy2_next: FP32 W1, W2, R");
-  if (W1.data == W2.data) throw std::runtime_error("MBlas::axpy2_next: W1 and W2 alias");
-  if (!basis16(H)) throw std::runtime_error("MBlas::axpy2_next: H must be an FP16 basis field");
-  same_layout2(W1, W2, "MBlas::axpy2_next");
-  same_layout2(W1, R, "MBlas::axpy2_next");
-  same_layout2(W1, H, "MBlas::axpy2_next");
-  if (R.data == W1.data || R.data == W2.data) throw std::runtime_error("MBlas::axpy2_next: R aliases W1 or W2");
-  if (nq < 1) throw std::runtime_error("MBlas::axpy2_next: at least one basis field");
+// grid along the rows of the block's pass of dots: at most about 1024 workgroups in all, so that its partials
+// (8 values for each of at most BCH fields and every slot) fit need(): nblk >= cap / nb, so
+// cap gx <= 1024 min(cap, 64)
+static int block_gx(long rows, int nb, int nblk) {
+  const long groups = (rows * nb + 63) / 64;
+  return (int)std::max(1L, std::min(groups, (long)(1024 / nblk)));
+}
+
+bool MBlas::can_block(int m, int nblk) { return m < 128 && nblk <= 1024; }
+
+template <typename F> static void with_s(int s, F &&f) {
+  switch (s) {
+    case 1: f(std::integral_constant<int, 1>()); break;
+    case 2: f(std::integral_constant<int, 2>()); break;
+    case 3: f(std::integral_constant<int, 3>()); break;
+    case 4: f(std::integral_constant<int, 4>()); break;
+    default: throw std::runtime_error("MBlas: 1..4 steps a block");
+  }
+}
+
+void MBlas::block(int j, int s, MultiSpinor *V, const MultiSpinor *const *U, MultiSpinor &R, double *H, int ldh,
+                  double *sums, float *coef, const int *nact) {
+  const int nq = j + 1;
+  if (s < 1 || s > 4 || j < 0 || j + s >= ldh || ldh > 128 || !can_block(j + s, R.nblk()))
+    throw std::runtime_error("MBlas::block: bad block");
+  if (R.prec != PREC_SINGLE) throw std::runtime_error("MBlas::block: FP32 work fields");
   std::vector<const void *> vp;
-  basis_fields(nq, V, W1, vp, "MBlas::axpy2_next");
-  for (int q = 0; q < nq; q++)
-    if (vp[q] == H.data) throw std::runtime_error("MBlas::axpy2_next: H is one of the basis fields read");
-  const MShape a = shape(W1, nact);
-  reserve((size_t)a.gx * W1.cap);
-  for (int q0 = 0, K; q0 < nq; q0 += K) {
-    K = chunk_len(nq, q0, MAXK2);
-    const bool last = q0 + K >= nq;
-    MPtr pk{};
-    for (int k = 0; k < K; k++) pk.p[k] = vp[q0 + k];
-    dim3 grid(a.gx, W1.nblk());
-    with_k<MAXK2>(K, [&](auto kk) {
-      constexpr int KK = decltype(kk)::value;
-      if (last)
-        hipLaunchKernelGGL((k_maxpy2n<KK>), grid, dim3(MB), 0, stream, a, pk, g1, g2, q0, W1.data, W2.data, R.data,
-                           H.data, b, part);
-      else
-        hipLaunchKernelGGL((k_maxpy2<KK, false>), grid, dim3(MB), 0, stream, a, pk, g1, g2, q0, W1.data, W2.data,
-                           part);
-    });
-    QQCD_HIP(hipGetLastError());
+  basis_fields(nq + s, V, R, vp, "MBlas::block");
+  BTab tab{};
+  for (int q = 0; q < nq + s; q++) tab.p[q] = const_cast<void *>(vp[q]);
+  BUTab ut{};
+  for (int c = 0; c < s; c++) {
+    if (U[c]->prec != PREC_SINGLE || U[c]->data == R.data) throw std::runtime_error("MBlas::block: FP32 work fields");
+    same_layout2(*U[c], R, "MBlas::block");
+    ut.p[c] = U[c]->data;
   }
-  hipLaunchKernelGGL(k_mfinal, dim3(W1.cap, 1), dim3(64), 0, stream, 1, W1.cap, a.gx, nact, (const double *)part, nr,
-                     0, 0);
-  QQCD_HIP(hipGetLastError());
-}
-
-void pythag_scalars(int nq, const double *g1, const double *g2, const double *self, double *sc, const int *nact,
-                    int cap, hipStream_t s) {
-  hipLaunchKernelGGL(k_pythag_scalars, dim3((cap + 63) / 64), dim3(64), 0, s, nq, g1, g2, self, sc, nact, cap);
+  MShape a = shape(R, nact);
+  const int gu = a.gx;
+  a.gx = block_gx(a.rows, R.nb, R.nblk());
+  reserve(need());
+  with_s(s, [&](auto SS) {
+    constexpr int S = decltype(SS)::value;
+    for (int q0 = 0; q0 < nq; q0 += BCH) {
+      const int n = std::min(BCH, nq - q0), last = q0 + n == nq;
+      const int nv = 2 * S * (n + (last ? S : 0));
+      hipLaunchKernelGGL((k_mbdot<S>), dim3(a.gx, R.nblk()), dim3(64 * ((n + BQ - 1) / BQ + last)), 0, stream, a, tab,
+                         ut, q0, n, part);
+      hipLaunchKernelGGL(k_mfinal, dim3(R.cap, nv), dim3(64), 0, stream, nv, R.cap, a.gx, nact, (const double *)part,
+                         sums, q0 * S, 1);
+    }
+    hipLaunchKernelGGL((k_mbcols<S>), dim3(R.cap), dim3(256), 0, stream, j, ldh, R.cap, nact, a.hinv,
+                       (const double2 *)sums, (double2 *)H, (float2 *)coef);
+    a.gx = gu;
+    // coefficients in LDS while four workgroups of a CU hold theirs
+    const size_t lds = sizeof(float2) * S * (nq + S) * R.nb;
+    if (lds <= 40960)
+      hipLaunchKernelGGL((k_mbupd<S, true>), dim3(a.gx, R.nblk()), dim3(MB), lds, stream, a, tab, ut, nq,
+                         (const float2 *)coef, R.data);
+    else
+      hipLaunchKernelGGL((k_mbupd<S, false>), dim3(a.gx, R.nblk()), dim3(MB), 0, stream, a, tab, ut, nq,
+                         (const float2 *)coef, R.data);
+  });
   QQCD_HIP(hipGetLastError());
 }
 

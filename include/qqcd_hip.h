@@ -420,23 +420,19 @@ int qqcd_trace16(const double *eta_e, const double *eta_o, const double *x_e, co
 int qqcd_batch_set(int reorth, int use_graph, double inner_tol, int inner_cycles, int max_outer, int op_prec,
                    int op_recon, int basis_prec);
 
-/* Arnoldi steps per Gram-Schmidt pass over an FP16 Krylov basis, in the
- * batched and the single-right-hand-side solvers: 2 (the default) runs the
- * steps in pairs -- u1 = A v_j, u2 = A u1, the dots of both and the updates
- * of both in one pass each over the basis, column j + 1 of the Hessenberg
- * matrix from the Arnoldi relation -- where one Gram-Schmidt pass (and, in
- * the batched solver, the two-slot operator and an even cycle length)
- * allows it; 1 one step at a time.  The single-right-hand-side solvers over
- * an FP64 or FP32 basis run four steps per pair of passes with 2, one with 1.
- * Tuning aid; no reference counterpart. */
+/* Arnoldi steps per Gram-Schmidt pass over the Krylov basis, in the batched
+ * (FP16 basis) and the single-right-hand-side solvers: 2 (the default) runs
+ * the steps in blocks of four -- four operator applications, the dots of all
+ * four and the updates of all four in one pass each over the basis, the
+ * Hessenberg columns from the operator's relations -- where one Gram-Schmidt
+ * pass is enough (qqcd_batch_set's reorth 0); 1 one step at a time.  Tuning
+ * aid; no reference counterpart. */
 int qqcd_set_arnoldi_steps(int steps);
 
-/* Paired Arnoldi steps of the batched solver: 1 (the default) takes the norm
- * of u1' = u1 - V V^H u1 and <u1', u2'> from those of u1, u2 (formed in the
- * pass of dots) less the projections, so that the update pass also writes
- * the next basis vector and the next operator input; 0 computes them from the
- * updated vectors, with a third pass over the pair.  Tuning aid; no reference
- * counterpart. */
+/* Blocks of the batched solver: 1 (the default) runs blocks of four steps; 0
+ * blocks of two, whose norms come from the updated vectors with a third pass
+ * over the pair (with the two-slot operator and an even cycle length; one step
+ * at a time otherwise).  Tuning aid; no reference counterpart. */
 int qqcd_set_pair_norms(int mode);
 
 /* Storage of the batched solver's inner operator's intermediate field (the
