@@ -608,7 +608,8 @@ TuneResult autotune_multi(Context &c, Prec p, int recon, int nrhs) {
         // a larger RHS block must beat the best smaller one by 5%: the hop is
         // a third of a batched step, and the passes over the slots' bases run
         // faster in smaller blocks (63 sources at 24^3x48: 10.5 s with block
-        // 16 against 11.0 s with block 32, whose hop was 3% faster)
+        // 16 against 11.0 s with block 32, whose hop was 3% faster; 23 sources at
+        // 16^3x32: 274 ms with 8, 355 with 16, 375 with 32)
         const double need = best.nb > 0 && nb > best.nb ? 0.95 * best.ms : best.ms;
         if (per < need) {
           best.ms = per;

@@ -13,10 +13,12 @@
 //    alternated with GMRES(m) cycles.
 //  * BiCGStab (inverters.f90:302-487).
 //
-// Differences of mechanism (same mathematics): the basis is orthogonalised
-// by classical Gram-Schmidt with one reorthogonalisation (two fused
-// multi-dot / multi-axpy passes per step) instead of modified Gram-Schmidt
-// (j dependent reductions per step, :3120-3140); the solution is formed
+// Differences of mechanism (same mathematics): the basis grows in blocks of
+// four steps, two passes over it and one synchronisation per block
+// (qqcd_arnoldi.h), or where a block cannot run (a preconditioner, a hook on
+// every step, more than 128 vectors) step by step by classical Gram-Schmidt
+// with one reorthogonalisation, instead of modified Gram-Schmidt (j dependent
+// reductions per step, :3120-3140); the solution is formed
 // once per cycle instead of at every Arnoldi step (:3242-3255); the small
 // least-squares problem is solved by Householder QR on the host; a cycle ends
 // early when its least-squares residual already meets the tolerance.
@@ -170,14 +172,14 @@ void set_arnoldi_steps(int steps) {
 }
 int arnoldi_steps() { return g_arnoldi_steps; }
 
-// Groups of synchronisation-free steps replayed from HIP graphs: a group
+// Groups of synchronisation-free single steps replayed from HIP graphs: a group
 // [j0, j0 + n) that already ran on the same vectors is launched as one
 // graph, which removes the launch gaps between its ~13 kernels per step.
 // Only for operators whose buffers stay put between applications (every
 // LinOp here except a preconditioner's).  A graph captured within one call
 // on a fresh basis is replayed about three times, and then the captures
-// cost more than the replays save (32^3x64 mixed FP16 solve: 1.32-1.35 s
-// with graphs, 1.25 s without); so by default (mode 2) graphs are kept only
+// cost more than the replays save (32^3x64 mixed FP16 solve, one step at a
+// time: 1.32-1.35 s with graphs, 1.25 s without); so by default (mode 2) graphs are kept only
 // with a ProjWork, whose basis outlives the call and whose graphs serve
 // every later outer step of the mixed solver.
 static int g_step_graphs = 2;

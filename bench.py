@@ -194,7 +194,7 @@ def rows_section(no_cpu=False):
     stream and the reference's heatbath sweep drawing from it."""
     V = int(np.prod(N))
     L = _lib.lib()
-    # HBM bytes per launch from the hardware counters (profiles/traffic_smear_lagfib_32x32x32x64.md)
+    # HBM bytes per launch of the generator from the hardware counters (profiles/traffic_smear_lagfib_32x32x32x64.md)
     traffic = {}
     tpath = os.path.join(ROOT, "profiles", "traffic_smear_lagfib_32x32x32x64.json")
     if os.path.exists(tpath):
@@ -202,13 +202,12 @@ def rows_section(no_cpu=False):
             traffic = json.load(f)
     ms = np.zeros(1)
     _lib.check(L.qqcd_bench_smear(3, 20, _lib.dp(ms)))
-    # unique bytes per output site and checkerboard launch: the site's own and the other
-    # checkerboard's input spinor, the six spatial links of its hops and the output once (FP64)
-    g = 1440 * V / (ms[0] * 1e-3) / 1e9
-    smear = {"us_per_iteration": round(ms[0] * 1e3, 1), "bytes_per_site": 1440, "bytes_model": "unique",
+    # unique bytes per site and iteration (one launch over both checkerboards): the input and
+    # output spinor and the three spatial links once (FP64)
+    g = 816 * V / (ms[0] * 1e-3) / 1e9
+    smear = {"us_per_iteration": round(ms[0] * 1e3, 1), "bytes_per_site": 816, "bytes_model": "unique",
              "GB/s": round(g, 1), "frac": round(g / HBM_PEAK_GBS, 3),
-             "neighbour_counted_GB/s": round(2400 * V / (ms[0] * 1e-3) / 1e9, 1),
-             "traffic_per_launch": traffic.get("k_smear", {}).get("bytes_per_launch")}
+             "neighbour_counted_GB/s": round(2400 * V / (ms[0] * 1e-3) / 1e9, 1)}
     print(f"[bench] smear {smear}", file=sys.stderr, flush=True)
     m = 2048 * 32768
     _lib.check(L.qqcd_bench_lagfib(m, 10, 0, _lib.dp(ms)))
