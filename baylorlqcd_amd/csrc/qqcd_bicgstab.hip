@@ -28,9 +28,16 @@ struct BState {
   unsigned arrived[4];  // workgroups of each reduction that have left their partials
 };
 
+// a / b by R. L. Smith's algorithm (Comm. ACM 5 (1962) 435): |b|^2 is not
+// formed, which for rho (a squared norm) leaves the range of FP64 at sources
+// of 1e-75 or 1e+80
 __device__ __forceinline__ double2 cdiv(double2 a, double2 b) {
-  const double d = 1.0 / (b.x * b.x + b.y * b.y);
-  return make_double2((a.x * b.x + a.y * b.y) * d, (a.y * b.x - a.x * b.y) * d);
+  if (fabs(b.x) >= fabs(b.y)) {
+    const double r = b.y / b.x, d = b.x + b.y * r;
+    return make_double2((a.x + a.y * r) / d, (a.y - a.x * r) / d);
+  }
+  const double r = b.x / b.y, d = b.x * r + b.y;
+  return make_double2((a.x * r + a.y) / d, (a.y * r - a.x) / d);
 }
 __device__ __forceinline__ double2 cmulz(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);

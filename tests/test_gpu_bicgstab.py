@@ -77,3 +77,27 @@ def test_against_numpy(n, kap, tol, itermin, start):
     assert np.allclose(np.array([v[2] for v in log])[keep], h[keep], rtol=1e-3)
     scale = np.linalg.norm(want)
     assert np.linalg.norm(got - want) <= max(1e-8, 1e-2 * tol if tol < 1 else 1e-12) * max(scale, 1e-300)
+
+
+@pytest.mark.parametrize("scale", [1e-90, 1e-75, 1e80])
+def test_source_scale(scale):
+    """The recurrence is linear in the source: a source scaled by a power of ten far from 1, whose squared scalars
+    leave the range of FP64 while its norms do not, takes the same iterations to the scaled solution."""
+    n, kap, tol = (8, 8, 8, 16), (0.12, 0.01), 1e-9
+    lattice.init(n, BC)
+    try:
+        co = O.coact_array()
+        diracops.gauge_random(1, 0.3, 21, co)
+        u = diracops.gauge_get_ref(n)
+        diracops.gauge_load(u, co)
+        psi = np.random.default_rng(9).standard_normal(24 * int(np.prod(n))).view(complex).reshape(-1, 4, 3)
+        phi, _ = O.spinor_canon_to_ref(n, psi)
+        x1, xs = np.zeros_like(phi), np.zeros_like(phi)
+        it1 = inverters.bicgstab(None, phi, x1, tol, 0, u, None, -1, kap, co, BC)
+        its = inverters.bicgstab(None, scale * phi, xs, tol, 0, u, None, -1, kap, co, BC)
+    finally:
+        lattice.finalize()
+    # the scale is no power of two: both runs round differently and end within an iteration or two of each other
+    assert abs(its - it1) <= 2
+    # residuals below 1e-9 each, condition number below 1e2
+    assert np.linalg.norm(xs / scale - x1) < 2e-7 * np.linalg.norm(x1)
