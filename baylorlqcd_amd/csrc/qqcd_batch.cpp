@@ -425,21 +425,30 @@ void Batch::inner() {
     for (int s = 0; s < n_in; s++) {
       // the slot's (m+1) x m Hessenberg matrix, cut at the first breakdown
       double hmax = 0;
-      for (int j = 0; j < m; j++)
+      int jj = m;  // columns of it
+      for (int j = 0; j < m; j++) {
+        double cmax = 0;
         for (int q = 0; q <= j + 1; q++) {
           const size_t o = 2 * (((size_t)j * ldh + q) * cap + s);
           Hs[q + (size_t)ldh * j] = zd(hH[o], hH[o + 1]);
-          hmax = std::max(hmax, std::abs(Hs[q + (size_t)ldh * j]));
+          cmax = std::max(cmax, std::abs(Hs[q + (size_t)ldh * j]));
         }
-      int jj = m;
-      for (int j = 0; j < m; j++)
+        // blocks of four: the columns past the one that a block gave up on are zero
+        if (quads && j > 0 && cmax == 0.0) {
+          jj = j;
+          break;
+        }
+        hmax = std::max(hmax, cmax);
+      }
+      // (blocks of four decide the end themselves, and the norm that they leave in the last row counts)
+      for (int j = 0; j < jj && !quads; j++)
         if (std::abs(Hs[j + 1 + (size_t)ldh * j]) <= 1e-14 * hmax) {
           jj = j + 1;
           break;
         }
-      // back from B = A - sigma to A (a column that a block gave up is zero)
-      for (int j = 0; j < jj && sigma != 0.0; j++)
-        if (Hs[j + 1 + (size_t)ldh * j] != zd(0.0)) Hs[j + (size_t)ldh * j] += sigma;
+      // back from B = A - sigma to A
+      for (int j = 0; j < jj; j++) Hs[j + (size_t)ldh * j] += sigma;
+      hmax += sigma;
       std::fill(cs.begin(), cs.end(), zd(0.0));
       cs[0] = beta[s];
       std::fill(y.begin(), y.end(), zd(0.0));

@@ -19,14 +19,18 @@ __device__ __forceinline__ double2 zcmul(double2 a, double2 b) {  // conj(a) b
 // the update coefficients C = -P R^-1 and D = R^-1, and the columns j..j+S-1 of
 // H.  again: the vectors are the Q of this block, io.p1 / io.r1 the P and R of
 // the first pass; the total projections are P + P2 R and the total factor R2 R.
-// A vector is taken while more than `least` of its squared norm is left.
+// A vector is taken while more than `least` of its squared norm is left.  The
+// column of the first that is not is written all the same: A times the last
+// vector taken has all of it but that rest in the basis, whose norm is the
+// column's last entry though no vector stands for it.  The columns after it are
+// zero, and so are the new vectors from there on.
 template <int S, typename IO>
 __device__ __forceinline__ void block_columns(IO io, int j, int ld, int again, double least) {
   constexpr int NM = 128;
   __shared__ double2 P[NM][S], C[NM][S], G[S][S], R[S][S], D[S][S], Pt[NM][S], Rt[S][S], col[S][NM + S];
   __shared__ double red[2][S];
   __shared__ int good;
-  __shared__ double worst;
+  __shared__ double worst, left;
   const int t = threadIdx.x, nv = j + 1;
   for (int i = t; i < nv * S; i += 256) P[i / S][i % S] = io.p(i / S, i % S);
   for (int i = t; i < S * S; i += 256) G[i / S][i % S] = io.g(i / S, i % S);
@@ -52,7 +56,7 @@ __device__ __forceinline__ void block_columns(IO io, int j, int ld, int again, d
   if (t == 0) {
     // Cholesky R^H R of the upper triangle, in place; D = R^-1 (upper)
     double2 r[S][S], d[S][S];
-    double least_seen = 1.0;
+    double least_seen = 1.0, rest = 0.0;
     int n = 0;
 #pragma unroll
     for (int i = 0; i < S; i++)
@@ -70,6 +74,8 @@ __device__ __forceinline__ void block_columns(IO io, int j, int ld, int again, d
       const double g = G[i][i].x;
       ok = ok && p > least * g && p > 0;
       const double h = ok ? sqrt(p) : 0.0, inv = ok ? 1.0 / h : 0.0;
+      // what is left of the first vector that is not taken: the last row of its column of H
+      if (!ok && n == i) rest = p > 0 ? sqrt(p) : 0.0;
       if (ok) {
         least_seen = fmin(least_seen, p / g);
         n++;
@@ -105,6 +111,7 @@ __device__ __forceinline__ void block_columns(IO io, int j, int ld, int again, d
         D[i][k] = d[i][k];
       }
     good = n;
+    left = rest;
     worst = least_seen;
   }
   __syncthreads();
@@ -186,10 +193,11 @@ __device__ __forceinline__ void block_columns(IO io, int j, int ld, int again, d
     const int rows = j + i + 2;
     if (t < ld) {
       double2 h = make_double2(0, 0);
-      if (i < good && t < rows) {
+      if (i <= good && t < rows) {
         // coef(u_{i+1}), u_1 first
         if (t <= j) h = Pt[t][i];
-        else if (t - nv <= i) h = Rt[t - nv][i];
+        else if (t - nv < i || i < good) h = Rt[t - nv][i];
+        else h = make_double2(again ? left * io.r1(i, i).x : left, 0);
         if (i > 0) {
           // B q_i: less what u_i's other components contribute
           h = zsub(zsub(h, old[i]), zmul(Pt[j][i - 1], col[0][t]));
