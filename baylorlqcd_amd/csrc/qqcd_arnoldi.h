@@ -35,7 +35,8 @@ class BlockArnoldi {
   void queue(const Vec *V, int j, int s, int slot);
   // the same over an FP16 basis with per-site norms; the B^i V[j] are the FP32 U[0..s-1]
   void queue_half(const Vec *V, const Vec *U, int j, int s, int slot);
-  // the same vectors orthogonalised once more, the columns corrected
+  // the first s of the same block's vectors orthogonalised once more, the
+  // columns corrected
   void queue_again(const Vec *V, int j, int s, int slot);
   // after the stream has been waited for: columns j.. of H (of A) from block
   // `slot`; returns how many of the s steps are sound (a vector that lies in

@@ -140,13 +140,14 @@ template <int S> struct BlockIO {
   static constexpr int SM = BlockArnoldi::SMAX, NM = BlockArnoldi::NMAX;
   __device__ double2 p(int k, int c_) const { return sums[k * S + c_]; }
   __device__ double2 g(int r, int c_) const { return sums[(long)(g0 + r) * S + c_]; }
-  __device__ double2 p1(int k, int c_) const { return pr[k * S + c_]; }
-  __device__ double2 r1(int l, int c_) const { return pr[nv * S + l * S + c_]; }
+  // (rows of SM: a second pass may take fewer vectors than the first)
+  __device__ double2 p1(int k, int c_) const { return pr[k * SM + c_]; }
+  __device__ double2 r1(int l, int c_) const { return pr[(nv + l) * SM + c_]; }
   __device__ void coef(int k, int c_, double2 x, double2 pt) {
     const int i = k * S + c_;
     c[i] = x;
     c32[i] = make_float2((float)x.x, (float)x.y);
-    pr[i] = pt;
+    pr[k * SM + c_] = pt;
     // the update walks the vectors four at a time
     if (k == nv - 1)
       for (int q = nv; q < (nv + 3) / 4 * 4; q++) {
@@ -157,7 +158,7 @@ template <int S> struct BlockIO {
   __device__ void factor(int r, int c_, double2 d, double2 rt) {
     c[NM * SM + r * S + c_] = d;
     c32[NM * SM + r * S + c_] = make_float2((float)d.x, (float)d.y);
-    pr[nv * S + r * S + c_] = rt;
+    pr[(nv + r) * SM + c_] = rt;
   }
   __device__ double2 h(int row, int col) const { return hd[row + (long)ld * col]; }
   __device__ void put(int row, int col, int i, double2 x) {

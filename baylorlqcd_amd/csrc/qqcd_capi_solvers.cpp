@@ -146,6 +146,23 @@ extern "C" int qqcd_gmresdr(const double *phi, double *x, const int GMRES[2], do
   API_END
 }
 
+extern "C" int qqcd_arnoldi_check(const double *phi, int m, const double *u, const double *coact,
+                                  const double kappa[2], const int *bc, int *steps, double out[3]) {
+  API_BEGIN
+  Context &c = ctx();
+  prepare(c, u, coact, bc, -1);
+  SpinorBuf b(c.g, PREC_DOUBLE);
+  to_device(c, phi, b.s, 0);
+  SchurOp A(c, PREC_DOUBLE, 18, kappa);
+  LinOp op = A.op();
+  const ArnoldiCheck r = arnoldi_check(c, op, b.s, m);
+  *steps = r.steps;
+  out[0] = r.loss;
+  out[1] = r.bound;
+  out[2] = r.relation;
+  API_END
+}
+
 extern "C" int qqcd_gmresproject(const double *bh, double *xshift, int nshift, const int GMRES[2], double resmax,
                                  int itermin, int *itercount, const double *u, const double *coact,
                                  const double kappa[2], int iflag, const int *bc, int isignal, int *mvp, double *gdr,

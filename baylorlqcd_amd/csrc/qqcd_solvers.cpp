@@ -264,11 +264,13 @@ static void arnoldi_steps_dev(Context &c, LinOp &A, std::vector<Spinor> &V, int 
 // keep (FP64): `loss` bounds ||E||, E = V^H V - 1 (Frobenius).  A block adds
 // V^H Q = -E P R^-1 twice and the rounding of G over what the cancellation
 // left, which at ||P R^-1|| = 0.8 is a factor of 1.5 a block.  Where the bound
-// passes 1e-8, the square root of the rounding unit, below which H is the
+// passes kLoss, the square root of the rounding unit, below which H is the
 // projection of A to rounding all the same (H. D. Simon, Math. Comp. 42 (1984)
-// 115, semiorthogonality), the block is orthogonalised a second time; a
-// restart past 1e-10 takes the true value instead, which is near rounding.
-// A block whose first vector cancels to below 9 digits is done step by step.
+// 115, semiorthogonality), the block's sound vectors are orthogonalised a
+// second time; a restart past 1e-10 takes the true value instead, which is near
+// rounding.  A block whose first vector cancels to less than the least that is
+// taken (BlockArnoldi::run) is done step by step.
+static constexpr double kLoss = 1e-8;
 static int arnoldi_blocks(Context &c, LinOp &A, std::vector<Spinor> &V, int j, int want, BlockArnoldi &ba, bool keep,
                           double &loss, std::vector<zd> &H, int ldh, bool &ended,
                           const std::vector<std::unique_ptr<SpinorBuf>> &work) {
@@ -292,18 +294,18 @@ static int arnoldi_blocks(Context &c, LinOp &A, std::vector<Spinor> &V, int j, i
   int q = j;
   for (int b = 0; b < n; b++) {
     const int s = std::min(S, j + want - q);
-    const int good = ba.fetch(b, q, s, A.sigma, H.data(), ldh);
+    int good = ba.fetch(b, q, s, A.sigma, H.data(), ldh);
     const double g = ba.growth(b);
-    double after = std::hypot(loss * std::sqrt(1.0 + 2.0 * g * g), 1e-15 / ba.pivot(b));
-    if (keep && good == s && after > 1e-8) {
-      ba.queue_again(Vb.data(), q, s, b);
+    const double after = std::hypot(loss * std::sqrt(1.0 + 2.0 * g * g), 1e-15 / ba.pivot(b));
+    const bool twice = keep && good > 0 && after > kLoss;
+    if (twice) {
+      ba.queue_again(Vb.data(), q, good, b);
       QQCD_HIP(hipStreamSynchronize(c.stream));
-      if (ba.fetch(b, q, s, A.sigma, H.data(), ldh) != s) return q - j;
-      after = std::max(loss, 1e-14);
+      good = ba.fetch(b, q, good, A.sigma, H.data(), ldh);
     }
-    loss = after;
+    if (good > 0) loss = twice ? std::max(loss, 1e-14) : after;
     q += good;
-    if (good == s) continue;
+    if (good == s && !twice) continue;  // (a second pass moves the vectors that the blocks after it began from)
     if (q == j) {
       std::vector<zd> col(j + 2);
       ended = arnoldi_step(c, A, V, j, col.data(), keep, nullptr, nullptr, work.empty() ? nullptr : &work[0]->s) == 0.0;
@@ -476,6 +478,45 @@ static bool first_enough(const std::vector<zd> &H, int ldh, const std::vector<zd
     }
   }
   return done;
+}
+
+ArnoldiCheck arnoldi_check(Context &c, LinOp &A, const Spinor &b, int m) {
+  if (A.prec != PREC_DOUBLE || A.basis() != PREC_DOUBLE || m < 1 || !block_steps(A, m, 1, nullptr, nullptr))
+    throw std::runtime_error("arnoldi_check: FP64 blocks only");
+  std::vector<Spinor> V;
+  BasisGuard g{V};
+  alloc_basis(c, V, m + 1, PREC_DOUBLE);
+  BlockArnoldi ba(c.stream, m);
+  const int ldh = m + 1;
+  std::vector<zd> H((size_t)ldh * m, 0.0);
+  const double bn = std::sqrt(c.blas->norm2(vv(b)));
+  if (bn == 0.0) throw std::runtime_error("arnoldi_check: zero vector");
+  scaled_copy(c, b, V[0], 1.0 / bn);
+  ArnoldiCheck r;
+  int j = 0;
+  bool ended = false;
+  while (j < m && !ended) {
+    const int got = arnoldi_blocks(c, A, V, j, std::min(kCheck, m - j), ba, true, r.bound, H, ldh, ended, {});
+    if (got < 1) throw std::runtime_error("arnoldi_check: no step made");
+    j += got;
+    // a last vector of rounding: the space has ended, as a solve's residual has there
+    double n2 = 0;
+    for (int i = 0; i <= j; i++) n2 += std::norm(H[i + (size_t)ldh * (j - 1)]);
+    ended = ended || std::abs(H[j + (size_t)ldh * (j - 1)]) <= 1e-13 * std::sqrt(n2);
+  }
+  r.steps = j;
+  r.loss = ba.loss_of(vecs(V, j).data(), j);
+  SpinorBuf w(c.g, PREC_DOUBLE);
+  Vec wv = vv(w.s);
+  double e = 0, h = 0;
+  for (int q = 0; q < j; q++) {
+    A.apply(V[q], w.s);
+    // the last vector may be rounding where the space ended: its column's last entry is too
+    e += c.blas->multi_axpy(q + 2, &H[(size_t)ldh * q], vecs(V, q + 2).data(), wv, true);
+    for (int i = 0; i <= q + 1; i++) h += std::norm(H[i + (size_t)ldh * q]);
+  }
+  r.relation = std::sqrt(e / h);
+  return r;
 }
 
 SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int k, double tol, int itermin,

@@ -141,6 +141,15 @@ typedef std::function<void(int iters, double rnorm, double r0)> IterHook;
 SolveStats bicgstab(Context &c, LinOp &A, const Spinor &b, Spinor &x, double tol, int itermin, int maxiter,
                     const IterHook *hook = nullptr);
 
+// n <= m Arnoldi steps from b as gmresdr makes them (verification hook; FP64)
+struct ArnoldiCheck {
+  int steps = 0;         // n: fewer than m where the Krylov space ended
+  double loss = 0;       // ||V^H V - 1||, Frobenius, of the n vectors
+  double bound = 0;      // what the steps took it for
+  double relation = 0;   // ||A V_n - V_{n+1} H|| / ||H||, Frobenius
+};
+ArnoldiCheck arnoldi_check(Context &c, LinOp &A, const Spinor &b, int m);
+
 // out = a0 in + a1 (i g5) in, FP64, on one checkerboard
 void local_spin(const Geom &g, const Spinor &in, Spinor &out, double a0, double a1, hipStream_t s);
 

@@ -658,6 +658,13 @@ int qqcd_dense_lsq(int rows, int cols, const double *h, int ldh, const double *c
  * H_m + |h_{m+1,m}|^2 H_m^{-H} e_m e_m^T for the k values of smallest modulus */
 int qqcd_dense_harmonic_ritz(int m, const double *hbar, int ldh, int k, double *p, double *theta);
 
+/* ---- the block Arnoldi steps (verification hook) -------------------------
+ * Up to m steps over an FP64 basis from phi (even checkerboard, arguments as
+ * qqcd_gmresdr's): steps made, and out = { ||V^H V - 1||, the bound that the
+ * solver kept for it, ||A V - V H|| / ||H|| }, Frobenius norms. */
+int qqcd_arnoldi_check(const double *phi, int m, const double *u, const double *coact, const double kappa[2],
+                       const int *bc, int *steps, double out[3]);
+
 #ifdef __cplusplus
 }
 #endif

@@ -154,3 +154,48 @@ def test_mixed_low_basis(basis, prec, recon, n, gm):
     assert blk[0] <= 1.15 * one[0] + 8, (one[0], blk[0])
     if (basis, prec) != (2, 1):
         assert blk[0] >= 0.85 * one[0] - 8, (one[0], blk[0])
+
+
+def check_basis(phi, m, u, co, kap, bc):
+    steps, out = np.zeros(1, np.int32), np.zeros(3)
+    _lib.check(_lib.lib().qqcd_arnoldi_check(_lib.dp(phi), m, _lib.dp(u), _lib.dp(np.asarray(co).ravel(order="F")),
+                                             _lib.dp(np.array(kap)), _lib.ints(bc).ctypes.data_as(_lib._ip),
+                                             steps.ctypes.data_as(_lib._ip), _lib.dp(out)))
+    return int(steps[0]), *out
+
+
+@pytest.mark.parametrize("m", [6, 23])
+@pytest.mark.parametrize("eps", [0.0, 1e-9, 1e-7, 1e-6, 1e-5, 3e-5, 5e-5, 1e-4, 3e-4, 1e-3, 1e-2, 1.0])
+def test_near_invariant_basis(m, eps):
+    """An eigenvector with a little noise: the first block's vectors cancel against it to any number of digits, so
+    that none, some or all of them are taken.  The basis stays orthogonal and the Arnoldi relation holds."""
+    n, bc, kap = (8, 4, 4, 8), (1, 1, 1, 1), (0.11, 0.0)
+    U, u, co = setup(n, kind=1, eps=0.0, bc=bc)
+    try:
+        even = ~O.parity_mask(n)
+        const = np.zeros((int(np.prod(n)), 4, 3), complex)
+        const[even] = np.arange(1, 13).reshape(4, 3)
+        noise, _ = rhs(n, 8)
+        psi = const + eps * noise * np.linalg.norm(const) / np.linalg.norm(noise)
+        phi, _ = O.spinor_canon_to_ref(n, psi)
+        steps, loss, bound, rel = check_basis(phi, m, u, co, kap, bc)
+    finally:
+        lattice.finalize()
+    print(f"[arnoldi] near invariant {m} {eps}: {steps} steps, loss {loss:.2e} <= {bound:.2e}, relation {rel:.2e}",
+          flush=True)
+    # the bound that the solver keeps, and what it says of the basis; the relation to the rounding of vectors that
+    # cancelled to the least that is taken (1e-9 of the squared norm)
+    assert loss <= bound <= 1e-8
+    assert rel < 1e-15 / 3e-5 * 10
+
+
+@pytest.mark.parametrize("n,m", [((4, 4, 4, 4), 11), ((8, 8, 8, 16), 40), ((12, 4, 8, 4), 61), ((8, 8, 8, 16), 120)])
+def test_basis(n, m):
+    U, u, co = setup(n)
+    try:
+        psi, phi = rhs(n, 9)
+        steps, loss, bound, rel = check_basis(phi, m, u, co, (0.125, 0.01), BC)
+    finally:
+        lattice.finalize()
+    print(f"[arnoldi] basis {n} {m}: {steps} steps, loss {loss:.2e} <= {bound:.2e}, relation {rel:.2e}", flush=True)
+    assert steps == m and loss <= bound <= 1e-8 and rel < 1e-13
