@@ -39,8 +39,9 @@ class BlockArnoldi {
   // columns corrected
   void queue_again(const Vec *V, int j, int s, int slot);
   // after the stream has been waited for: columns j.. of H (of A) from block
-  // `slot`; returns how many of the s steps are sound (a vector that lies in
-  // the span of the ones before it to 9 digits ends the block)
+  // `slot`; returns how many of the s steps are sound (a vector of whose squared
+  // norm the span of the ones before it leaves less than 1e-6 -- FP32 basis:
+  // 1e-10 -- ends the block)
   int fetch(int slot, int j, int s, double sigma, std::complex<double> *H, int ldh) const;
   // ||V^H V - 1|| (Frobenius) of n FP64 vectors
   double loss_of(const Vec *V, int n);

@@ -476,10 +476,10 @@ void BlockArnoldi::run(const Vec *V, int j, int s, int slot, bool again) {
       constexpr int S = decltype(SS)::value;
       hipLaunchKernelGGL((k_bdot<T, S>), dim3(gx, ny), dim3(64 * w), 0, stream, nu, tab, nleft, part);
       hipLaunchKernelGGL(k_bsum, dim3(chunks), dim3(1024), 0, stream, gx, 2 * KV * S, part, sums);
-      // a vector is taken while at least 1e-9 (FP64; FP32: 1e-10, its rounding squared being 4e-15) of its
-      // squared norm is left
+      // a vector is taken while at least 1e-6 (FP64: the Arnoldi relation then holds to 1e-13, the rounding over the
+      // square root of this; FP32: 1e-10, its rounding squared being 4e-15) of its squared norm is left
       hipLaunchKernelGGL((k_bcols<S>), dim3(1), dim3(256), 0, stream, j, ld, again ? 1 : 0, j + 1,
-                         sizeof(T) == 8 ? 1e-9 : 1e-10, (const double2 *)sums, (double2 *)hd, (double2 *)pr,
+                         sizeof(T) == 8 ? 1e-6 : 1e-10, (const double2 *)sums, (double2 *)hd, (double2 *)pr,
                          (double2 *)coef, (float2 *)coef32, (double2 *)slot_h, slot_h + 2L * SMAX * ld);
       hipLaunchKernelGGL((k_bupdate<T, S>), dim3(gu), dim3(UB), 0, stream, nu, tab, j + 1, coef);
     });

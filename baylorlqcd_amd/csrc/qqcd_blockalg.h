@@ -30,7 +30,7 @@ __device__ __forceinline__ void block_columns(IO io, int j, int ld, int again, d
   __shared__ double2 P[NM][S], C[NM][S], G[S][S], R[S][S], D[S][S], Pt[NM][S], Rt[S][S], col[S][NM + S];
   __shared__ double red[2][S];
   __shared__ int good;
-  __shared__ double worst, left;
+  __shared__ double worst;
   const int t = threadIdx.x, nv = j + 1;
   for (int i = t; i < nv * S; i += 256) P[i / S][i % S] = io.p(i / S, i % S);
   for (int i = t; i < S * S; i += 256) G[i / S][i % S] = io.g(i / S, i % S);
@@ -56,7 +56,7 @@ __device__ __forceinline__ void block_columns(IO io, int j, int ld, int again, d
   if (t == 0) {
     // Cholesky R^H R of the upper triangle, in place; D = R^-1 (upper)
     double2 r[S][S], d[S][S];
-    double least_seen = 1.0, rest = 0.0;
+    double least_seen = 1.0;
     int n = 0;
 #pragma unroll
     for (int i = 0; i < S; i++)
@@ -74,13 +74,13 @@ __device__ __forceinline__ void block_columns(IO io, int j, int ld, int again, d
       const double g = G[i][i].x;
       ok = ok && p > least * g && p > 0;
       const double h = ok ? sqrt(p) : 0.0, inv = ok ? 1.0 / h : 0.0;
-      // what is left of the first vector that is not taken: the last row of its column of H
-      if (!ok && n == i) rest = p > 0 ? sqrt(p) : 0.0;
+      r[i][i] = make_double2(h, 0);
       if (ok) {
         least_seen = fmin(least_seen, p / g);
         n++;
+      } else if (n == i && p > 0) {
+        r[i][i].x = sqrt(p);  // of the first not taken: the last row of its column of H
       }
-      r[i][i] = make_double2(h, 0);
 #pragma unroll
       for (int k = i + 1; k < S; k++) {
         double2 x = r[i][k];
@@ -111,7 +111,6 @@ __device__ __forceinline__ void block_columns(IO io, int j, int ld, int again, d
         D[i][k] = d[i][k];
       }
     good = n;
-    left = rest;
     worst = least_seen;
   }
   __syncthreads();
@@ -196,8 +195,7 @@ __device__ __forceinline__ void block_columns(IO io, int j, int ld, int again, d
       if (i <= good && t < rows) {
         // coef(u_{i+1}), u_1 first
         if (t <= j) h = Pt[t][i];
-        else if (t - nv < i || i < good) h = Rt[t - nv][i];
-        else h = make_double2(again ? left * io.r1(i, i).x : left, 0);
+        else if (t - nv <= i) h = Rt[t - nv][i];
         if (i > 0) {
           // B q_i: less what u_i's other components contribute
           h = zsub(zsub(h, old[i]), zmul(Pt[j][i - 1], col[0][t]));

@@ -261,16 +261,19 @@ static void arnoldi_steps_dev(Context &c, LinOp &A, std::vector<Spinor> &V, int 
 // 188 ms in blocks; 16^3x32 GMRES-DR(60,20) and GMRES-Proj(40): 279 -> 89 ms;
 // 16^3x32 FP32 mixed solve: 56.5 ms, 38.9 (blocks of two), 37.6 (four).
 //
-// keep (FP64): `loss` bounds ||E||, E = V^H V - 1 (Frobenius).  A block adds
-// V^H Q = -E P R^-1 twice and the rounding of G over what the cancellation
-// left, which at ||P R^-1|| = 0.8 is a factor of 1.5 a block.  Where the bound
-// passes kLoss, the square root of the rounding unit, below which H is the
-// projection of A to rounding all the same (H. D. Simon, Math. Comp. 42 (1984)
-// 115, semiorthogonality), the block's sound vectors are orthogonalised a
-// second time; a restart past 1e-10 takes the true value instead, which is near
-// rounding.  A block whose first vector cancels to less than the least that is
-// taken (BlockArnoldi::run) is done step by step.
-static constexpr double kLoss = 1e-8;
+// keep (FP64): E = V^H V - 1 stays near rounding (Frobenius norm at most 5e-13
+// over GMRES-DR(40,10) on 12x8x20x28, (40,16) on 24^3x48 and (60,20) on
+// 16^3x32).  A block adds V^H Q = -E P R^-1 twice and the rounding of G over what
+// the cancellation left, R_ii^2 / G_ii.  Ordinary blocks have ||P R^-1|| = 0.67
+// and 0.076, the first one after a restart up to 6 and down to 0.0026: a block
+// past 8 or below 1e-3 is orthogonalised a second time, its sound vectors if not
+// all are.  `loss` is the bound on ||E|| that follows, a factor of 1.4 a block:
+// where it passes kLoss, the square root of the rounding unit, below which H is
+// the projection of A to rounding all the same (H. D. Simon, Math. Comp. 42
+// (1984) 115, semiorthogonality), the second pass runs too; a restart past
+// kLossRestart takes the true value instead.  A block whose first vector cancels
+// to less than the least that is taken (BlockArnoldi::run) is done step by step.
+static constexpr double kLoss = 1e-8, kLossRestart = 1e-10, kGrowth = 8.0, kPivot = 1e-3;
 static int arnoldi_blocks(Context &c, LinOp &A, std::vector<Spinor> &V, int j, int want, BlockArnoldi &ba, bool keep,
                           double &loss, std::vector<zd> &H, int ldh, bool &ended,
                           const std::vector<std::unique_ptr<SpinorBuf>> &work) {
@@ -297,7 +300,7 @@ static int arnoldi_blocks(Context &c, LinOp &A, std::vector<Spinor> &V, int j, i
     int good = ba.fetch(b, q, s, A.sigma, H.data(), ldh);
     const double g = ba.growth(b);
     const double after = std::hypot(loss * std::sqrt(1.0 + 2.0 * g * g), 1e-15 / ba.pivot(b));
-    const bool twice = keep && good > 0 && after > kLoss;
+    const bool twice = keep && good > 0 && (g > kGrowth || ba.pivot(b) < kPivot || after > kLoss);
     if (twice) {
       ba.queue_again(Vb.data(), q, good, b);
       QQCD_HIP(hipStreamSynchronize(c.stream));
@@ -657,7 +660,7 @@ SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int 
       restarted = true;
       if (ba) {
         ba->load(Hnew.data(), k + 1, k, A.sigma);
-        if (reorth && loss > 1e-10) loss = ba->loss_of(vecs(V, k + 1).data(), k + 1);
+        if (reorth && loss > kLossRestart) loss = ba->loss_of(vecs(V, k + 1).data(), k + 1);
       }
     } else {
       // plain restart from the true residual
