@@ -35,6 +35,8 @@ class BlockArnoldi {
   void queue(const Vec *V, int j, int s, int slot);
   // the same over an FP16 basis with per-site norms; the B^i V[j] are the FP32 U[0..s-1]
   void queue_half(const Vec *V, const Vec *U, int j, int s, int slot);
+  // waits; the sums of the queue_half before: rows <V_q, u_c> of nv vectors, then <u_r, u_c>
+  void half_sums(int nv, int s, std::complex<double> *out) const;
   // the first s of the same block's vectors orthogonalised once more, the
   // columns corrected
   void queue_again(const Vec *V, int j, int s, int slot);

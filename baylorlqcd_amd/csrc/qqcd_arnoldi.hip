@@ -246,13 +246,15 @@ __device__ __forceinline__ void ld4(const void *p, long i, float2 (&e)[4]) {
 // k_bdot for an FP16 basis: the chunks of KV basis vectors, and after them one
 // of the u_c themselves (G).  A lane takes four consecutive sites and walks
 // their 12 component runs (nq = stride / 4 site quads), so each vector's norms
-// are read once; 16 bytes of a vector a lane.  Sums in FP32 within a lane (the
-// basis carries 11 bits), in FP64 across lanes.
+// are read once; 16 bytes of a vector a lane.  Sums in FP32 over the 48 products
+// of a lane's quad (the basis carries 11 bits), in FP64 beyond.
 template <int S>
 __global__ void __launch_bounds__(64 * DW) k_bdot_h(long nq, VTab v, NTab vn, UTab ut, int nv, double *part) {
   const int lane = threadIdx.x & 63, cv = (nv + KV - 1) / KV;
   const int chunk = __builtin_amdgcn_readfirstlane(blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6));
   if (chunk > cv) return;
+  constexpr int HV = S % 4 == 0 ? 5 : S % 2 == 0 ? 4 : 3;  // 2 KV S is a multiple of 2^HV
+  Runs<2 * KV * S, HV> runs;
   float af[2 * KV * S];
 #pragma unroll
   for (int k = 0; k < 2 * KV * S; k++) af[k] = 0.f;
@@ -270,7 +272,8 @@ __global__ void __launch_bounds__(64 * DW) k_bdot_h(long nq, VTab v, NTab vn, UT
     const void *pv[KV];
 #pragma unroll
     for (int k = 0; k < KV; k++) pv[k] = v.p[k0 + k < nv ? k0 + k : nv - 1];
-    for (long q = blockIdx.x * 64L + lane; q < nq; q += gridDim.x * 64L) {
+    for (long q0 = blockIdx.x * 64L; q0 < nq; q0 += gridDim.x * 64L) {
+      const long q = q0 + lane < nq ? q0 + lane : nq - 1;  // lanes past the end repeat the last quad for nothing
       float4 m[KV], ub[2 * S];
       h8v vb[KV];
       auto fetch = [&](long i) {
@@ -284,7 +287,10 @@ __global__ void __launch_bounds__(64 * DW) k_bdot_h(long nq, VTab v, NTab vn, UT
       };
       fetch(q);
 #pragma unroll
-      for (int k = 0; k < KV; k++) m[k] = *(const float4 *)(vn.n[k0 + k < nv ? k0 + k : nv - 1] + 4 * q);
+      for (int k = 0; k < KV; k++) {
+        m[k] = *(const float4 *)(vn.n[k0 + k < nv ? k0 + k : nv - 1] + 4 * q);
+        if (q0 + lane >= nq) m[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
       for (int r = 0; r < 12; r++) {
         float2 b[S][4];
         h8v vc[KV];
@@ -308,26 +314,31 @@ __global__ void __launch_bounds__(64 * DW) k_bdot_h(long nq, VTab v, NTab vn, UT
           add(e, b, k);
         }
       }
+      runs.add(af, lane);
     }
   } else {
-    for (long q = blockIdx.x * 64L + lane; q < nq; q += gridDim.x * 64L)
-      for (int r = 0; r < 12; r++) {
+    for (long q0 = blockIdx.x * 64L; q0 < nq; q0 += gridDim.x * 64L) {
+      const long q = q0 + lane;
+      for (int r = 0; r < 12 && q < nq; r++) {
         float2 b[S][4];
 #pragma unroll
         for (int c = 0; c < S; c++) ld4(ut.p[c], r * nq + q, b[c]);
 #pragma unroll
         for (int k = 0; k < S; k++) add(b[k], b, k);
       }
+      runs.add(af, lane);
+    }
   }
-  double mine = 0;
+  // a lane is left with M totals (2 KV S / 32 where that is whole), over the lanes of its lower bits
+  constexpr int M = decltype(runs)::M;
 #pragma unroll
-  for (int k = 0; k < 2 * KV * S; k++) {
-    double s = (double)af[k];
+  for (int q = 0; q < M; q++) {
+    double s = runs.tot[q];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (lane == k) mine = s;
+    for (int o = (64 >> HV) / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((lane & ((64 >> HV) - 1)) == 0)
+      part[((long)chunk * gridDim.x + blockIdx.x) * (2 * KV * S) + runs.first(lane) + q] = s;
   }
-  if (lane < 2 * KV * S) part[((long)chunk * gridDim.x + blockIdx.x) * (2 * KV * S) + lane] = mine;
 }
 
 // k_bupdate for an FP16 basis, one lane per site: the S new vectors of a site
@@ -521,6 +532,14 @@ void BlockArnoldi::queue_half(const Vec *V, const Vec *U, int j, int s, int slot
                        ut, nv, coef32);
   });
   QQCD_HIP(hipGetLastError());
+}
+
+void BlockArnoldi::half_sums(int nv, int s, zd *out) const {
+  const int cv = (nv + KV - 1) / KV;
+  QQCD_HIP(hipMemcpyAsync(out, sums, sizeof(zd) * nv * s, hipMemcpyDeviceToHost, stream));
+  QQCD_HIP(hipMemcpyAsync(out + (size_t)nv * s, sums + 2L * cv * KV * s, sizeof(zd) * s * s, hipMemcpyDeviceToHost,
+                          stream));
+  QQCD_HIP(hipStreamSynchronize(stream));
 }
 
 void BlockArnoldi::queue(const Vec *V, int j, int s, int slot) { run(V, j, s, slot, false); }

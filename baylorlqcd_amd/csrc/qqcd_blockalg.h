@@ -14,6 +14,91 @@ __device__ __forceinline__ double2 zcmul(double2 a, double2 b) {  // conj(a) b
   return make_double2(a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x);
 }
 
+// a of the lanes whose bit is clear and b of those whose bit is set stay; the
+// other halves change places: afterwards a + b is, in a lane, the sum of a (bit
+// clear) or of b (bit set) over the lane and the one that differs in the bit.
+template <int BIT> __device__ __forceinline__ void swap_halves(unsigned &a, unsigned &b, int lane) {
+  if constexpr (BIT >= 16) {
+    const auto r = BIT == 32 ? __builtin_amdgcn_permlane32_swap(a, b, false, false)
+                             : __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+  } else {
+    const bool hi = lane & BIT;
+    const unsigned got = __shfl_xor(hi ? a : b, BIT, 64);
+    a = hi ? got : a;
+    b = hi ? b : got;
+  }
+}
+template <int BIT> __device__ __forceinline__ void swap_halves(float &a, float &b, int lane) {
+  unsigned x = __float_as_uint(a), y = __float_as_uint(b);
+  swap_halves<BIT>(x, y, lane);
+  a = __uint_as_float(x);
+  b = __uint_as_float(y);
+}
+template <int BIT> __device__ __forceinline__ void swap_halves(double &a, double &b, int lane) {
+  unsigned x0 = __double2loint(a), x1 = __double2hiint(a), y0 = __double2loint(b), y1 = __double2hiint(b);
+  swap_halves<BIT>(x0, y0, lane);
+  swap_halves<BIT>(x1, y1, lane);
+  a = __hiloint2double(x1, x0);
+  b = __hiloint2double(y1, y0);
+}
+
+// FP32 sums of a run of products, kept in FP64 across runs.  A wavefront's lanes
+// hold N sums each; the H halvings below add them (in FP64) over the lanes that
+// differ in their H highest bits and leave a lane with N >> H of them: those from
+// `first` on.  About N lane swaps, and 2 (N >> H) registers between runs instead
+// of 2 N.
+template <int N, int H> struct Runs {
+  static_assert(N % (1 << H) == 0, "halvings");
+  static constexpr int M = N >> H;
+  double tot[M];
+  __device__ Runs() {
+#pragma unroll
+    for (int k = 0; k < M; k++) tot[k] = 0;
+  }
+  // adds af and clears it
+  __device__ __forceinline__ void add(float (&af)[N], int lane) {
+    if constexpr (H == 0) {
+#pragma unroll
+      for (int k = 0; k < N; k++) tot[k] += (double)af[k];
+    } else {
+      double d[N / 2];
+#pragma unroll
+      for (int k = 0; k < N / 2; k++) {
+        swap_halves<32>(af[k], af[k + N / 2], lane);
+        d[k] = (double)af[k] + (double)af[k + N / 2];
+      }
+      halve<1>(d, lane);
+    }
+#pragma unroll
+    for (int k = 0; k < N; k++) af[k] = 0.f;
+  }
+  static __device__ __forceinline__ int first(int lane) {
+    int f = 0;
+#pragma unroll
+    for (int h = 0; h < H; h++)
+      if (lane & (32 >> h)) f += N >> (h + 1);
+    return f;
+  }
+
+ private:
+  template <int D, int C> __device__ __forceinline__ void halve(double (&d)[C], int lane) {
+    if constexpr (D == H) {
+#pragma unroll
+      for (int k = 0; k < C; k++) tot[k] += d[k];
+    } else {
+      double e[C / 2];
+#pragma unroll
+      for (int k = 0; k < C / 2; k++) {
+        swap_halves<(32 >> D)>(d[k], d[k + C / 2], lane);
+        e[k] = d[k] + d[k + C / 2];
+      }
+      halve<D + 1>(e, lane);
+    }
+  }
+};
+
 // One workgroup of 256 threads per right-hand side, a basis of at most 128
 // vectors (j + S < ld <= 128): from the sums P (rows 0..j) and G the factor R,
 // the update coefficients C = -P R^-1 and D = R^-1, and the columns j..j+S-1 of

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../../include/qqcd_hip.h"
+#include "qqcd_arnoldi.h"
 #include "qqcd_batch.h"
 #include "qqcd_solvers.h"
 #include "qqcd_loops.h"
@@ -113,6 +114,69 @@ void multi_canonical(int which, int nrhs, int nact, int nb, int prec, int recon,
   pool_free(d_n);
 }
 
+// sums of the block Arnoldi pass of dots over constant fields: nq FP16 basis
+// vectors of re[0], s FP32 vectors of re[1..s]; nrhs 0: the single-RHS pass
+void block_dots(int nrhs, int nb, int nq, int s, const double *re, double *sums) {
+  Context &c = ctx();
+  if (nrhs < 0 || nrhs > 256 || nq < 1 || s < 1 || s > 4 || nq + s > 127) throw std::runtime_error("bad block of vectors");
+  const int ld = nq + s;
+  SpinorBuf f(c.g, PREC_DOUBLE);
+  if (nrhs == 0) {
+    std::vector<std::unique_ptr<SpinorBuf>> V, U;
+    std::vector<Vec> v, u;
+    for (int q = 0; q < ld; q++) {
+      const bool basis = q < nq;
+      V.emplace_back(new SpinorBuf(c.g, PREC_HALF));
+      fill_spinor(c.g, f.s, re[0], 0.0, c.stream);
+      if (basis) spinor_copy_convert(c.g, f.s, V.back()->s, c.stream);
+      v.push_back(as_vec(V.back()->s));
+    }
+    for (int i = 0; i < s; i++) {
+      U.emplace_back(new SpinorBuf(c.g, PREC_SINGLE));
+      fill_spinor(c.g, f.s, re[1 + i], 0.0, c.stream);
+      spinor_copy_convert(c.g, f.s, U.back()->s, c.stream);
+      u.push_back(as_vec(U.back()->s));
+    }
+    BlockArnoldi ba(c.stream, ld);
+    ba.queue_half(v.data(), u.data(), nq - 1, s, 0);
+    ba.half_sums(nq, s, (std::complex<double> *)sums);
+    return;
+  }
+  nb = check_nb(nb, nrhs);
+  std::vector<std::unique_ptr<MultiBuf>> V, U;
+  std::vector<MultiSpinor> v;
+  std::vector<MultiSpinor *> u;
+  MultiBuf X(c.g, PREC_SINGLE, nrhs, nb), R(c.g, PREC_SINGLE, nrhs, nb);
+  MBlas mb(c.stream, nrhs);
+  DevArr n2(nullptr, nrhs, c.stream), H(nullptr, (size_t)2 * ld * ld * nrhs, c.stream),
+      ds(nullptr, (size_t)2 * s * ld * nrhs, c.stream), cf(nullptr, (size_t)s * ld * nrhs, c.stream),
+      dn(nullptr, 1, c.stream);
+  int *d_n = (int *)dn.p;
+  QQCD_HIP(hipMemcpyAsync(d_n, &nrhs, sizeof(int), hipMemcpyHostToDevice, c.stream));
+  auto fill = [&](MultiSpinor &m, double x) {
+    fill_spinor(c.g, f.s, x, 0.0, c.stream);
+    for (int r = 0; r < nrhs; r++) mb.put(f.s, m, r);
+  };
+  fill(X.m, re[0]);
+  mb.norm2(X.m, d_n, n2.p);
+  for (int q = 0; q < ld; q++) {
+    V.emplace_back(new MultiBuf(c.g, PREC_HALF, nrhs, nb, false));
+    v.push_back(V.back()->m);
+    if (q < nq) mb.scale_inv_norm2(X.m, R.m, v[q], n2.p, d_n);
+  }
+  for (int i = 0; i < s; i++) {
+    U.emplace_back(new MultiBuf(c.g, PREC_SINGLE, nrhs, nb));
+    fill(U.back()->m, re[1 + i]);
+    u.push_back(&U.back()->m);
+  }
+  mb.block(nq - 1, s, v.data(), u.data(), R.m, H.p, ld, ds.p, (float *)cf.p, d_n);
+  std::vector<double> h((size_t)2 * s * ld * nrhs);
+  QQCD_HIP(hipMemcpyAsync(h.data(), ds.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+  QQCD_HIP(hipStreamSynchronize(c.stream));
+  for (size_t i = 0; i < (size_t)s * ld; i++)
+    for (int x = 0; x < 2; x++) sums[2 * i + x] = h[2 * (i * nrhs + nrhs - 1) + x];
+}
+
 BatchParams batch_params(const int GMRES[2], double tol, int nb_rhs) {
   BatchParams p = g_bp;
   p.m = GMRES[0] - GMRES[1];
@@ -122,6 +186,12 @@ BatchParams batch_params(const int GMRES[2], double tol, int nb_rhs) {
 }
 
 }  // namespace
+
+extern "C" int qqcd_block_dots(int nrhs, int nb, int nq, int s, const double *re, double *sums) {
+  API_BEGIN
+  block_dots(nrhs, nb, nq, s, re, sums);
+  API_END
+}
 
 extern "C" int qqcd_z4source(double *be, double *bo, unsigned long long seed, long rhs, double scale) {
   API_BEGIN

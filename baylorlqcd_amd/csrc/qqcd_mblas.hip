@@ -566,6 +566,7 @@ __global__ void k_set_subdiag(double *H, int ldh, int j, const double *n2, const
 // ---- blocks of up to four Arnoldi steps (FP16 basis V, FP32 u_c = B^c v_j) ----
 
 static constexpr int BQ = 6;     // basis fields of a wavefront in the pass of dots
+static constexpr int BRUN = 32;  // elements of a lane summed in FP32 at most
 static constexpr int BWV = 8;    // its wavefronts at most: 7 BQ fields and the u_c
 static constexpr int BCH = (BWV - 1) * BQ;  // basis fields of one launch of the pass
 struct BTab {
@@ -579,12 +580,13 @@ struct BUTab {
 // <u_q, u_c>.
 //
 // Bound by reading the basis: the wavefronts of a workgroup take BQ fields each (the last one the u_c) of the same
-// 64 elements, so the u_c come from memory once and from the L1 for the other wavefronts.  Sums in FP32 within a lane
-// (the basis carries 11 bits), in FP64 across lanes; two elements are in flight, one is worked on.  16^3x32, 23
-// sources, 1..37 basis vectors: 591 us a block of four with 6 fields a wavefront, 631 with 8 (141 registers), 606
-// with 4; with the update below 1.23 ms for four steps, where two pairs of steps took about 1.5.
-template <int S>
-__global__ void __launch_bounds__(64 * BWV) k_mbdot(MShape a, BTab v, BUTab ut, int q0, int nq, double *part) {
+// 64 elements, so the u_c come from memory once and from the L1 for the other wavefronts.  Sums in FP32 over runs of
+// `most` elements of a lane (the basis carries 11 bits), in FP64 beyond; two elements are in flight, one is worked on.
+// 16^3x32, 23 sources, 1..37 basis vectors: 586 us a block of four (578 with all of a lane's 290 elements in FP32);
+// 6 fields a wavefront against 8 (141 registers) and 4, in FP32 throughout: 591, 631, 606; with the update below
+// 1.22 ms for four steps, where two pairs of steps took about 1.5.
+template <int S, int HV>
+__global__ void __launch_bounds__(64 * BWV) k_mbdot(MShape a, BTab v, BUTab ut, int q0, int nq, int most, double *part) {
   const int nact = *a.nact, nb = 1 << a.lognb, blk = blockIdx.y;
   if ((blk << a.lognb) >= nact) return;
   const int lane = threadIdx.x & 63, rr = lane & (nb - 1), slot = (blk << a.lognb) + rr;
@@ -593,6 +595,7 @@ __global__ void __launch_bounds__(64 * BWV) k_mbdot(MShape a, BTab v, BUTab ut, 
   typedef typename E2<f16>::raw h2;
   // the 64 elements of a wavefront are consecutive: a uniform address and the lane (12 stride is a multiple of 64)
   const long base = (long)blk * a.blk_elems, groups = a.rows >> (6 - a.lognb);
+  Runs<2 * BQ * S, HV> runs;
   float af[2 * BQ * S];
 #pragma unroll
   for (int k = 0; k < 2 * BQ * S; k++) af[k] = 0.f;
@@ -604,65 +607,72 @@ __global__ void __launch_bounds__(64 * BWV) k_mbdot(MShape a, BTab v, BUTab ut, 
       im = fmaf(-y, u[c][0], fmaf(x, u[c][1], im));
     }
   };
+  // two elements in flight, one worked on; every `most` of them (even) into FP64
+  auto walk = [&](auto &&fetch, auto &&work) {
+    long g = blockIdx.x;
+    const long st = a.gx;
+    fetch(0, g);
+    for (int run = 0; g + 2 * st < groups; g += 2 * st) {
+      fetch(1, g + st);
+      work(0);
+      fetch(0, g + 2 * st);
+      work(1);
+      if ((run += 2) == most) {
+        runs.add(af, lane);
+        run = 0;
+      }
+    }
+    if (g + st < groups) {
+      fetch(1, g + st);
+      work(0);
+      work(1);
+    } else {
+      work(0);
+    }
+    runs.add(af, lane);
+  };
+  const f2 *up[S];
+#pragma unroll
+  for (int c = 0; c < S; c++) up[c] = (const f2 *)ut.p[c] + base;
+  const unsigned l4 = lane * 4u;
+  f2 u[2][S];
+  auto fetch_u = [&](int h, long g) {
+#pragma unroll
+    for (int c = 0; c < S; c++) u[h][c] = *(const f2 *)((const char *)(up[c] + g * 64) + 2 * l4);
+  };
   int left = S;
   if (wv < nw) {
     left = nq - k0 < BQ ? nq - k0 : BQ;
-    if (slot < nact) {
+    if (slot < nact) {  // (the lanes that a sum runs over have one slot)
       const h2 *vp[BQ];
-      const f2 *up[S];
 #pragma unroll
       for (int k = 0; k < BQ; k++) vp[k] = (const h2 *)v.p[q0 + (k < left ? k0 + k : nq - 1)] + base;
-#pragma unroll
-      for (int c = 0; c < S; c++) up[c] = (const f2 *)ut.p[c] + base;
-      const unsigned l4 = (threadIdx.x & 63) * 4u;
       h2 x[2][BQ];
-      f2 u[2][S];
-      auto fetch = [&](int h, long g) {
+      walk(
+          [&](int h, long g) {
 #pragma unroll
-        for (int k = 0; k < BQ; k++) x[h][k] = *(const h2 *)((const char *)(vp[k] + g * 64) + l4);
+            for (int k = 0; k < BQ; k++) x[h][k] = *(const h2 *)((const char *)(vp[k] + g * 64) + l4);
+            fetch_u(h, g);
+          },
+          [&](int h) {
 #pragma unroll
-        for (int c = 0; c < S; c++) u[h][c] = *(const f2 *)((const char *)(up[c] + g * 64) + 2 * l4);
-      };
-      auto work = [&](int h) {
-#pragma unroll
-        for (int k = 0; k < BQ; k++) add((float)x[h][k][0], (float)x[h][k][1], u[h], k);
-      };
-      long g = blockIdx.x;
-      const long st = a.gx;
-      fetch(0, g);
-      for (; g + 2 * st < groups; g += 2 * st) {
-        fetch(1, g + st);
-        work(0);
-        fetch(0, g + 2 * st);
-        work(1);
-      }
-      if (g + st < groups) {
-        fetch(1, g + st);
-        work(0);
-        work(1);
-      } else {
-        work(0);
-      }
+            for (int k = 0; k < BQ; k++) add((float)x[h][k][0], (float)x[h][k][1], u[h], k);
+          });
     }
-    const float f = (float)a.hinv;
-#pragma unroll
-    for (int k = 0; k < 2 * BQ * S; k++) af[k] *= f;
   } else if (slot < nact) {
-    for (long g = blockIdx.x; g < groups; g += a.gx) {
-      f2 u[S];
+    walk(fetch_u, [&](int h) {
 #pragma unroll
-      for (int c = 0; c < S; c++) u[c] = ((const f2 *)ut.p[c] + base + g * 64)[lane];
-#pragma unroll
-      for (int q = 0; q < S; q++) add(u[q][0], u[q][1], u, q);
-    }
+      for (int q = 0; q < S; q++) add(u[h][q][0], u[h][q][1], u[h], q);
+    });
   }
-  const int first = wv < nw ? k0 : nq;
+  const double f = wv < nw ? a.hinv : 1.0;
+  const int first = wv < nw ? k0 : nq, k1 = runs.first(lane);
 #pragma unroll
-  for (int k = 0; k < 2 * BQ * S; k++) {
-    double s = (double)af[k];
-    for (int o = 32; o >= nb; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (k < 2 * left * S && lane < nb && slot < nact)
-      part[((long)(2 * first * S + k) * a.cap + slot) * a.gx + blockIdx.x] = s;
+  for (int k = 0; k < decltype(runs)::M; k++) {
+    double s = f * runs.tot[k];
+    for (int o = (64 >> HV) / 2; o >= nb; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (k1 + k < 2 * left * S && (lane & ((64 >> HV) - 1)) < nb && slot < nact)
+      part[((long)(2 * first * S + k1 + k) * a.cap + slot) * a.gx + blockIdx.x] = s;
   }
 }
 
@@ -1178,14 +1188,19 @@ void MBlas::block(int j, int s, MultiSpinor *V, const MultiSpinor *const *U, Mul
   MShape a = shape(R, nact);
   const int gu = a.gx;
   a.gx = block_gx(a.rows, R.nb, R.nblk());
+  // FP32 sums no longer than a lane's in the other passes over these fields
+  const int most = (int)std::max(4L, std::min((long)BRUN, (a.rows * R.nb / ((long)MB * gu) + 1) / 2 * 2));
   reserve(need());
   with_s(s, [&](auto SS) {
     constexpr int S = decltype(SS)::value;
     for (int q0 = 0; q0 < nq; q0 += BCH) {
       const int n = std::min(BCH, nq - q0), last = q0 + n == nq;
       const int nv = 2 * S * (n + (last ? S : 0));
-      hipLaunchKernelGGL((k_mbdot<S>), dim3(a.gx, R.nblk()), dim3(64 * ((n + BQ - 1) / BQ + last)), 0, stream, a, tab,
-                         ut, q0, n, part);
+      const dim3 grid(a.gx, R.nblk()), wg(64 * ((n + BQ - 1) / BQ + last));
+      // halvings over the lanes of one slot: two where a wavefront has four rows of the slots
+      if (R.lognb <= 4) hipLaunchKernelGGL((k_mbdot<S, 2>), grid, wg, 0, stream, a, tab, ut, q0, n, most, part);
+      else if (R.lognb == 5) hipLaunchKernelGGL((k_mbdot<S, 1>), grid, wg, 0, stream, a, tab, ut, q0, n, most, part);
+      else hipLaunchKernelGGL((k_mbdot<S, 0>), grid, wg, 0, stream, a, tab, ut, q0, n, most, part);
       hipLaunchKernelGGL(k_mfinal, dim3(R.cap, nv), dim3(64), 0, stream, nv, R.cap, a.gx, nact, (const double *)part,
                          sums, q0 * S, 1);
     }

@@ -664,6 +664,12 @@ int qqcd_dense_harmonic_ritz(int m, const double *hbar, int ldh, int k, double *
  * solver kept for it, ||A V - V H|| / ||H|| }, Frobenius norms. */
 int qqcd_arnoldi_check(const double *phi, int m, const double *u, const double *coact, const double kappa[2],
                        const int *bc, int *steps, double out[3]);
+/* The pass of dots of a block of s steps over nq FP16 basis vectors on constant
+ * real fields: the basis vectors re[0] (batched: of unit length, stored times
+ * sqrt(12 stride)), the s new ones re[1..s].  sums: (nq + s) x s complex, row q
+ * <V_q, u_c>, then <u_r, u_c>, of the last of nrhs slots in blocks of nb
+ * (nrhs 0: the single-right-hand-side pass). */
+int qqcd_block_dots(int nrhs, int nb, int nq, int s, const double *re, double *sums);
 
 #ifdef __cplusplus
 }
