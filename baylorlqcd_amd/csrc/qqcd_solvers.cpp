@@ -461,21 +461,22 @@ static void alloc_work(Context &c, std::vector<std::unique_ptr<SpinorBuf>> &work
 }
 
 // The least-squares residual after columns j + 1 .. j + got: true once it is
-// below goal with at least `more` of these steps taken, got then cut to the
-// first such column (every column's residual is looked at only in the block
-// that gets there, or where res wants them all).
-static bool first_enough(const std::vector<zd> &H, int ldh, const std::vector<zd> &cv, std::vector<zd> &y, int j,
-                         int &got, double goal, int more, std::vector<double> *res = nullptr) {
+// below goal with at least `more` of these steps taken.  first: got is then cut to
+// the first such column (every column's residual is looked at only in the block
+// that gets there, or where res wants them all); otherwise all columns, whose
+// vectors have been paid for, go into the solution.
+static bool enough(const std::vector<zd> &H, int ldh, const std::vector<zd> &cv, std::vector<zd> &y, int j, int &got,
+                   double goal, int more, bool first, std::vector<double> *res = nullptr) {
   if (got < 1) return false;
   auto at = [&](int q) { return dense::lsq(j + q + 1, j + q, H.data(), ldh, cv.data(), y.data()); };
   const double last = at(got);
   const bool done = last < goal && got >= more;
   const int n = got;
-  if (!done && !res) return false;
+  if (!(done && first) && !res) return done;
   for (int q = 1; q <= n; q++) {
     const double r = q < n ? at(q) : last;
     if (res) res->push_back(r);
-    if (done && r < goal && q >= more) {
+    if (done && first && r < goal && q >= more) {
       got = q;
       break;
     }
@@ -573,7 +574,7 @@ SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int 
         bool ended = false;
         const int want = std::min(std::min(kCheck, m - j), std::max(1, maxiter - st.iters));
         int got = arnoldi_blocks(c, A, V, j, want, *ba, reorth != 0, loss, H, ldh, ended, work);
-        const bool done = first_enough(H, ldh, cv, y, j, got, tol * r0, itermin - st.iters);
+        const bool done = enough(H, ldh, cv, y, j, got, tol * r0, itermin - st.iters, reorth != 0);
         st.matvecs += got;
         st.iters += got;
         j += got;
@@ -766,7 +767,8 @@ SolveStats gmresproj(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, co
         const int want = std::min(std::min(kCheck, m - j), std::max(1, maxiter - st.iters));
         int got = arnoldi_blocks(c, A, V, j, want, *ba, reorth != 0, loss, H, ldh, ended, work);
         std::vector<double> res;
-        const bool done = first_enough(H, ldh, cv, y, j, got, tol * r0, itermin - st.iters, hist ? &res : nullptr);
+        const bool done =
+            enough(H, ldh, cv, y, j, got, tol * r0, itermin - st.iters, reorth != 0, hist ? &res : nullptr);
         for (size_t q = 0; q < res.size(); q++) hist->emplace_back(st.matvecs + 1 + (int)q, res[q]);
         st.matvecs += got;
         st.iters += got;
