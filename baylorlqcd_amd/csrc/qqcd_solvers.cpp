@@ -443,14 +443,14 @@ static void store_deflation(Context &c, Deflation *defl, const std::vector<Spino
   }
 }
 
-// whether a solve runs its Arnoldi steps in blocks: the basis in the work
-// precision (FP64, FP32), or in FP16 under FP32 with one Gram-Schmidt pass, an
-// operator without its diagonal, no preconditioner and no hook that wants
-// every step
+// whether a solve runs its Arnoldi steps in blocks: an FP64 basis (held
+// orthogonal where reorth asks for it), an FP32 one or FP16 under FP32 with one
+// Gram-Schmidt pass, an operator without its diagonal, no preconditioner and no
+// hook that wants every step
 static bool block_steps(const LinOp &A, int m, int reorth, const LinOp *M, const StepHook *step_hook) {
-  const bool own = A.basis() == A.prec && (A.prec == PREC_DOUBLE || A.prec == PREC_SINGLE);
-  const bool half = A.basis() == PREC_HALF && A.prec == PREC_SINGLE && !reorth;
-  return g_arnoldi_steps == 2 && A.apply_less && (own || half) && !M && !(step_hook && *step_hook) &&
+  const bool high = A.basis() == PREC_DOUBLE && A.prec == PREC_DOUBLE;
+  const bool low = A.prec == PREC_SINGLE && (A.basis() == PREC_SINGLE || A.basis() == PREC_HALF) && !reorth;
+  return g_arnoldi_steps == 2 && A.apply_less && (high || low) && !M && !(step_hook && *step_hook) &&
          m + 1 <= BlockArnoldi::NMAX;
 }
 
