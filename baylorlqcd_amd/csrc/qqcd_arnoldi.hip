@@ -426,7 +426,6 @@ BlockArnoldi::BlockArnoldi(hipStream_t s, int m_) : stream(s), m(m_), ld(m_ + 1)
 }
 
 BlockArnoldi::~BlockArnoldi() {
-  (void)hipStreamSynchronize(stream);  // a queued block still writes to the pinned slots
   pool_free(hd);
   pool_free(part);
   pool_free(sums);

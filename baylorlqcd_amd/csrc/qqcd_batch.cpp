@@ -102,8 +102,6 @@ class Batch {
  public:
   Batch(Context &c, const double kappa[2], MultiSpinor &B, MultiSpinor &X, const Deflation &D, const BatchParams &p,
         std::vector<int> &id);
-  // copies from the pinned buffers may be queued when an error unwinds
-  ~Batch() { (void)hipStreamSynchronize(c.stream); }
   BatchStats run(int n);
 
  private:

@@ -204,7 +204,6 @@ BiCGStabDev::BiCGStabDev(hipStream_t s, long n_) : stream(s), n(n_) {
 }
 
 BiCGStabDev::~BiCGStabDev() {
-  (void)hipStreamSynchronize(stream);  // a queued pass may still write the history
   pool_free(part);
   pool_free(state);
   pool_free_host(hist);

@@ -106,7 +106,11 @@ void *pool_alloc(size_t bytes) {
 }
 void pool_free(void *p) { give(p); }
 void *pool_alloc_host(size_t bytes) { return take(-1, bytes); }
-void pool_free_host(void *p) { give(p); }
+void pool_free_host(void *p) {
+  if (!p) return;
+  (void)hipDeviceSynchronize();
+  give(p);
+}
 
 void pool_trim() {
   Pool &P = pool();

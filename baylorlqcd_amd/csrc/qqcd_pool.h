@@ -9,7 +9,8 @@
 //
 //  * Order: a buffer may be freed while work on it is still queued on the
 //    context's stream; its next user queues on that same stream (the library
-//    has one) or on the null stream, which waits for it.
+//    has one) or on the null stream, which waits for it.  A pinned buffer's next
+//    user is the host, so returning one waits for the device.
 //  * Bounds: the free lists hold at most a quarter of the device's memory
 //    (buffers beyond that are released at once); a failed hipMalloc releases
 //    them and tries again; qqcd_init and qqcd_finalize release them all.

@@ -1,0 +1,26 @@
+"""The pool of device and pinned buffers, built for the CPU on a stand-in for
+the runtime that counts allocations, releases and waits."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "baylorlqcd_amd", "csrc")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("pool") / "pool_check")
+    subprocess.check_call([os.path.join(ROCM, "llvm", "bin", "clang++"), "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__",
+                           "-I" + os.path.join(ROCM, "include"), "-I" + CSRC, "-x", "c++",
+                           os.path.join(ROOT, "tests", "host", "pool_check.cpp"), os.path.join(CSRC, "qqcd_pool.cpp"),
+                           "-o", out])
+    return out
+
+
+@pytest.mark.parametrize("what", ["pinned_wait"])
+def test_pool(program, what):
+    r = subprocess.run([program, what], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
