@@ -1,13 +1,14 @@
 // qqcd_pool.cpp -- see qqcd_pool.h.
 #include "qqcd_pool.h"
 
+#include <cstdint>
+#include <deque>
 #include <map>
 #include <mutex>
 #include <stdexcept>
 #include <string>
 #include <unordered_map>
 #include <utility>
-#include <vector>
 
 #include "qqcd_internal.h"
 
@@ -17,11 +18,18 @@ namespace {
 
 typedef std::pair<int, size_t> Key;  // device (-1: pinned host memory) and rounded size
 
+// the free lists of device or of pinned memory; the newest of a size is at the back
+struct Idle {
+  std::map<Key, std::deque<std::pair<uint64_t, void *>>> lists;
+  size_t bytes = 0, cap = 0;
+};
+
 struct Pool {
   std::mutex mu;
-  std::map<Key, std::vector<void *>> idle;
+  Idle device, pinned;
   std::unordered_map<void *, Key> live;
-  size_t idle_bytes = 0, cap = 0;
+  uint64_t returned = 0;  // buffers given back so far: what orders them
+  Idle &of(const Key &k) { return k.first < 0 ? pinned : device; }
 };
 
 // never destroyed: buffers may be returned by objects of static storage
@@ -41,11 +49,25 @@ void release(const Key &k, void *p) {
   else (void)hipFree(p);
 }
 
-void drop_idle(Pool &P) {
-  for (auto &e : P.idle)
-    for (void *p : e.second) release(e.first, p);
-  P.idle.clear();
-  P.idle_bytes = 0;
+void drop_idle(Idle &I) {
+  for (auto &e : I.lists)
+    for (auto &b : e.second) release(e.first, b.second);
+  I.lists.clear();
+  I.bytes = 0;
+}
+
+// releases the buffers given back longest ago until `bytes` more fit
+void make_room(Idle &I, size_t bytes) {
+  while (I.bytes + bytes > I.cap) {
+    auto old = I.lists.end();
+    for (auto it = I.lists.begin(); it != I.lists.end(); ++it)
+      if (old == I.lists.end() || it->second.front().first < old->second.front().first) old = it;
+    if (old == I.lists.end()) return;
+    release(old->first, old->second.front().second);
+    I.bytes -= old->first.second;
+    old->second.pop_front();
+    if (old->second.empty()) I.lists.erase(old);
+  }
 }
 
 void *take(int dev, size_t bytes) {
@@ -53,18 +75,20 @@ void *take(int dev, size_t bytes) {
   std::lock_guard<std::mutex> lock(P.mu);
   const Key k(dev, rounded(bytes ? bytes : 1));
   void *p = nullptr;
-  auto it = P.idle.find(k);
-  if (it != P.idle.end() && !it->second.empty()) {
-    p = it->second.back();
+  Idle &I = P.of(k);
+  auto it = I.lists.find(k);
+  if (it != I.lists.end()) {
+    p = it->second.back().second;
     it->second.pop_back();
-    P.idle_bytes -= k.second;
+    if (it->second.empty()) I.lists.erase(it);
+    I.bytes -= k.second;
   } else {
     auto get = [&]() { return dev < 0 ? hipHostMalloc(&p, k.second, hipHostMallocDefault) : hipMalloc(&p, k.second); };
     hipError_t e = get();
-    if (e == hipErrorOutOfMemory && P.idle_bytes > 0) {
+    if (e == hipErrorOutOfMemory && I.bytes > 0) {
       (void)hipGetLastError();
       (void)hipDeviceSynchronize();
-      drop_idle(P);
+      drop_idle(I);
       e = get();
     }
     if (e != hipSuccess) {
@@ -85,16 +109,19 @@ void give(void *p) {
   if (it == P.live.end()) return;
   const Key k = it->second;
   P.live.erase(it);
-  if (!P.cap) {
+  Idle &I = P.of(k);
+  if (!I.cap) {
     size_t free_b = 0, total = 0;
-    P.cap = hipMemGetInfo(&free_b, &total) == hipSuccess && total ? total / 4 : size_t(1) << 30;
+    const bool known = k.first >= 0 && hipMemGetInfo(&free_b, &total) == hipSuccess && total;
+    I.cap = known ? total / 4 : size_t(1) << 30;
   }
-  if (P.idle_bytes + k.second > P.cap) {
+  if (k.second > I.cap) {
     release(k, p);
     return;
   }
-  P.idle[k].push_back(p);
-  P.idle_bytes += k.second;
+  make_room(I, k.second);
+  I.lists[k].emplace_back(P.returned++, p);
+  I.bytes += k.second;
 }
 
 }  // namespace
@@ -115,9 +142,10 @@ void pool_free_host(void *p) {
 void pool_trim() {
   Pool &P = pool();
   std::lock_guard<std::mutex> lock(P.mu);
-  if (P.idle.empty()) return;
+  if (P.device.lists.empty() && P.pinned.lists.empty()) return;
   (void)hipDeviceSynchronize();
-  drop_idle(P);
+  drop_idle(P.device);
+  drop_idle(P.pinned);
 }
 
 }  // namespace qqcd

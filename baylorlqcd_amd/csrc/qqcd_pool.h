@@ -11,9 +11,11 @@
 //    context's stream; its next user queues on that same stream (the library
 //    has one) or on the null stream, which waits for it.  A pinned buffer's next
 //    user is the host, so returning one waits for the device.
-//  * Bounds: the free lists hold at most a quarter of the device's memory
-//    (buffers beyond that are released at once); a failed hipMalloc releases
-//    them and tries again; qqcd_init and qqcd_finalize release them all.
+//  * Bounds: the free lists hold at most a quarter of the device's memory and 1
+//    GiB of pinned memory (beyond that the buffers given back longest ago are
+//    released, so that a program that changes its sizes keeps its current ones);
+//    a failed hipMalloc releases them and tries again; qqcd_init and
+//    qqcd_finalize release them all.
 //  * Contents are undefined: a caller that needs zeros clears the buffer.
 //  * Calls from several threads are serialised by a mutex.
 #pragma once

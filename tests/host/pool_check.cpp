@@ -87,9 +87,53 @@ int pinned_wait() {
   return 0;
 }
 
+// the lists are full of buffers of one size: a program that goes on with another gets its own back all the same, and
+// the bound (a quarter of the card) holds
+int other_size() {
+  std::vector<void *> a;
+  for (int i = 0; i < 8; i++) a.push_back(pool_alloc(2 * MB));
+  for (void *p : a) pool_free(p);
+  EXPECT(used == 16 * MB);
+  for (int i = 0; i < 5; i++) {
+    void *p = pool_alloc(4 * MB), *q = pool_alloc(4 * MB);
+    pool_free(p);
+    pool_free(q);
+    EXPECT(used <= 16 * MB);
+  }
+  EXPECT(mallocs == 8 + 2);
+  // the ones given back longest ago went: what is left of the first size is kept
+  EXPECT(used == 16 * MB && frees == 4);
+  // a buffer larger than the bound is not kept
+  void *big = pool_alloc(20 * MB);
+  pool_free(big);
+  EXPECT(used <= 16 * MB);
+  pool_trim();
+  EXPECT(used == 0);
+  return 0;
+}
+
+// pinned memory is the host's: it takes nothing of the card's share, and has a bound of its own
+int pinned_share() {
+  void *h = pool_alloc_host(15 * MB);
+  pool_free_host(h);
+  void *a = pool_alloc(8 * MB);
+  pool_free(a);
+  EXPECT(used == 8 * MB);
+  EXPECT(pool_alloc(8 * MB) == a);
+  std::vector<void *> v;
+  for (int i = 0; i < 100; i++) v.push_back(pool_alloc_host(16 * MB));
+  for (void *p : v) pool_free_host(p);
+  EXPECT(pinned <= 1024 * MB);
+  pool_trim();
+  EXPECT(pinned == 0);
+  return 0;
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "pinned_wait") return pinned_wait();
+  if (what == "other_size") return other_size();
+  if (what == "pinned_share") return pinned_share();
   std::printf("no such check\n");
   return 2;
 }
