@@ -18,6 +18,7 @@
 #include <type_traits>
 #include <vector>
 #include "qqcd_blas.h"
+#include "qqcd_pool.h"
 
 namespace qqcd {
 
@@ -492,13 +493,13 @@ __global__ void __launch_bounds__(RB) k_recombine(long n, int m, const void *con
 
 Blas::Blas(hipStream_t s) : stream(s) {
   // partials: RG rows of 2 per vector
-  QQCD_HIP(hipMalloc(&part, sizeof(double) * RG * 2 * kmax));
+  QQCD_HIP(device_malloc(&part, sizeof(double) * RG * 2 * kmax));
   // one 2*KMAXP slab of results per pass of up to KMAXP vectors
   const long nres = 2L * KMAXP * ((kmax + KMAXP - 1) / KMAXP);
-  QQCD_HIP(hipMalloc(&res, sizeof(double) * nres));
+  QQCD_HIP(device_malloc(&res, sizeof(double) * nres));
   QQCD_HIP(hipHostMalloc(&hres, sizeof(double) * nres, hipHostMallocDefault));
-  QQCD_HIP(hipMalloc(&zbuf, sizeof(double) * 2 * zcap));
-  QQCD_HIP(hipMalloc(&vptr, sizeof(void *) * 256));  // 128 vector and 128 norm pointers
+  QQCD_HIP(device_malloc(&zbuf, sizeof(double) * 2 * zcap));
+  QQCD_HIP(device_malloc(&vptr, sizeof(void *) * 256));  // 128 vector and 128 norm pointers
 }
 
 Blas::~Blas() {
@@ -852,14 +853,14 @@ double bench_blas(long n, Prec p, int k, int op, int grid, int niter, hipStream_
   try {
     for (int q = 0; q <= k; q++) {
       const size_t b = q < k ? bytes : wbytes;
-      QQCD_HIP(hipMalloc(&v[q], b));
+      QQCD_HIP(device_malloc(&v[q], b));
       QQCD_HIP(hipMemsetAsync(v[q], 0, b, s));
       if (q < k && p == PREC_HALF) {
-        QQCD_HIP(hipMalloc(&nv[q], sizeof(float) * (n / 12)));
+        QQCD_HIP(device_malloc(&nv[q], sizeof(float) * (n / 12)));
         QQCD_HIP(hipMemsetAsync(nv[q], 0, sizeof(float) * (n / 12), s));
       }
     }
-    QQCD_HIP(hipMalloc(&part, sizeof(double) * grid * 2 * KMAXP));
+    QQCD_HIP(device_malloc(&part, sizeof(double) * grid * 2 * KMAXP));
     PtrPack pp{};
     CoefPack cp{};
     for (int q = 0; q < k; q++) {

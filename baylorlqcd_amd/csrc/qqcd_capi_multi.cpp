@@ -241,7 +241,7 @@ void lag_out(const LagState &st, int *iw, int *jr, int *kr) {
 
 struct DevU32 {
   uint32_t *p = nullptr;
-  explicit DevU32(size_t n) { QQCD_HIP(hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(uint32_t))); }
+  explicit DevU32(size_t n) { QQCD_HIP(device_malloc(&p, std::max<size_t>(n, 1) * sizeof(uint32_t))); }
   ~DevU32() {
     if (p) (void)hipFree(p);
   }

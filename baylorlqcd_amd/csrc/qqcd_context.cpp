@@ -58,7 +58,7 @@ Gauge alloc_gauge(const Geom &g, Prec p, int recon) {
   u.prec = p;
   u.recon = recon;
   u.stride = g.stride;
-  QQCD_HIP(hipMalloc(&u.data, u.bytes()));
+  QQCD_HIP(device_malloc(&u.data, u.bytes()));
   QQCD_HIP(hipMemset(u.data, 0, u.bytes()));
   return u;
 }

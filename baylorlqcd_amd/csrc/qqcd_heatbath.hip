@@ -301,7 +301,7 @@ double plaquette(Context &c) {
   const Geom &g = c.g;
   const int nb = (int)((g.Vh + 255) / 256);
   double *part = nullptr;
-  QQCD_HIP(hipMalloc(&part, sizeof(double) * nb));
+  QQCD_HIP(device_malloc(&part, sizeof(double) * nb));
   std::vector<double> h(nb);
   double tot = 0;
   for (int par = 0; par < 2; par++) {

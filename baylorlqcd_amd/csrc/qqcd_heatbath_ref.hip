@@ -534,7 +534,7 @@ namespace {
 
 template <typename T> struct DBuf {
   T *p = nullptr;
-  explicit DBuf(size_t n) { QQCD_HIP(hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(T))); }
+  explicit DBuf(size_t n) { QQCD_HIP(device_malloc(&p, std::max<size_t>(n, 1) * sizeof(T))); }
   ~DBuf() {
     if (p) (void)hipFree(p);
   }
@@ -555,8 +555,8 @@ struct HbStream {
   HbStream(const LagState &st, long cap_, hipStream_t s_) : gen(st), cap(cap_), s(s_) {
     for (int k = 0; k < 521; k++) start_w[k] = st.w[k];
     start_jr = st.jr;
-    QQCD_HIP(hipMalloc(&buf, sizeof(uint32_t) * cap));
-    QQCD_HIP(hipMalloc(&alt, sizeof(uint32_t) * cap));
+    QQCD_HIP(device_malloc(&buf, sizeof(uint32_t) * cap));
+    QQCD_HIP(device_malloc(&alt, sizeof(uint32_t) * cap));
   }
   ~HbStream() {
     (void)hipFree(buf);

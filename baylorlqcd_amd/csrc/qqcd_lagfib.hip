@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "qqcd_lagfib.h"
+#include "qqcd_pool.h"
 
 namespace qqcd {
 
@@ -182,7 +183,7 @@ static const uint32_t *table_for(long L, int K, hipStream_t s) {
     QQCD_HIP(hipFree(t->d));
     t->d = nullptr;
   }
-  QQCD_HIP(hipMalloc(&t->d, sizeof(uint32_t) * t->h.size()));
+  QQCD_HIP(device_malloc(&t->d, sizeof(uint32_t) * t->h.size()));
   QQCD_HIP(hipMemcpyAsync(t->d, t->h.data(), sizeof(uint32_t) * t->h.size(), hipMemcpyHostToDevice, s));
   QQCD_HIP(hipStreamSynchronize(s));
   t->K = K;
@@ -433,9 +434,9 @@ void lagfib_generate(LagState &st, long m, uint32_t *d_out, hipStream_t s) {
   if (m < 0) throw std::runtime_error("lagfib_generate: negative count");
   LagWork w;
   w.table = [](void *, long L, int K, hipStream_t st) { return table_for(L, K, st); };
-  QQCD_HIP(hipMalloc(&w.base, sizeof(uint32_t) * 2 * LP));
-  QQCD_HIP(hipMalloc(&w.dz, sizeof(unsigned long long)));
-  QQCD_HIP(hipMalloc(&w.bad, sizeof(int)));
+  QQCD_HIP(device_malloc(&w.base, sizeof(uint32_t) * 2 * LP));
+  QQCD_HIP(device_malloc(&w.dz, sizeof(unsigned long long)));
+  QQCD_HIP(device_malloc(&w.bad, sizeof(int)));
   try {
     lag_generate_with(st, m, d_out, s, w);
   } catch (...) {
@@ -549,9 +550,9 @@ double bench_lagfib(long m, int niter, long chunk, hipStream_t s) {
   const uint32_t *rows = table_for(L, K, s);
   uint32_t *dbase = nullptr, *out = nullptr;
   unsigned long long *dz = nullptr;
-  QQCD_HIP(hipMalloc(&dbase, sizeof(hb)));
-  QQCD_HIP(hipMalloc(&dz, sizeof(unsigned long long)));
-  QQCD_HIP(hipMalloc(&out, sizeof(uint32_t) * m));
+  QQCD_HIP(device_malloc(&dbase, sizeof(hb)));
+  QQCD_HIP(device_malloc(&dz, sizeof(unsigned long long)));
+  QQCD_HIP(device_malloc(&out, sizeof(uint32_t) * m));
   QQCD_HIP(hipMemcpyAsync(dbase, hb, sizeof(hb), hipMemcpyHostToDevice, s));
   QQCD_HIP(hipMemsetAsync(dz, 0xff, sizeof(unsigned long long), s));
   hipEvent_t e0, e1;

@@ -275,7 +275,7 @@ extern "C" int qqcd_nn_layer_canonical(int layer, int adjoint, const double *in,
   NNField fi = alloc_nn(c.g, ci), fo = alloc_nn(c.g, co);
   double *d = nullptr;
   try {
-    QQCD_HIP(hipMalloc(&d, n * sizeof(double)));
+    QQCD_HIP(device_malloc(&d, n * sizeof(double)));
     for (int ch = 0; ch < ci; ch++) {
       QQCD_HIP(hipMemcpyAsync(d, in + ch * n, n * sizeof(double), hipMemcpyHostToDevice, c.stream));
       nn_from_canon(c.g, d, fi, ch, c.stream);
@@ -310,7 +310,7 @@ extern "C" int qqcd_nn_wgrad_canonical(int layer, const double *psi, const doubl
   NNField fi = alloc_nn(c.g, ci), fg = alloc_nn(c.g, co);
   double *d = nullptr;
   try {
-    QQCD_HIP(hipMalloc(&d, n * sizeof(double)));
+    QQCD_HIP(device_malloc(&d, n * sizeof(double)));
     for (int ch = 0; ch < ci; ch++) {
       QQCD_HIP(hipMemcpyAsync(d, psi + ch * n, n * sizeof(double), hipMemcpyHostToDevice, c.stream));
       nn_from_canon(c.g, d, fi, ch, c.stream);
@@ -383,7 +383,7 @@ extern "C" int qqcd_nn_train(int nconf, double beta, int nsweep, double kappa_lo
   M.upload(c.stream);
   M.alloc_grads(c.g);
   double *d_scr = nullptr;
-  QQCD_HIP(hipMalloc(&d_scr, sizeof(double) * ((2 * c.g.Vh + 255) / 256 + 16)));
+  QQCD_HIP(device_malloc(&d_scr, sizeof(double) * ((2 * c.g.Vh + 255) / 256 + 16)));
   // the mean loss over a fixed sample of at most 512 pairs, evenly spaced
   // over the harvest (every configuration and every stage of the solves)
   const size_t nsample = std::min<size_t>(512, T.pairs.size());
@@ -492,7 +492,7 @@ extern "C" int qqcd_nn_apply_canonical(const double *r, double *z) {
   NNModel &M = nn_model(c);
   const size_t n = (size_t)24 * c.g.V;
   double *d = nullptr;
-  QQCD_HIP(hipMalloc(&d, n * sizeof(double)));
+  QQCD_HIP(device_malloc(&d, n * sizeof(double)));
   try {
     SpinorBuf a(c.g, PREC_SINGLE), b(c.g, PREC_SINGLE);
     QQCD_HIP(hipMemcpyAsync(d, r, n * sizeof(double), hipMemcpyHostToDevice, c.stream));

@@ -321,8 +321,8 @@ __global__ void __launch_bounds__(256) k_copy(long n, const double2 *__restrict_
 double bench_copy(size_t bytes, int iters, hipStream_t s) {
   const long n = (long)(bytes / 16);
   double2 *a = nullptr, *b = nullptr;
-  QQCD_HIP(hipMalloc(&a, n * 16));
-  QQCD_HIP(hipMalloc(&b, n * 16));
+  QQCD_HIP(device_malloc(&a, n * 16));
+  QQCD_HIP(device_malloc(&b, n * 16));
   QQCD_HIP(hipMemsetAsync(a, 0, n * 16, s));
   hipEvent_t e0, e1;
   QQCD_HIP(hipEventCreate(&e0));

@@ -979,7 +979,7 @@ static void upload_vec(const std::vector<uint16_t> &h, uint16_t *&d, size_t &n, 
     (void)hipFree(d);
     d = nullptr;
   }
-  if (!d) QQCD_HIP(hipMalloc(&d, h.size() * 2));
+  if (!d) QQCD_HIP(device_malloc(&d, h.size() * 2));
   n = h.size();
   QQCD_HIP(hipMemcpyAsync(d, h.data(), h.size() * 2, hipMemcpyHostToDevice, s));
 }
@@ -1008,7 +1008,7 @@ NNLinks nn_links(const Geom &g, const Gauge &U32, hipStream_t s) {
   NNLinks L;
   L.stride = U32.stride;
   const long n = 2L * 4 * 9 * U32.stride;
-  QQCD_HIP(hipMalloc(&L.data, n * sizeof(uint32_t)));
+  QQCD_HIP(device_malloc(&L.data, n * sizeof(uint32_t)));
   hipLaunchKernelGGL(k_nn_links, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, (const float2 *)U32.data,
                      L.data);
   QQCD_HIP(hipGetLastError());
@@ -1084,8 +1084,8 @@ void nn_wgrad(const Geom &g, const NNLinks &U, int cin, int cout, const NNField 
     part = nullptr;
     res = nullptr;
     cap = 0;
-    QQCD_HIP(hipMalloc(&part, sizeof(float) * ne * nwg));
-    QQCD_HIP(hipMalloc(&res, sizeof(double) * ne * nwg));
+    QQCD_HIP(device_malloc(&part, sizeof(float) * ne * nwg));
+    QQCD_HIP(device_malloc(&res, sizeof(double) * ne * nwg));
     cap = ne * nwg;
   }
   std::vector<double> P(ne);

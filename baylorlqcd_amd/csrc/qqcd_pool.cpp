@@ -139,6 +139,21 @@ void pool_free_host(void *p) {
   give(p);
 }
 
+hipError_t device_malloc_bytes(void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();  // the caller reports it, no later launch
+    Pool &P = pool();
+    std::lock_guard<std::mutex> lock(P.mu);
+    if (P.device.lists.empty()) return e;
+    (void)hipDeviceSynchronize();
+    drop_idle(P.device);
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+  }
+  return e;
+}
+
 void pool_trim() {
   Pool &P = pool();
   std::lock_guard<std::mutex> lock(P.mu);

@@ -31,6 +31,13 @@ void *pool_alloc_host(size_t bytes);  // pinned
 void pool_free_host(void *p);
 void pool_trim();  // releases every free buffer (waits for the device first)
 
+// hipMalloc for a buffer that outlives calls (freed by hipFree): idle buffers
+// are released where the card has no room for it
+hipError_t device_malloc_bytes(void **p, size_t bytes);
+template <typename T> hipError_t device_malloc(T **p, size_t bytes) {
+  return device_malloc_bytes(reinterpret_cast<void **>(p), bytes);
+}
+
 template <typename T> void pool_get(T **p, size_t bytes) { *p = static_cast<T *>(pool_alloc(bytes)); }
 
 }  // namespace qqcd

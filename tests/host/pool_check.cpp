@@ -129,11 +129,28 @@ int pinned_share() {
   return 0;
 }
 
+// a buffer that is not pooled gets the memory that idle ones hold
+int unpooled() {
+  for (int i = 0; i < 4; i++) {
+    void *p = pool_alloc((2 + 2 * i) * MB);
+    pool_free(p);
+  }
+  EXPECT(used > 0);
+  void *p = nullptr;
+  EXPECT(device_malloc(&p, 60 * MB) == hipSuccess);
+  EXPECT(used == 60 * MB);
+  double *q = nullptr;
+  EXPECT(device_malloc(&q, 10 * MB) == hipErrorOutOfMemory);
+  EXPECT(hipFree(p) == hipSuccess && used == 0);
+  return 0;
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "pinned_wait") return pinned_wait();
   if (what == "other_size") return other_size();
   if (what == "pinned_share") return pinned_share();
+  if (what == "unpooled") return unpooled();
   std::printf("no such check\n");
   return 2;
 }

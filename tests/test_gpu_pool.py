@@ -79,3 +79,36 @@ def test_failed_allocation_is_an_error():
         diracops.gauge_random(0, 0.0, 1, O.coact_array())
         assert np.isfinite(diracops.gauge_plaquette())
         lattice.finalize()
+
+
+def test_full_card():
+    """The card is full but for what the pool holds idle: calls that need memory outside the pool (gauge copies in
+    other formats) and pooled buffers of new sizes get it."""
+    n = (16, 16, 16, 8)
+    lattice.init(n, BC)
+    hold = []
+    try:
+        diracops.gauge_random(1, 0.1, 7, O.coact_array())
+        u = diracops.gauge_get_ref(n)
+        diracops.gauge_load(u, O.coact_array())
+        L = int(np.prod(lattice.spinor_shape(n)))
+        b, x = np.zeros(L), np.zeros(L)
+        disconloops.z4source(b, None, 5, 0)
+        disconloops.noise_loop(16, 5, (0.14, 0.0), (60, 10), tol=1e-10, coact=O.coact_array(), bc=BC, u=u)
+        torch.zeros(1, device="cuda")
+        step = free_bytes()
+        while step >= 2 << 20:  # all of it, in falling halves
+            try:
+                hold.append(torch.empty(step, dtype=torch.uint8, device="cuda"))
+            except torch.OutOfMemoryError:
+                step //= 2
+        psi = np.random.default_rng(2).standard_normal((1, int(np.prod(n)), 4, 6)).view(complex)
+        out = np.empty_like(psi)
+        disconloops.schur_multi_canonical(psi, out, (0.14, 0.0), prec=1, recon=18)  # 9 MB of links in FP32 first
+        assert np.all(np.isfinite(out)) and np.any(out)
+        it = inverters.solve_mixed(b, x, (20, 5), 1e-10, 1, 1, 12, 0.0, 0, u, O.coact_array(), (0.14, 0.01), BC)
+        assert it > 0 and np.all(np.isfinite(x)) and np.any(x)
+    finally:
+        hold.clear()
+        torch.cuda.empty_cache()
+        lattice.finalize()
