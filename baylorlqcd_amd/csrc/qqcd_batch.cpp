@@ -224,6 +224,7 @@ Batch::Batch(Context &c_, const double kappa[2], MultiSpinor &B_, MultiSpinor &X
     basis_bufs.emplace_back(new MultiBuf(c.g, p.basis, cap, nb, false));
     V.push_back(basis_bufs.back()->m);
   }
+  A32.set_half_mid(p.half_mid != 0);
   if (half()) {
     Wf.reset(new MultiBuf(c.g, PREC_SINGLE, cap, nb));
     Qf.reset(new MultiBuf(c.g, PREC_SINGLE, cap, nb));
@@ -231,15 +232,22 @@ Batch::Batch(Context &c_, const double kappa[2], MultiSpinor &B_, MultiSpinor &X
     hs = std::sqrt(12.0 * (double)c.g.stride);
     quads = p.sstep == 2 && p.reorth == 0 && p.pair_norms && MBlas::can_block(m, B.nblk());
     paired = !quads && fused && p.sstep == 2 && p.reorth == 0 && m % 2 == 0;
-    if (quads) {
-      sigma = A32.diag();
-      U3f.reset(new MultiBuf(c.g, PREC_SINGLE, cap, nb));
-      U4f.reset(new MultiBuf(c.g, PREC_SINGLE, cap, nb));
-    }
     if (paired || quads) U2f.reset(new MultiBuf(c.g, PREC_SINGLE, cap, nb));
+    // where the card has no room for the two fields and the larger partial sums that blocks of four take beyond
+    // pairs of steps, the batch runs in pairs
+    if (quads) try {
+        U3f.reset(new MultiBuf(c.g, PREC_SINGLE, cap, nb));
+        U4f.reset(new MultiBuf(c.g, PREC_SINGLE, cap, nb));
+        mb.reserve(mb.need(true));
+        sigma = A32.diag();
+      } catch (const std::exception &) {
+        quads = false;
+        U3f.reset();
+        U4f.reset();
+        paired = fused && m % 2 == 0;
+      }
   }
-  A32.set_half_mid(p.half_mid != 0);
-  mb.reserve(mb.need());
+  mb.reserve(mb.need(quads));
   clear_flags(d_flag(), d_any(), cap, c.stream);
   st.iters.assign(cap, 0);
   st.rel_res.assign(cap, 0.0);

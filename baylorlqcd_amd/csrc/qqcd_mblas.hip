@@ -857,8 +857,9 @@ static int gx_of(long rows, int nb, int nblk) {
 // (MAXK complex dots and a norm, or MAXK2 complex dots with each of two
 // fields): sized once, before any capture, so that no later pass moves the
 // buffer a captured graph names
-size_t MBlas::need() const {
-  return std::max((size_t)2048 * std::max(2 * MAXK + 2, 4 * MAXK2 + 4) * cap, (size_t)8 * (BCH + 4) * 1024 * std::min(cap, 64)) + 64;
+size_t MBlas::need(bool blocks) const {
+  const size_t steps = (size_t)2048 * std::max(2 * MAXK + 2, 4 * MAXK2 + 4) * cap;
+  return (blocks ? std::max(steps, (size_t)8 * (BCH + 4) * 1024 * std::min(cap, 64)) : steps) + 64;
 }
 
 static MShape shape(const MultiSpinor &W, const int *nact) {
@@ -1190,7 +1191,7 @@ void MBlas::block(int j, int s, MultiSpinor *V, const MultiSpinor *const *U, Mul
   a.gx = block_gx(a.rows, R.nb, R.nblk());
   // FP32 sums no longer than a lane's in the other passes over these fields
   const int most = (int)std::max(4L, std::min((long)BRUN, (a.rows * R.nb / ((long)MB * gu) + 1) / 2 * 2));
-  reserve(need());
+  reserve(need(true));
   with_s(s, [&](auto SS) {
     constexpr int S = decltype(SS)::value;
     for (int q0 = 0; q0 < nq; q0 += BCH) {

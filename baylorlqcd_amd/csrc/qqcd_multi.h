@@ -96,7 +96,7 @@ class MBlas {
  public:
   // size the partial-sum scratch before a graph capture (no allocation inside one)
   void reserve(size_t n);
-  size_t need() const;
+  size_t need(bool blocks) const;  // blocks: with block()
 };
 
 // Element-wise per-slot Arnoldi bookkeeping (qqcd_mblas.hip):

@@ -454,10 +454,18 @@ static bool block_steps(const LinOp &A, int m, int reorth, const LinOp *M, const
          m + 1 <= BlockArnoldi::NMAX;
 }
 
-// the work-precision vectors of a solve whose basis is stored lower: one, or a block's
-static void alloc_work(Context &c, std::vector<std::unique_ptr<SpinorBuf>> &work, bool lower, bool blocks, Prec p) {
+// the work-precision vectors of a solve whose basis is stored lower: a block's,
+// or one where the card has no room for those; returns whether it is blocks
+static bool alloc_work(Context &c, std::vector<std::unique_ptr<SpinorBuf>> &work, bool lower, bool blocks, Prec p) {
   work.clear();
-  for (int i = 0; lower && i < (blocks ? BlockArnoldi::SMAX : 1); i++) work.emplace_back(new SpinorBuf(c.g, p));
+  if (!lower) return blocks;
+  try {
+    for (int i = 0; i < (blocks ? BlockArnoldi::SMAX : 1); i++) work.emplace_back(new SpinorBuf(c.g, p));
+    return blocks;
+  } catch (const std::exception &) {
+    if (!blocks) throw;
+  }
+  return alloc_work(c, work, lower, false, p);
 }
 
 // The least-squares residual after columns j + 1 .. j + got: true once it is
@@ -539,9 +547,8 @@ SolveStats gmresdr(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, int 
     alloc_basis(c, Z, m, p);
     alloc_basis(c, ZW, k, p);
   }
-  const bool blocks = block_steps(A, m, reorth, M, step_hook);
   std::vector<std::unique_ptr<SpinorBuf>> work;
-  alloc_work(c, work, vp != p, blocks, p);
+  const bool blocks = alloc_work(c, work, vp != p, block_steps(A, m, reorth, M, step_hook), p);
   std::unique_ptr<DevHess> dh;
   if (!reorth && !blocks) dh.reset(new DevHess(m));
   std::unique_ptr<BlockArnoldi> ba;
@@ -697,14 +704,13 @@ SolveStats gmresproj(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, co
   std::vector<std::unique_ptr<SpinorBuf>> *wp = &work_own;
   DevHess *dh = nullptr;
   StepGraphs *sg = nullptr;
-  const bool blocks = block_steps(A, m, reorth, nullptr, nullptr);
-  const bool dev = !reorth && !blocks;
+  bool blocks = block_steps(A, m, reorth, nullptr, nullptr);
   if (ws) {
-    if (ws->m != m || ws->p != p || ws->vp != vp || dev != (ws->dh != nullptr)) {
+    if (ws->m != m || ws->p != p || ws->vp != vp || (!reorth && !blocks) != (ws->dh != nullptr)) {
       ws->reset();
       alloc_basis(c, ws->V, m + 1, vp);
-      alloc_work(c, ws->work, vp != p, blocks, p);
-      if (dev) ws->dh.reset(new DevHess(m));
+      blocks = alloc_work(c, ws->work, vp != p, blocks, p);
+      if (!reorth && !blocks) ws->dh.reset(new DevHess(m));
       ws->m = m;
       ws->p = p;
       ws->vp = vp;
@@ -717,8 +723,8 @@ SolveStats gmresproj(Context &c, LinOp &A, const Spinor &b, Spinor &x, int m, co
     sg = ws->sg.get();
   } else {
     alloc_basis(c, Vown, m + 1, vp);
-    alloc_work(c, work_own, vp != p, blocks, p);
-    if (dev) dh_own.reset(new DevHess(m));
+    blocks = alloc_work(c, work_own, vp != p, blocks, p);
+    if (!reorth && !blocks) dh_own.reset(new DevHess(m));
     if (dh_own && g_step_graphs == 1) sg_own.reset(new StepGraphs);
     dh = dh_own.get();
     sg = sg_own.get();

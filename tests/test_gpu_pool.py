@@ -112,3 +112,51 @@ def test_full_card():
         hold.clear()
         torch.cuda.empty_cache()
         lattice.finalize()
+
+
+def fill_card(leave):
+    """Takes all of the card's free memory but about `leave` bytes."""
+    hold, step = [], max(free_bytes() - leave, 0)
+    while step >= 2 << 20:
+        if free_bytes() - leave >= step:
+            try:
+                hold.append(torch.empty(step, dtype=torch.uint8, device="cuda"))
+                continue
+            except torch.OutOfMemoryError:
+                pass
+        step //= 2
+    return hold
+
+
+@pytest.mark.parametrize("room", [26.5, 27.5])
+def test_batch_with_less_memory(room):
+    """Blocks of four steps take two FP32 fields and 22 MB of partial sums more than pairs of steps do (28 fields in
+    all here, 26 in pairs): where the card has no room for those the batch runs in pairs, as it did when there were
+    no blocks."""
+    n, nrhs, gm, kappa = (16, 16, 16, 16), 16, (30, 10), (0.12, 0.0)
+    hold = []
+    lattice.init(n, BC)
+    try:
+        torch.zeros(1, device="cuda")
+        diracops.gauge_random(1, 0.1, 7, O.coact_array())
+        u = diracops.gauge_get_ref(n)
+        diracops.gauge_load(u, O.coact_array())
+
+        def loop():
+            nz = disconloops.noise_loop(nrhs, 5, kappa, gm, tol=1e-10, coact=O.coact_array(), bc=BC, u=u, loops=False,
+                                        nb=8)
+            assert np.all(nz["res_full"] < 1e-9) and disconloops.batch_stats()["fallback"] == 0
+            return nz["traces"]
+
+        want = loop()
+        lattice.finalize()
+        lattice.init(n, BC)
+        diracops.gauge_load(u, O.coact_array())
+        hold = fill_card(int(room * nrhs * (int(np.prod(n)) // 2) * 96))
+        got = loop()
+    finally:
+        hold.clear()
+        torch.cuda.empty_cache()
+        lattice.finalize()
+    # two solutions to 1e-10 of a system of condition number below 1e2
+    assert np.linalg.norm(got - want) < 1e-8 * np.linalg.norm(want)
