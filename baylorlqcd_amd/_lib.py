@@ -55,6 +55,7 @@ SIGNATURES = {
     "qqcd_set_pair_norms": [ctypes.c_int],
     "qqcd_set_batch_mid": [ctypes.c_int],
     "qqcd_set_step_graphs": [ctypes.c_int],
+    "qqcd_step_graph_replays": [_lp],
     "qqcd_gauge_random": [ctypes.c_int, ctypes.c_double, ctypes.c_ulonglong, _dp],
     "qqcd_gauge_get_canonical": [_dp],
     "qqcd_gauge_heatbath": [ctypes.c_double, ctypes.c_int, ctypes.c_ulonglong, ctypes.c_int, _dp],

@@ -315,6 +315,12 @@ extern "C" int qqcd_set_step_graphs(int mode) {
   API_END
 }
 
+extern "C" int qqcd_step_graph_replays(long *n) {
+  API_BEGIN
+  *n = step_graph_replays();
+  API_END
+}
+
 extern "C" int qqcd_deflation_clear(void) {
   API_BEGIN
   if (g_defl) {

@@ -188,6 +188,8 @@ void set_step_graphs(int mode) {
   g_step_graphs = mode;
 }
 
+static long g_graph_replays = 0;
+long step_graph_replays() { return g_graph_replays; }
 struct StepGraphs {
   struct Entry {
     std::vector<const void *> key;
@@ -195,7 +197,6 @@ struct StepGraphs {
     hipGraphExec_t e = nullptr;
   };
   std::vector<Entry> list;
-  int replays = 0;
   StepGraphs() = default;
   StepGraphs(const StepGraphs &) = delete;
   StepGraphs &operator=(const StepGraphs &) = delete;
@@ -225,7 +226,7 @@ static void arnoldi_steps_dev(Context &c, LinOp &A, std::vector<Spinor> &V, int 
   for (auto &x : sg->list)
     if (x.key == key) {
       QQCD_HIP(hipGraphLaunch(x.e, c.stream));
-      sg->replays++;
+      g_graph_replays++;
       return;
     }
   // first time: run the steps, then record them for the next time

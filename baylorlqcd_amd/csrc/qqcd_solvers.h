@@ -170,6 +170,7 @@ namespace qqcd {
 // graphs: 0 never, 1 in every solve, 2 (the default) only where the basis is
 // kept between calls (ProjWork), so that a capture serves many solves
 void set_step_graphs(int mode);
+long step_graph_replays();  // since the library was loaded
 // Arnoldi steps per Gram-Schmidt pass: 2 (the default) in blocks of four (the
 // batched solver: in pairs), 1 one at a time
 void set_arnoldi_steps(int steps);

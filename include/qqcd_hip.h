@@ -626,8 +626,12 @@ int qqcd_set_multi_lds(int bytes);
  * fresh basis replays about three times, too few to repay its capture), 2
  * (the default) only in the mixed solver's later outer steps, whose
  * GMRES-Proj keeps its basis and graphs from one outer step to the next.
+ * Only steps taken one at a time are recorded (qqcd_set_arnoldi_steps(1), or
+ * cycles of more than 127 steps); blocks of four are launched as they are.
  * Tuning aid; no reference counterpart. */
 int qqcd_set_step_graphs(int mode);
+/* Graphs replayed so far by the single-right-hand-side solvers. */
+int qqcd_step_graph_replays(long *n);
 
 /* Toggle the XCD-aware workgroup order of the Dslash (default on). */
 int qqcd_set_xcd_remap(int on);

@@ -304,13 +304,12 @@ def test_fermprop_multi(cfg1, reorth, graph, basis):
 def test_fermprop_multi_normalisation_in_operator(cfg1):
     """With the FP16 basis and the two-slot operator each Arnoldi step's
     normalisation is done by the next operator application (the second hop
-    scales its result by 1 / ||w|| and writes the FP16 basis vector), and the
-    steps run in pairs (one Gram-Schmidt pass over the basis for the dots of
-    A v_j and A^2 v_j, one for both updates, column j + 1 from the Arnoldi
-    relation) or one at a time; with the one-slot launch form (2) a separate
-    pass normalises.  Paired steps take the norms of the updated vectors from
-    the projections (the update pass then writes the next basis vector) or
-    from the updated vectors (a third pass).  The operator's intermediate
+    scales its result by 1 / ||w|| and writes the FP16 basis vector) where the
+    steps run one at a time or in pairs (norms 0: one pass over the basis for
+    the dots of A v_j and A^2 v_j, one for both updates, a third for the norms
+    of the updated vectors); with the one-slot launch form (2) a separate
+    pass normalises.  By default (norms 1) the steps run in blocks of four,
+    whose update pass normalises.  The operator's intermediate
     field is FP16 with per-(site, slot) norms where the two-slot kernel runs,
     or FP32.  All reach the same true residuals and solutions to the solve's
     tolerance, with graph replays and eagerly."""
@@ -358,11 +357,14 @@ def test_fermprop_multi_normalisation_in_operator(cfg1):
             assert np.array_equal(sols[key + (1,)][r], sols[key + (0,)][r]), (key, r)
 
 
+@pytest.mark.parametrize("norms", [0, 1])
 @pytest.mark.parametrize("nsrc,gm", [(2, (40, 10)), (6, (41, 10))])
-def test_fermprop_multi_unpaired_shapes(cfg1, nsrc, gm):
-    # shapes where the batched solver cannot pair its Arnoldi steps: one
-    # batched source (RHS block 1: no two-slot operator) and an odd cycle
-    # length (m - k = 31); every source still reaches the true residual
+def test_fermprop_multi_unpaired_shapes(cfg1, nsrc, gm, norms):
+    # shapes where the batched solver cannot pair its Arnoldi steps (norms 0,
+    # which asks for pairs, then takes them one at a time): one batched source
+    # (RHS block 1: no two-slot operator) and an odd cycle length (m - k = 31),
+    # which cut the last block of four (norms 1); every source reaches the true
+    # residual
     n, bc, U, u, co, g = cfg1
     kappa = (0.150, 0.0)
     srcs = []
@@ -372,9 +374,14 @@ def test_fermprop_multi_unpaired_shapes(cfg1, nsrc, gm):
         disconloops.z4source(be, bo, 55, r, 1.0)
         srcs.append((be, bo))
     disconloops.batch_set(basis_prec=2)
-    print(f"[multi] unpaired shapes: {nsrc} sources, GMRES {gm}", flush=True)
-    xe, xo, it, rr = disconloops.fermprop_multi([s[0] for s in srcs], [s[1] for s in srcs], kappa, co, bc, 1e-10,
-                                                gm, u)
+    print(f"[multi] unpaired shapes: {nsrc} sources, GMRES {gm}, norms {norms}", flush=True)
+    try:
+        _lib.check(_lib.lib().qqcd_set_pair_norms(norms))
+        xe, xo, it, rr = disconloops.fermprop_multi([s[0] for s in srcs], [s[1] for s in srcs], kappa, co, bc, 1e-10,
+                                                    gm, u)
+        assert disconloops.batch_stats()["fallback"] == 0
+    finally:
+        _lib.check(_lib.lib().qqcd_set_pair_norms(1))
     for r, (be, bo) in enumerate(srcs):
         b = O.spinor_ref_to_canon(n, be, bo)
         x = O.spinor_ref_to_canon(n, xe[r], xo[r])

@@ -8,6 +8,7 @@ relative (max norm).  GMRES-Proj inside psc runs at the tolerance the
 reference hard-codes there (1e-8, inverters.f90:4442); its solution is
 compared at 1e-6 and a tighter direct call is held to the 1e-10 bar.
 """
+import ctypes
 import os
 
 import numpy as np
@@ -224,14 +225,21 @@ def test_solve_log_lines():
         lattice.finalize()
 
 
+def graph_replays():
+    from baylorlqcd_amd import _lib
+    n = ctypes.c_long()
+    _lib.check(_lib.lib().qqcd_step_graph_replays(ctypes.byref(n)))
+    return n.value
+
+
 def test_step_graphs_replay_same_solve():
-    """The mixed solver (FP16 operator and basis, one Gram-Schmidt pass) with
-    its groups of Arnoldi steps replayed from HIP graphs gives the eager
-    launches' solution bit for bit and the same step count, twice in a row
-    (graphs captured in the first solve are not carried into the second):
-    graphs in every inner solve (mode 1), and only in the later outer steps'
-    GMRES-Proj, whose basis and graphs are kept from one outer step to the
-    next (mode 2, the default)."""
+    """The mixed solver (FP16 operator and basis, one Gram-Schmidt pass, one
+    Arnoldi step at a time) with its groups of steps replayed from HIP graphs
+    gives the eager launches' solution bit for bit and the same step count,
+    twice in a row (graphs captured in the first solve are not carried into
+    the second): graphs in every inner solve (mode 1), and only in the later
+    outer steps' GMRES-Proj, whose basis and graphs are kept from one outer
+    step to the next (mode 2, the default)."""
     from baylorlqcd_amd import _lib
     g = np.load(os.path.join(GOLD, "golden_8x8x8x16.npz"))
     lattice.init(N8, BC)
@@ -243,12 +251,15 @@ def test_step_graphs_replay_same_solve():
     quark.pointsource(be, bo, (1, 1, 1, 1), 1, 1)
     runs = []
     try:
+        _lib.check(_lib.lib().qqcd_set_arnoldi_steps(1))
         for graphs in (0, 1, 1, 2, 2):
             _lib.check(_lib.lib().qqcd_set_step_graphs(graphs))
-            x = np.zeros_like(be)
+            x, before = np.zeros_like(be), graph_replays()
             it = inverters.solve_mixed(be, x, (40, 10), 1e-10, 2, 2, 12, 0.0, 0, u, co, kappa, BC)
             runs.append((it, x))
+            assert (graph_replays() > before) == (graphs > 0), graphs
     finally:
+        _lib.check(_lib.lib().qqcd_set_arnoldi_steps(2))
         _lib.check(_lib.lib().qqcd_set_step_graphs(2))
         lattice.finalize()
     for it, x in runs[1:]:
@@ -260,13 +271,13 @@ def test_step_graphs_replay_same_solve():
     r = bb - O.schur(N8, U, BC, [1] * 4, [1] * 4, 0, kappa, xm)
     assert np.linalg.norm(r[~odd]) / np.linalg.norm(bb[~odd]) < 1e-10
 
-def test_mixed_paired_steps():
+
+def test_mixed_block_steps():
     """The mixed solver over an FP16 basis runs its inner Arnoldi steps in
-    pairs (A v_j and A^2 v_j orthogonalised with one pass over the basis for
-    both sets of dots and one for both updates, column j + 1 from the Arnoldi
-    relation) or one at a time: both reach the true residual, their solutions
-    agree to the solve's tolerance, and the paired solve replays from HIP
-    graphs bit for bit."""
+    blocks of four (one pass over the basis for the dots of all four and one
+    for the updates) or one at a time: both reach the true residual and their
+    solutions agree to the solve's tolerance.  One at a time they replay from
+    HIP graphs bit for bit; blocks record none, whatever the mode."""
     from baylorlqcd_amd import _lib
     g = np.load(os.path.join(GOLD, "golden_8x8x8x16.npz"))
     lattice.init(N8, BC)
@@ -276,15 +287,16 @@ def test_mixed_paired_steps():
     kappa = (0.150, 0.0)
     be, bo = lattice.new_spinor(N8), lattice.new_spinor(N8)
     quark.pointsource(be, bo, (1, 1, 1, 1), 1, 1)
-    runs = {}
+    runs, replays = {}, {}
     lib = _lib.lib()
     try:
-        for steps, graphs in ((1, 0), (2, 0), (2, 1), (2, 2)):
+        for steps, graphs in ((1, 0), (1, 1), (1, 2), (2, 0), (2, 1), (2, 2)):
             _lib.check(lib.qqcd_set_arnoldi_steps(steps))
             _lib.check(lib.qqcd_set_step_graphs(graphs))
-            x = np.zeros_like(be)
+            x, before = np.zeros_like(be), graph_replays()
             it = inverters.solve_mixed(be, x, (40, 10), 1e-10, 2, 2, 12, 0.0, 0, u, co, kappa, BC)
             runs[(steps, graphs)] = (it, x)
+            replays[(steps, graphs)] = graph_replays() - before
     finally:
         _lib.check(lib.qqcd_set_arnoldi_steps(2))
         _lib.check(lib.qqcd_set_step_graphs(2))
@@ -298,6 +310,7 @@ def test_mixed_paired_steps():
         x1 = O.spinor_ref_to_canon(N8, runs[(1, 0)][1].ravel(order="F"), None)
         assert np.linalg.norm(xm[~odd] - x1[~odd]) / np.linalg.norm(x1[~odd]) < 1e-8, key
         assert abs(it - runs[(1, 0)][0]) <= 0.15 * runs[(1, 0)][0], (key, it, runs[(1, 0)][0])
-    for key in ((2, 1), (2, 2)):
-        assert runs[key][0] == runs[(2, 0)][0]
-        assert np.array_equal(runs[key][1], runs[(2, 0)][1]), key
+    for steps, graphs in runs:
+        assert (replays[(steps, graphs)] > 0) == (steps == 1 and graphs > 0)
+        assert runs[(steps, graphs)][0] == runs[(steps, 0)][0]
+        assert np.array_equal(runs[(steps, graphs)][1], runs[(steps, 0)][1]), (steps, graphs)
