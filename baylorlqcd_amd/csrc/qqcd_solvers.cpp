@@ -252,9 +252,8 @@ static void arnoldi_steps_dev(Context &c, LinOp &A, std::vector<Spinor> &V, int 
 
 // Arnoldi steps j .. j + want - 1 in blocks (qqcd_arnoldi.h), the columns into
 // H; returns how many were made.  work: over an FP16 basis, the FP32 vectors of
-// a block.  A block
-// reads the basis twice whatever its length, where a step of its own with the
-// DGKS test read it four times.
+// a block.  A block reads the basis twice whatever its length, where a step of
+// its own with the DGKS test read it four times.
 //
 // Four steps a block: the smallest R_ii^2 / G_ii is 0.077 (two steps: 0.38), so
 // R^-1 costs a factor of 3.6 in rounding; the same Krylov steps as one at a

@@ -168,11 +168,12 @@ namespace qqcd {
 // true residual the judge of every result.
 // replay repeated groups of synchronisation-free Arnoldi steps from HIP
 // graphs: 0 never, 1 in every solve, 2 (the default) only where the basis is
-// kept between calls (ProjWork), so that a capture serves many solves
+// kept between calls (ProjWork), so that a capture serves many solves; steps
+// taken one at a time only, blocks are launched as they are
 void set_step_graphs(int mode);
 long step_graph_replays();  // since the library was loaded
-// Arnoldi steps per Gram-Schmidt pass: 2 (the default) in blocks of four (the
-// batched solver: in pairs), 1 one at a time
+// Arnoldi steps per Gram-Schmidt pass, in these solvers and the batched one: 2
+// (the default) in blocks of four, 1 one at a time
 void set_arnoldi_steps(int steps);
 int arnoldi_steps();
 

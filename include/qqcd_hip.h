@@ -424,15 +424,20 @@ int qqcd_batch_set(int reorth, int use_graph, double inner_tol, int inner_cycles
  * (FP16 basis) and the single-right-hand-side solvers: 2 (the default) runs
  * the steps in blocks of four -- four operator applications, the dots of all
  * four and the updates of all four in one pass each over the basis, the
- * Hessenberg columns from the operator's relations -- where one Gram-Schmidt
- * pass is enough (qqcd_batch_set's reorth 0); 1 one step at a time.  Tuning
- * aid; no reference counterpart. */
+ * Hessenberg columns from the operator's relations -- in the FP64 solvers with
+ * a second pass for vectors that cancelled, over FP32 and FP16 bases with one
+ * (the batched solver: with qqcd_batch_set's reorth 0); 1 one step at a time,
+ * the slower form that blocks are checked against and that cycles of more than
+ * 127 steps and flexible solves take in any case.  Tuning aid; no reference
+ * counterpart. */
 int qqcd_set_arnoldi_steps(int steps);
 
 /* Blocks of the batched solver: 1 (the default) runs blocks of four steps; 0
  * blocks of two, whose norms come from the updated vectors with a third pass
  * over the pair (with the two-slot operator and an even cycle length; one step
- * at a time otherwise).  Tuning aid; no reference counterpart. */
+ * at a time otherwise).  Slower, but with two FP32 fields less: what a batch
+ * takes by itself where the card has no room for those.  Tuning aid; no
+ * reference counterpart. */
 int qqcd_set_pair_norms(int mode);
 
 /* Storage of the batched solver's inner operator's intermediate field (the
