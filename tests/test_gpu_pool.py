@@ -103,7 +103,7 @@ def test_full_card():
             except torch.OutOfMemoryError:
                 step //= 2
         psi = np.random.default_rng(2).standard_normal((1, int(np.prod(n)), 4, 6)).view(complex)
-        out = np.empty_like(psi)
+        out = np.zeros_like(psi)  # the odd half stays
         disconloops.schur_multi_canonical(psi, out, (0.14, 0.0), prec=1, recon=18)  # 9 MB of links in FP32 first
         assert np.all(np.isfinite(out)) and np.any(out)
         it = inverters.solve_mixed(b, x, (20, 5), 1e-10, 1, 1, 12, 0.0, 0, u, O.coact_array(), (0.14, 0.01), BC)
