@@ -102,6 +102,8 @@ class Batch {
  public:
   Batch(Context &c, const double kappa[2], MultiSpinor &B, MultiSpinor &X, const Deflation &D, const BatchParams &p,
         std::vector<int> &id);
+  // a graph may be running when an error unwinds
+  ~Batch() { (void)hipStreamSynchronize(c.stream); }
   BatchStats run(int n);
 
  private:

@@ -582,9 +582,9 @@ struct BUTab {
 // Bound by reading the basis: the wavefronts of a workgroup take BQ fields each (the last one the u_c) of the same
 // 64 elements, so the u_c come from memory once and from the L1 for the other wavefronts.  Sums in FP32 over runs of
 // `most` elements of a lane (the basis carries 11 bits), in FP64 beyond; two elements are in flight, one is worked on.
-// 16^3x32, 23 sources, 1..37 basis vectors: 586 us a block of four (578 with all of a lane's 290 elements in FP32);
-// 6 fields a wavefront against 8 (141 registers) and 4, in FP32 throughout: 591, 631, 606; with the update below
-// 1.22 ms for four steps, where two pairs of steps took about 1.5.
+// 16^3x32, 23 sources, 1..37 basis vectors: 586-601 us a block of four (578-587 in the same runs with all of a lane's
+// 290 elements in FP32); 6 fields a wavefront against 8 (141 registers) and 4, in FP32 throughout: 591, 631, 606; with
+// the update below 1.23 ms for four steps, where two pairs of steps took about 1.5.
 template <int S, int HV>
 __global__ void __launch_bounds__(64 * BWV) k_mbdot(MShape a, BTab v, BUTab ut, int q0, int nq, int most, double *part) {
   const int nact = *a.nact, nb = 1 << a.lognb, blk = blockIdx.y;
