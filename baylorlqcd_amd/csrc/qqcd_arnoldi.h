@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "qqcd_blas.h"
+#include "qqcd_pool.h"
 
 namespace qqcd {
 
@@ -21,7 +22,6 @@ class BlockArnoldi {
   static constexpr int SMAX = 4;
   static constexpr int NMAX = 128;  // vectors of a basis
   BlockArnoldi(hipStream_t s, int m);  // cycles of at most m steps
-  ~BlockArnoldi();
   BlockArnoldi(const BlockArnoldi &) = delete;
   BlockArnoldi &operator=(const BlockArnoldi &) = delete;
 
@@ -56,6 +56,7 @@ class BlockArnoldi {
   void run(const Vec *V, int j, int s, int slot, bool again);
   hipStream_t stream;
   int m, ld;
+  PoolSet bufs;
   double *hd = nullptr;    // H of B on the device: ld rows, m columns, complex
   double *part = nullptr;  // partial sums
   double *sums = nullptr;  // their totals: left vectors x s, complex

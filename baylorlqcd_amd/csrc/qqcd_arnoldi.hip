@@ -416,23 +416,13 @@ static constexpr int CHUNKS = BlockArnoldi::NMAX / KV + 1;
 BlockArnoldi::BlockArnoldi(hipStream_t s, int m_) : stream(s), m(m_), ld(m_ + 1) {
   if (m < 1 || m + 1 > NMAX) throw std::runtime_error("BlockArnoldi: at most 127 steps");
   const int slots = m;  // one per block at least
-  pool_get(&hd, sizeof(double) * 2 * ld * m);
-  pool_get(&part, sizeof(double) * 2 * KV * SMAX * DGRID * CHUNKS);
-  pool_get(&sums, sizeof(double) * 2 * KV * SMAX * CHUNKS);
-  pool_get(&pr, sizeof(double) * 2 * SMAX * (NMAX + SMAX));
-  pool_get(&coef, sizeof(double) * 2 * SMAX * (NMAX + SMAX));
-  pool_get(&coef32, sizeof(float) * 2 * SMAX * (NMAX + SMAX));
-  hh = static_cast<double *>(pool_alloc_host(sizeof(double) * slot_len() * slots));
-}
-
-BlockArnoldi::~BlockArnoldi() {
-  pool_free(hd);
-  pool_free(part);
-  pool_free(sums);
-  pool_free(pr);
-  pool_free(coef);
-  pool_free(coef32);
-  pool_free_host(hh);
+  bufs.get(&hd, sizeof(double) * 2 * ld * m);
+  bufs.get(&part, sizeof(double) * 2 * KV * SMAX * DGRID * CHUNKS);
+  bufs.get(&sums, sizeof(double) * 2 * KV * SMAX * CHUNKS);
+  bufs.get(&pr, sizeof(double) * 2 * SMAX * (NMAX + SMAX));
+  bufs.get(&coef, sizeof(double) * 2 * SMAX * (NMAX + SMAX));
+  bufs.get(&coef32, sizeof(float) * 2 * SMAX * (NMAX + SMAX));
+  bufs.get_host(&hh, sizeof(double) * slot_len() * slots);
 }
 
 void BlockArnoldi::load(const zd *h, int ldh, int n, double sigma) {

@@ -1,6 +1,7 @@
 // qqcd_bicgstab.h -- the vector passes of BiCGStab with their scalars on the device.
 #pragma once
 #include "qqcd_blas.h"
+#include "qqcd_pool.h"
 
 namespace qqcd {
 
@@ -13,7 +14,6 @@ class BiCGStabDev {
  public:
   static constexpr int AHEAD = 32;  // iterations queued between two reads of the history at most
   BiCGStabDev(hipStream_t s, long n);
-  ~BiCGStabDev();
   BiCGStabDev(const BiCGStabDev &) = delete;
   BiCGStabDev &operator=(const BiCGStabDev &) = delete;
 
@@ -31,6 +31,7 @@ class BiCGStabDev {
  private:
   hipStream_t stream;
   long n;
+  PoolSet bufs;
   double *part = nullptr;
   void *state = nullptr;     // device scalars
   double *hist = nullptr;    // pinned: AHEAD residual norms, iterations done, ended

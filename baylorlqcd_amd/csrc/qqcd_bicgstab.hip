@@ -198,15 +198,9 @@ __global__ void __launch_bounds__(TB) k_bi_x(long n, BState *s, const double2 *r
 
 BiCGStabDev::BiCGStabDev(hipStream_t s, long n_) : stream(s), n(n_) {
   if (n < 1) throw std::runtime_error("bicgstab: empty vectors");
-  pool_get(&part, sizeof(double) * 3 * GMAX);
-  pool_get(&state, sizeof(BState));
-  hist = static_cast<double *>(pool_alloc_host(sizeof(double) * (AHEAD + 2)));
-}
-
-BiCGStabDev::~BiCGStabDev() {
-  pool_free(part);
-  pool_free(state);
-  pool_free_host(hist);
+  bufs.get(&part, sizeof(double) * 3 * GMAX);
+  bufs.get(&state, sizeof(BState));
+  bufs.get_host(&hist, sizeof(double) * (AHEAD + 2));
 }
 
 static void check(const Vec &v, long n) {

@@ -842,6 +842,7 @@ void MBlas::reserve(size_t n) {
     QQCD_HIP(hipStreamSynchronize(stream));
     pool_free(part);
     part = nullptr;
+    part_cap = 0;
   }
   pool_get(&part, n * sizeof(double));
   part_cap = n;

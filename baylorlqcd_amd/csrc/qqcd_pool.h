@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <vector>
 
 namespace qqcd {
 
@@ -39,5 +40,29 @@ template <typename T> hipError_t device_malloc(T **p, size_t bytes) {
 }
 
 template <typename T> void pool_get(T **p, size_t bytes) { *p = static_cast<T *>(pool_alloc(bytes)); }
+
+// The buffers of one object, returned with it, also where its constructor fails
+// halfway.
+class PoolSet {
+ public:
+  PoolSet() = default;
+  ~PoolSet() {
+    for (void *p : device) pool_free(p);
+    for (void *p : pinned) pool_free_host(p);
+  }
+  PoolSet(const PoolSet &) = delete;
+  PoolSet &operator=(const PoolSet &) = delete;
+  template <typename T> void get(T **p, size_t bytes) {
+    device.reserve(device.size() + 1);
+    device.push_back(*p = static_cast<T *>(pool_alloc(bytes)));
+  }
+  template <typename T> void get_host(T **p, size_t bytes) {
+    pinned.reserve(pinned.size() + 1);
+    pinned.push_back(*p = static_cast<T *>(pool_alloc_host(bytes)));
+  }
+
+ private:
+  std::vector<void *> device, pinned;
+};
 
 }  // namespace qqcd

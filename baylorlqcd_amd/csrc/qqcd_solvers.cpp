@@ -118,14 +118,11 @@ struct DevHess {
   int m, ld;              // ld = 2 (m + 1) doubles per column
   double *d = nullptr;    // m columns of complex <V_i, w>, then m squared norms
   double *h = nullptr;    // pinned host copy
+  PoolSet bufs;
   explicit DevHess(int m_) : m(m_), ld(2 * (m_ + 1)) {
     const size_t n = (size_t)(ld + 1) * m;
-    pool_get(&d, sizeof(double) * n);
-    h = static_cast<double *>(pool_alloc_host(sizeof(double) * n));
-  }
-  ~DevHess() {
-    pool_free(d);
-    pool_free_host(h);
+    bufs.get(&d, sizeof(double) * n);
+    bufs.get_host(&h, sizeof(double) * n);
   }
   DevHess(const DevHess &) = delete;
   DevHess &operator=(const DevHess &) = delete;

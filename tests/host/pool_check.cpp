@@ -145,12 +145,36 @@ int unpooled() {
   return 0;
 }
 
+// an object whose constructor fails returns what it has got so far
+int half_built() {
+  struct Object {
+    PoolSet bufs;
+    double *a = nullptr, *b = nullptr, *c = nullptr;
+    Object() {
+      bufs.get(&a, 2 * MB);
+      bufs.get_host(&b, 2 * MB);
+      bufs.get(&c, 100 * MB);
+    }
+  };
+  bool thrown = false;
+  try {
+    Object o;
+  } catch (const std::runtime_error &) {
+    thrown = true;
+  }
+  EXPECT(thrown);
+  pool_trim();
+  EXPECT(used == 0 && pinned == 0);
+  return 0;
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "pinned_wait") return pinned_wait();
   if (what == "other_size") return other_size();
   if (what == "pinned_share") return pinned_share();
   if (what == "unpooled") return unpooled();
+  if (what == "half_built") return half_built();
   std::printf("no such check\n");
   return 2;
 }

@@ -22,7 +22,7 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("what", ["pinned_wait", "other_size", "pinned_share", "unpooled"])
+@pytest.mark.parametrize("what", ["pinned_wait", "other_size", "pinned_share", "unpooled", "half_built"])
 def test_pool(program, what):
     r = subprocess.run([program, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
