@@ -28,16 +28,13 @@ struct BState {
   unsigned arrived[4];  // workgroups of each reduction that have left their partials
 };
 
-// a / b by R. L. Smith's algorithm (Comm. ACM 5 (1962) 435): |b|^2 is not
-// formed, which for rho (a squared norm) leaves the range of FP64 at sources
-// of 1e-75 or 1e+80
+// a / b with b brought to order one by a power of two first: |b|^2 for rho (a
+// squared norm) would leave the range of FP64 at sources of 1e-75 or 1e+80
 __device__ __forceinline__ double2 cdiv(double2 a, double2 b) {
-  if (fabs(b.x) >= fabs(b.y)) {
-    const double r = b.y / b.x, d = b.x + b.y * r;
-    return make_double2((a.x + a.y * r) / d, (a.y - a.x * r) / d);
-  }
-  const double r = b.x / b.y, d = b.x * r + b.y;
-  return make_double2((a.x * r + a.y) / d, (a.y * r - a.x) / d);
+  const int e = -__builtin_amdgcn_frexp_exp(fmax(fabs(b.x), fabs(b.y)));
+  b = make_double2(ldexp(b.x, e), ldexp(b.y, e));
+  const double d = 1.0 / (b.x * b.x + b.y * b.y);
+  return make_double2(ldexp((a.x * b.x + a.y * b.y) * d, e), ldexp((a.y * b.x - a.x * b.y) * d, e));
 }
 __device__ __forceinline__ double2 cmulz(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
